@@ -7,8 +7,8 @@
 // v1.w and the leaf end flagged by the bit pattern 0x80000000 in v2.w, 64-byte instance
 // records ending a top-level leaf with pad = {-1,-1}.
 //
-// Per ray the traversal is depth first: both child boxes of a node are tested, the nearer
-// child (ties: left) is visited first and the other is pushed.  Entering an instance
+// Per ray the traversal is depth first: the child boxes of a node are tested, the nearest hit
+// child (ties: the lower one) is visited first and the others are pushed.  Entering an instance
 // transforms the ray into object space and remembers the stack depth; when the stack falls
 // back to that depth the next instance of the same leaf is entered, or the world ray is
 // restored.  Arithmetic (fixed, shared with the CPU restatement used as the checker):
@@ -47,8 +47,6 @@ struct TraceArgs {
     int spill_depth;      // spill entries per thread
     int* work_counter;    // persistent variant: next ray to fetch
     const int* count_dev; // device ray count read when the launch runs (<= count), or null
-    int tl_base, tl_nodes; // quantized tree: nodes [tl_base, tl_base + tl_nodes) are read from
-                           // the block's copy in LDS (dynamic shared memory, 64 B per node)
 };
 
 // Rays of this launch: count, or the device count clamped to [0, count].
@@ -172,16 +170,7 @@ __device__ __forceinline__ IMBA_AS(1) T* gview_w(T* p) {
 }
 
 // Per-lane traversal stack: entry 0..sp-1 in LDS ([depth][lane], conflict free), then in the
-// global spill buffer.  With IMBA_STACK_TOP_REG=1 the top entry lives in a register instead: a
-// pop returns it at once and issues the load that refills it, which has a whole node step to
-// arrive; a push writes the previous top out.  Measured on the 21M-triangle PT frame (quantized
-// 4-wide, 256 x 16): 970 / 973 against 975 Mrays/s with every entry in LDS (one more VGPR, 4
-// more bytes of scratch per lane in the 7-wave variants), so the pops' LDS latency is hidden
-// already and the option stays off.
-#ifndef IMBA_STACK_TOP_REG
-#define IMBA_STACK_TOP_REG 0
-#endif
-
+// global spill buffer.  (Holding the top entry in a register measured no faster.)
 template <int BLOCK, int STACK_LDS>
 struct LaneStack {
     int* lds;     // [STACK_LDS][BLOCK]
@@ -191,23 +180,8 @@ struct LaneStack {
     int spill_slot;  // global thread index
     int spill_stride;
     int sp;
-    int top;          // entry sp - 1 (IMBA_STACK_TOP_REG)
-    const uint4* tl;  // LDS copy of the treelet nodes (64 B each, as in memory), or null
 
-    __device__ __forceinline__ void store(int k, int v) {
-        if (k < STACK_LDS) lds_view(lds)[k * BLOCK + lane_slot] = v;
-        else spill[(size_t)(k - STACK_LDS) * spill_stride + spill_slot] = v;
-    }
-    __device__ __forceinline__ int load(int k) {
-        if (k < STACK_LDS) return lds_view(lds)[k * BLOCK + lane_slot];
-        return spill[(size_t)(k - STACK_LDS) * spill_stride + spill_slot];
-    }
     __device__ __forceinline__ bool push(int v) {
-#if IMBA_STACK_TOP_REG
-        if (sp - STACK_LDS >= spill_depth) return false;
-        if (sp > 0) store(sp - 1, top);
-        top = v;
-#else
         // (the capacity test only on the spill path: testing it first for every push measured
         // 14% slower on the deep trees of 256 queues over 10K-4M random triangles)
         if (sp < STACK_LDS) {
@@ -217,41 +191,63 @@ struct LaneStack {
             if (k >= spill_depth) return false;
             spill[(size_t)k * spill_stride + spill_slot] = v;
         }
-#endif
         sp++;
         return true;
     }
+    // Pushes the first n of c1, c2, c3 (n <= 3), the last one deepest.
+    __device__ __forceinline__ bool push3(int c1, int c2, int c3, int n) {
+        if (sp + 3 <= STACK_LDS) {
+            // written without branches: an entry past the new top is overwritten by a later push
+            auto* p = lds_view(lds) + sp * BLOCK + lane_slot;
+            p[0] = n >= 3 ? c3 : n == 2 ? c2 : c1;
+            p[BLOCK] = n >= 3 ? c2 : c1;
+            p[2 * BLOCK] = c1;
+            sp += n;
+            return true;
+        }
+        bool ok = true;
+        if (n >= 3) ok &= push(c3);
+        if (n >= 2) ok &= push(c2);
+        if (n >= 1) ok &= push(c1);
+        return ok;
+    }
     __device__ __forceinline__ int pop() {
         sp--;
-#if IMBA_STACK_TOP_REG
-        const int v = top;
-        if (sp > 0) top = load(sp - 1);
-        return v;
-#else
         if (sp < STACK_LDS) return lds_view(lds)[sp * BLOCK + lane_slot];
         return spill[(size_t)(sp - STACK_LDS) * spill_stride + spill_slot];
-#endif
     }
 };
 
-enum : int { kTop = 1, kInstLast = 2, kBad = 4, kDone = 8 };
+__device__ __forceinline__ float4 as_float4(const uint4& u) {
+    return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
+}
 
-// Traversal state of one ray (kept in registers across the steps of the persistent kernel).
+
+// The world-space ray, kept while the ray is inside an instance.
 struct WorldRay {
     float ox, oy, oz, dx, dy, dz;
     float idx, idy, idz;  // 1 / safe_dir(d), as setup_space computes them
 };
 
+// What a ray does in its next step: a node, a triangle of the current leaf, an instance, or
+// (kNone) whatever comes off the stack.
+enum : int { kNode = 0, kTri = 1, kInst = 2, kNone = 3 };
+
+// Traversal state of one ray.  Every member is assigned from every path of a step by value: a
+// member stored on one side of a branch and another on the other side is merged into one store
+// through a selected address, which puts the state into scratch memory.
 struct TraceState {
     WorldRay world;  // world-space ray (its reciprocals are recomputed when the ray returns to it)
     RaySpace cs;     // ray in the space of the current level (world or an instance's object space)
     float tmin;      // the ray's tmax is best_t until a hit
     float best_t, best_u;
     int best_tri, best_inst;
-    int node;        // next node / leaf link to process, kNoNode if none
-    int tri;         // next triangle record of the current leaf, -1 if none
-    int inst, inst_id, inst_sp;  // current instance, its id, stack depth when it was entered
-    int flags;
+    int kind;        // what comes next
+    int item;        // its index (node, Vec4 of the triangle's first vertex, instance record)
+    int inst_id;     // id of the current instance
+    int inst_next;   // the next instance record of the same leaf, -1: none
+    int inst_sp;     // stack depth when the instance was entered, -1 in world space
+    int bad;         // the ray met a malformed structure
     uint32_t cn, ct, ci;  // visit counts (stats variant)
     uint32_t cd;          // deepest stack entry used (stats variant)
 };
@@ -279,26 +275,21 @@ __device__ __forceinline__ void state_init(TraceState& s, const float4& ro, cons
     s.best_u = 0.0f;
     s.best_tri = -1;
     s.best_inst = -1;
-    s.node = root;
-    s.tri = -1;
-    s.inst = -1;
+    s.kind = kNode;
+    s.item = root;
     s.inst_id = -1;
+    s.inst_next = -1;
     s.inst_sp = -1;
-    s.flags = kTop | kInstLast;
+    s.bad = 0;
     s.cn = s.ct = s.ci = s.cd = 0;
 }
 
-// Enters instance i of the current top-level leaf: the ray goes to its object space.
-// Returns the instance's root node, or kNoNode for a malformed record.
+// Instance record i (r0..r2 its transform, r3 its id, root and list end): the ray goes to its
+// object space and on to the instance's root node.
 template <bool STATS>
-__device__ __forceinline__ int enter_instance(const TraceArgs& a, TraceState& s, int i, int sp) {
-    if ((unsigned)i >= (unsigned)a.n_inst) {
-        s.flags |= kBad | kInstLast;
-        return kNoNode;
-    }
-    const auto* inst = gview(a.inst);
-    const float4 m0 = inst[4 * i + 0], m1 = inst[4 * i + 1], m2 = inst[4 * i + 2];
-    const int4 meta = gview(reinterpret_cast<const int4*>(a.inst))[4 * i + 3];
+__device__ __forceinline__ int enter_instance(TraceState& s, const uint4& r0, const uint4& r1, const uint4& r2,
+                                               const uint4& r3, int sp) {
+    const float4 m0 = as_float4(r0), m1 = as_float4(r1), m2 = as_float4(r2);
     if (STATS) s.ci++;
     const WorldRay& w = s.world;
     s.cs.ox = fmaf(m0.x, w.ox, fmaf(m0.y, w.oy, fmaf(m0.z, w.oz, m0.w)));
@@ -317,61 +308,32 @@ __device__ __forceinline__ int enter_instance(const TraceArgs& a, TraceState& s,
     } else {
         setup_space(s.cs);
     }
-    s.inst = i;
-    s.inst_id = meta.x;
+    s.inst_id = (int)r3.x;
+    s.inst_next = (int)r3.z == -1 ? -1 : s.item + 1;
     s.inst_sp = sp;
-    s.flags = (s.flags & ~(kTop | kInstLast)) | (meta.z == -1 ? kInstLast : 0);
-    if ((unsigned)meta.y >= (unsigned)a.n_nodes) {
-        s.flags |= kBad;
-        return kNoNode;
-    }
-    return meta.y;
-}
-
-// A leaf link in s.node: top-level leaves enter their first instance, mesh leaves start
-// their triangle list.
-template <bool STATS>
-__device__ __forceinline__ void resolve_leaf(const TraceArgs& a, TraceState& s, int sp) {
-    if (s.node < 0 && s.node != kNoNode) {
-        if (s.flags & kTop) {
-            s.node = enter_instance<STATS>(a, s, ~s.node, sp);
-        } else {
-            s.tri = ~s.node;
-            s.node = kNoNode;
-        }
-    }
+    return (int)r3.y & 0x7fffffff;  // out of range (a negative root included): the next step's bounds check
 }
 
 // One inner node of the BVH2: both child boxes are tested, the nearer hit child (ties: left)
 // is next and the other is pushed.
 template <int BLOCK, int STACK_LDS, bool STATS>
-__device__ __forceinline__ void node_step2(const TraceArgs& a, TraceState& s, LaneStack<BLOCK, STACK_LDS>& st) {
-    const int n = s.node;
-    if (n >= a.n_nodes) {
-        s.flags |= kBad;
-        s.node = kNoNode;
-        return;
-    }
-    const auto* nodes = gview(a.nodes);
-    const float4 n0 = nodes[4 * n + 0];
-    const float4 n1 = nodes[4 * n + 1];
-    const float4 n2 = nodes[4 * n + 2];
-    const int4 n3 = gview(reinterpret_cast<const int4*>(a.nodes))[4 * n + 3];
+__device__ __forceinline__ int node_step2(TraceState& s, LaneStack<BLOCK, STACK_LDS>& st, const uint4& r0,
+                                           const uint4& r1, const uint4& r2, const uint4& r3) {
+    const int n = s.item;
+    const float4 n0 = as_float4(r0), n1 = as_float4(r1), n2 = as_float4(r2);
+    const int cl = (int)r3.x, cr = (int)r3.y;
     if (STATS) s.cn++;
     float tl = 0.0f, tr = 0.0f;
     bool hl = box_hit(s.cs, n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, s.tmin, s.best_t, tl);
-    bool hr = n3.y != kDummyChild && box_hit(s.cs, n1.z, n1.w, n2.x, n2.y, n2.z, n2.w, s.tmin, s.best_t, tr);
-    if (hl && n3.x >= 0 && n3.x <= n) { hl = false; s.flags |= kBad; }
-    if (hr && n3.y >= 0 && n3.y <= n) { hr = false; s.flags |= kBad; }
+    bool hr = cr != kDummyChild && box_hit(s.cs, n1.z, n1.w, n2.x, n2.y, n2.z, n2.w, s.tmin, s.best_t, tr);
+    if (hl && cl >= 0 && cl <= n) { hl = false; s.bad = 1; }
+    if (hr && cr >= 0 && cr <= n) { hr = false; s.bad = 1; }
+    const bool left_first = hl && !(hr && tr < tl);
     if (hl && hr) {
-        const bool left_first = tl <= tr;
-        if (!st.push(left_first ? n3.y : n3.x)) s.flags |= kBad;
+        if (!st.push(left_first ? cr : cl)) s.bad = 1;
         if (STATS) s.cd = max(s.cd, (uint32_t)st.sp);
-        s.node = left_first ? n3.x : n3.y;
-    } else {
-        s.node = hl ? n3.x : (hr ? n3.y : kNoNode);
     }
-    resolve_leaf<STATS>(a, s, st.sp);
+    return hl || hr ? (left_first ? cl : cr) : kNoNode;
 }
 
 // Ordered exchange of two (distance, link) pairs: the nearer first, the lower slot on a tie.
@@ -385,194 +347,259 @@ __device__ __forceinline__ void order2(float& da, int& ca, float& db, int& cb) {
     ca = c;
 }
 
-// One node of the 4-wide tree (ImbaNode4 layout: 8 float4 = min_x, max_x, min_y, max_y, min_z,
-// max_z, children, count): the used child boxes are tested, the nearest hit child is next and
-// the other hit children are pushed, farthest deepest.
+// The hit children of a 4-wide node, given their distances (infinity: not hit): the nearest is
+// next, the others are pushed, farthest deepest.
 template <int BLOCK, int STACK_LDS, bool STATS>
-__device__ __forceinline__ void node_step4(const TraceArgs& a, TraceState& s, LaneStack<BLOCK, STACK_LDS>& st) {
-    const int n = s.node;
-    if (n >= a.n_nodes) {
-        s.flags |= kBad;
-        s.node = kNoNode;
-        return;
-    }
-    const auto* p = gview(a.nodes + 8 * (size_t)n);
-    const float4 lx = p[0], hx = p[1], ly = p[2], hy = p[3], lz = p[4], hz = p[5];
-    const int4 ch = gview(reinterpret_cast<const int4*>(a.nodes + 8 * (size_t)n))[6];
-    if (STATS) s.cn++;
-    float d0, d1, d2, d3;
-    bool h0 = ch.x != 0 && box_hit(s.cs, lx.x, hx.x, ly.x, hy.x, lz.x, hz.x, s.tmin, s.best_t, d0);
-    bool h1 = ch.y != 0 && box_hit(s.cs, lx.y, hx.y, ly.y, hy.y, lz.y, hz.y, s.tmin, s.best_t, d1);
-    bool h2 = ch.z != 0 && box_hit(s.cs, lx.z, hx.z, ly.z, hy.z, lz.z, hz.z, s.tmin, s.best_t, d2);
-    bool h3 = ch.w != 0 && box_hit(s.cs, lx.w, hx.w, ly.w, hy.w, lz.w, hz.w, s.tmin, s.best_t, d3);
-    if (h0 && ch.x > 0 && ch.x <= n) { h0 = false; s.flags |= kBad; }
-    if (h1 && ch.y > 0 && ch.y <= n) { h1 = false; s.flags |= kBad; }
-    if (h2 && ch.z > 0 && ch.z <= n) { h2 = false; s.flags |= kBad; }
-    if (h3 && ch.w > 0 && ch.w <= n) { h3 = false; s.flags |= kBad; }
-    const int cnt = (int)h0 + (int)h1 + (int)h2 + (int)h3;
-    const float inf = __int_as_float(0x7f800000);
-    float e0 = h0 ? d0 : inf, e1 = h1 ? d1 : inf, e2 = h2 ? d2 : inf, e3 = h3 ? d3 : inf;
-    int c0 = ch.x, c1 = ch.y, c2 = ch.z, c3 = ch.w;
+__device__ __forceinline__ int descend4(TraceState& s, LaneStack<BLOCK, STACK_LDS>& st, float e0, float e1, float e2,
+                                         float e3, int c0, int c1, int c2, int c3, int cnt) {
     // sorting network; misses (at infinity) end up last
     order2(e0, c0, e1, c1);
     order2(e2, c2, e3, c3);
     order2(e0, c0, e2, c2);
     order2(e1, c1, e3, c3);
     order2(e1, c1, e2, c2);
-    if (cnt == 0) {
-        s.node = kNoNode;
-    } else {
-        bool ok = true;
-        if (cnt >= 4) ok &= st.push(c3);
-        if (cnt >= 3) ok &= st.push(c2);
-        if (cnt >= 2) ok &= st.push(c1);
-        if (STATS) s.cd = max(s.cd, (uint32_t)st.sp);
-        if (!ok) s.flags |= kBad;
-        s.node = c0;
-    }
-    resolve_leaf<STATS>(a, s, st.sp);
+    if (!st.push3(c1, c2, c3, max(cnt - 1, 0))) s.bad = 1;
+    if (STATS) s.cd = max(s.cd, (uint32_t)st.sp);
+    return cnt ? c0 : kNoNode;
 }
 
-// Child box j of a quantized 4-wide node, one axis: [fma(q_lo, 2^e, o), fma(q_hi, 2^e, o)].
-__device__ __forceinline__ float dequant(uint32_t word, int j, float scale, float origin) {
-    return fmaf((float)((word >> (8 * j)) & 255u), scale, origin);
-}
-
-// One node of the quantized 4-wide tree (64 B: origin, exponents, children, 8-bit child
-// bounds per axis); otherwise as node_step4.  The dequantized boxes contain the exact ones.
-template <int BLOCK, int STACK_LDS, bool STATS, bool TLK>
-__device__ __forceinline__ void node_step4q(const TraceArgs& a, TraceState& s, LaneStack<BLOCK, STACK_LDS>& st) {
-    const int n = s.node;
-    if (n >= a.n_nodes) {
-        s.flags |= kBad;
-        s.node = kNoNode;
-        return;
-    }
-    uint4 w0, w1, w2, w3;
-    const unsigned in_tl = (unsigned)(n - a.tl_base);
-    if (TLK && in_tl < (unsigned)a.tl_nodes) {
-        const uint4* q = st.tl + 4 * in_tl;
-        w0 = q[0]; w1 = q[1]; w2 = q[2]; w3 = q[3];
-    } else if (TLK) {
-        // merged with the branch above into one flat load by the compiler
-        const uint4* p = reinterpret_cast<const uint4*>(a.nodes) + 4 * (size_t)n;
-        w0 = p[0]; w1 = p[1]; w2 = p[2]; w3 = p[3];
-    } else {
-        const auto* p = gview(reinterpret_cast<const uint4*>(a.nodes) + 4 * (size_t)n);
-        w0 = p[0]; w1 = p[1]; w2 = p[2]; w3 = p[3];
-    }
+// One node of the 4-wide tree (ImbaNode4 layout: 8 float4 = min_x, max_x, min_y, max_y, min_z,
+// max_z, children, count): the used child boxes are tested.
+template <int BLOCK, int STACK_LDS, bool STATS>
+__device__ __forceinline__ int node_step4(const TraceArgs& a, TraceState& s, LaneStack<BLOCK, STACK_LDS>& st,
+                                           const uint4& r0, const uint4& r1, const uint4& r2, const uint4& r3) {
+    const int n = s.item;
+    const auto* p = gview(a.nodes + 8 * (size_t)n);
+    const float4 lz = p[4], hz = p[5];
+    const int4 ch = gview(reinterpret_cast<const int4*>(a.nodes + 8 * (size_t)n))[6];
+    const float4 lx = as_float4(r0), hx = as_float4(r1), ly = as_float4(r2), hy = as_float4(r3);
     if (STATS) s.cn++;
-    const float ox = __uint_as_float(w0.x), oy = __uint_as_float(w0.y), oz = __uint_as_float(w0.z);
-    const float sx = __uint_as_float((uint32_t)((int)(int8_t)(w0.w & 255u) + 127) << 23);
-    const float sy = __uint_as_float((uint32_t)((int)(int8_t)((w0.w >> 8) & 255u) + 127) << 23);
-    const float sz = __uint_as_float((uint32_t)((int)(int8_t)((w0.w >> 16) & 255u) + 127) << 23);
-    const int4 ch = make_int4((int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w);
+    const float inf = __int_as_float(0x7f800000);
     float d[4];
-    bool h[4];
+    int cnt = 0;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
+        auto at = [&](const float4& v) { return j == 0 ? v.x : j == 1 ? v.y : j == 2 ? v.z : v.w; };
         const int c = j == 0 ? ch.x : j == 1 ? ch.y : j == 2 ? ch.z : ch.w;
-        h[j] = c != 0 && box_hit(s.cs, dequant(w2.x, j, sx, ox), dequant(w2.y, j, sx, ox), dequant(w2.z, j, sy, oy),
-                                 dequant(w2.w, j, sy, oy), dequant(w3.x, j, sz, oz), dequant(w3.y, j, sz, oz), s.tmin,
-                                 s.best_t, d[j]);
-        if (h[j] && c > 0 && c <= n) { h[j] = false; s.flags |= kBad; }
+        // a used link is a leaf (negative) or a node after this one; anything else (0: unused) is
+        // not followed
+        const bool h = (unsigned)c > (unsigned)n &&
+                       box_hit(s.cs, at(lx), at(hx), at(ly), at(hy), at(lz), at(hz), s.tmin, s.best_t, d[j]);
+        cnt += h;
+        d[j] = h ? d[j] : inf;
     }
-    const int cnt = (int)h[0] + (int)h[1] + (int)h[2] + (int)h[3];
-    const float inf = __int_as_float(0x7f800000);
-    float e0 = h[0] ? d[0] : inf, e1 = h[1] ? d[1] : inf, e2 = h[2] ? d[2] : inf, e3 = h[3] ? d[3] : inf;
-    int c0 = ch.x, c1 = ch.y, c2 = ch.z, c3 = ch.w;
-    order2(e0, c0, e1, c1);
-    order2(e2, c2, e3, c3);
-    order2(e0, c0, e2, c2);
-    order2(e1, c1, e3, c3);
-    order2(e1, c1, e2, c2);
-    if (cnt == 0) {
-        s.node = kNoNode;
-    } else {
-        bool ok = true;
-        if (cnt >= 4) ok &= st.push(c3);
-        if (cnt >= 3) ok &= st.push(c2);
-        if (cnt >= 2) ok &= st.push(c1);
-        if (STATS) s.cd = max(s.cd, (uint32_t)st.sp);
-        if (!ok) s.flags |= kBad;
-        s.node = c0;
-    }
-    resolve_leaf<STATS>(a, s, st.sp);
+    return descend4<BLOCK, STACK_LDS, STATS>(s, st, d[0], d[1], d[2], d[3], ch.x, ch.y, ch.z, ch.w, cnt);
 }
 
-// Advances one ray by one step: bookkeeping (next instance, back to world space, pop) if
-// nothing is pending, then one triangle test or one inner node.  Returns true when the ray
-// is finished.
-template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, bool STATS, int TREE, bool TLK = true>
-__device__ __forceinline__ bool advance(const TraceArgs& a, TraceState& s, LaneStack<BLOCK, STACK_LDS>& st) {
-    if (s.tri < 0 && s.node == kNoNode) {
-        // the current instance's tree is exhausted: next instance of the leaf or world space
-        while (!(s.flags & kTop) && st.sp == s.inst_sp) {
-            if (s.flags & kInstLast) {
-                s.flags |= kTop;
-                to_world(s);
-                s.inst_sp = -1;
-                break;
-            }
-            s.node = enter_instance<STATS>(a, s, s.inst + 1, st.sp);
-            if (s.node != kNoNode) break;
-        }
-        if (s.node == kNoNode) {
-            if (st.sp == 0) return true;
-            s.node = st.pop();
-            resolve_leaf<STATS>(a, s, st.sp);
-        }
+// Origin and steps of a quantized 4-wide node's child bounds (its first 16 bytes); a bound is
+// fma(byte, 2^e, origin).
+struct QuantFrame {
+    float ox, oy, oz, sx, sy, sz;
+    __device__ __forceinline__ explicit QuantFrame(const uint4& w)
+        : ox(__uint_as_float(w.x)), oy(__uint_as_float(w.y)), oz(__uint_as_float(w.z)),
+          sx(ldexpf(1.0f, (int)(int8_t)(w.w & 255u))), sy(ldexpf(1.0f, (int)(int8_t)((w.w >> 8) & 255u))),
+          sz(ldexpf(1.0f, (int)(int8_t)((w.w >> 16) & 255u))) {}
+};
+__device__ __forceinline__ float byte_of(uint32_t word, int k) { return (float)((word >> (8 * k)) & 255u); }
+
+// box_hit for the box whose near and far bounds are byte k* of the words n* and f*: t grows with
+// the bound when the direction's reciprocal is positive and falls when it is negative (fma rounds
+// monotonically), so the bounds chosen by the direction's sign give the min and max of box_hit.
+__device__ __forceinline__ bool quant_box_hit(const TraceState& s, const QuantFrame& q, uint32_t nx, int knx,
+                                              uint32_t fx, int kfx, uint32_t ny, int kny, uint32_t fy, int kfy,
+                                              uint32_t nz, int knz, uint32_t fz, int kfz, float& tnear) {
+    const RaySpace& r = s.cs;
+    const float t0x = fmaf(fmaf(byte_of(nx, knx), q.sx, q.ox), r.idx, -r.oidx);
+    const float t1x = fmaf(fmaf(byte_of(fx, kfx), q.sx, q.ox), r.idx, -r.oidx);
+    const float t0y = fmaf(fmaf(byte_of(ny, kny), q.sy, q.oy), r.idy, -r.oidy);
+    const float t1y = fmaf(fmaf(byte_of(fy, kfy), q.sy, q.oy), r.idy, -r.oidy);
+    const float t0z = fmaf(fmaf(byte_of(nz, knz), q.sz, q.oz), r.idz, -r.oidz);
+    const float t1z = fmaf(fmaf(byte_of(fz, kfz), q.sz, q.oz), r.idz, -r.oidz);
+    tnear = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, s.tmin));
+    return tnear <= fminf(fminf(t1x, t1y), fminf(t1z, s.best_t));
+}
+
+// One node of the quantized 4-wide tree (64 B: origin and exponents, children, 8-bit child
+// bounds per axis); otherwise as node_step4.  The dequantized boxes contain the exact ones.
+template <int BLOCK, int STACK_LDS, bool STATS>
+__device__ __forceinline__ int node_step4q(TraceState& s, LaneStack<BLOCK, STACK_LDS>& st, const uint4& w0,
+                                           const uint4& w1, const uint4& w2, const uint4& w3) {
+    const uint32_t n = (uint32_t)s.item;
+    if (STATS) s.cn++;
+    const QuantFrame q(w0);
+    const bool px = s.cs.idx >= 0.0f, py = s.cs.idy >= 0.0f, pz = s.cs.idz >= 0.0f;
+    const uint32_t nx = px ? w2.x : w2.y, fx = px ? w2.y : w2.x;
+    const uint32_t ny = py ? w2.z : w2.w, fy = py ? w2.w : w2.z;
+    const uint32_t nz = pz ? w3.x : w3.y, fz = pz ? w3.y : w3.x;
+    float d[4];
+    int cnt = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t c = j == 0 ? w1.x : j == 1 ? w1.y : j == 2 ? w1.z : w1.w;
+        const bool h = quant_box_hit(s, q, nx, j, fx, j, ny, j, fy, j, nz, j, fz, j, d[j]) && c > n;
+        cnt += h;
+        d[j] = h ? d[j] : __int_as_float(0x7f800000);
     }
-    if (s.tri >= 0) {
-        const int t = s.tri;
-        if (t + 2 >= a.n_tris4) {
-            s.flags |= kBad;
-            s.tri = -1;
-            return false;
-        }
-        const auto* tris = gview(a.tris);
-        const float4 v0 = tris[t], v1 = tris[t + 1], v2 = tris[t + 2];
-        if (STATS) s.ct++;
-        s.tri = (__float_as_uint(v2.w) == kLeafEnd) ? -1 : t + 3;
-        float th, uh, vh;
-        if (tri_hit(s.cs, v0, v1, v2, th, uh, vh) && th >= s.tmin) {
-            const int tid = __float_as_int(v1.w);
-            if (ANY) {
-                if (th <= s.best_t) {
-                    int op = 1;
-                    if (MASKED) {
-                        op = texel_opaque(a, tid, uh, vh);
-                        if (op & 2) s.flags |= kBad;
-                    }
-                    if (op & 1) {
-                        s.best_t = th; s.best_u = uh; s.best_tri = tid; s.best_inst = s.inst_id;
-                        return true;
-                    }
-                }
+    return descend4<BLOCK, STACK_LDS, STATS>(s, st, d[0], d[1], d[2], d[3], (int)w1.x, (int)w1.y, (int)w1.z, (int)w1.w,
+                                             cnt);
+}
+
+// Whether a hit at t on triangle tid of the current instance replaces the ray's best one.
+template <bool ANY>
+__device__ __forceinline__ bool is_better(const TraceState& s, float t, int tid) {
+    if (ANY) return t <= s.best_t;
+    return t < s.best_t || (t == s.best_t && ((unsigned)tid < (unsigned)s.best_tri ||
+                                              (tid == s.best_tri && (unsigned)s.inst_id < (unsigned)s.best_inst)));
+}
+
+// One triangle of the current leaf; returns true when it is the ray's new best hit.
+template <bool ANY, bool MASKED, bool STATS>
+__device__ __forceinline__ bool tri_step(const TraceArgs& a, TraceState& s, const uint4& r0, const uint4& r1,
+                                         const uint4& r2) {
+    const float4 v0 = as_float4(r0), v1 = as_float4(r1), v2 = as_float4(r2);
+    if (STATS) s.ct++;
+    float th = 0.0f, uh = 0.0f, vh = 0.0f;
+    const int tid = (int)r1.w;
+    bool better = tri_hit(s.cs, v0, v1, v2, th, uh, vh) && th >= s.tmin;
+    better = better && is_better<ANY>(s, th, tid);
+    if (MASKED && better) {
+        const int op = texel_opaque(a, tid, uh, vh);
+        if (op & 2) s.bad = 1;
+        better = op & 1;
+    }
+    s.best_t = better ? th : s.best_t;
+    s.best_u = better ? uh : s.best_u;
+    s.best_tri = better ? tid : s.best_tri;
+    s.best_inst = better ? s.inst_id : s.best_inst;
+    return better;
+}
+
+// A ray whose subtree is done: the next instance of its leaf, or (back in world space if that
+// was the last one) the top of the stack.  Returns false when the ray is finished.
+template <typename POP>
+__device__ __forceinline__ bool resume(TraceState& s, int sp, POP pop) {
+    const bool exhausted = sp == s.inst_sp;
+    const bool leave = exhausted && s.inst_next < 0;
+    if (leave) {
+        to_world(s);
+        s.inst_sp = -1;
+    }
+    const bool again = exhausted && !leave;
+    int link = ~s.inst_next;
+    if (!again) {
+        if (sp == 0) return false;
+        link = pop();
+    }
+    s.kind = link >= 0 ? kNode : (again || s.inst_sp < 0) ? kInst : kTri;
+    s.item = link >= 0 ? link : ~link;
+    return true;
+}
+
+// The instance s.item: its record is fetched and the ray goes to its object space and root node.
+template <bool STATS>
+__device__ __forceinline__ void inst_step(const TraceArgs& a, TraceState& s, int sp) {
+    const uint32_t i = (uint32_t)s.item;
+    if (i < (uint32_t)a.n_inst) {
+        const auto* p = gview(reinterpret_cast<const uint4*>(a.inst)) + 4u * (size_t)i;
+        const uint4 r0 = p[0], r1 = p[1], r2 = p[2], r3 = p[3];
+        s.item = enter_instance<STATS>(s, r0, r1, r2, r3, sp);
+    } else {
+        s.item = -1;  // fails the node's bounds check
+        s.inst_next = -1;
+    }
+    s.kind = kNode;
+}
+
+// Where a node's link leads: an inner node, the first instance of a top-level leaf or the first
+// triangle of a mesh leaf.
+__device__ __forceinline__ void follow(TraceState& s, int link) {
+    s.kind = link >= 0 ? kNode : link == kNoNode ? kNone : s.inst_sp < 0 ? kInst : kTri;
+    s.item = link >= 0 ? link : ~link;
+}
+
+// Advances one ray by one step; returns true when the ray is finished.
+//
+// A step's time is its instructions, not its loads: with one wave per SIMD a step of the
+// quantized tree took about 1,400 cycles of issue and 500 of load latency, and every kind of
+// record that any lane of the wave is at costs the whole wave its code.  So each kind's code
+// appears once per step, and a step takes a ray as far as one pass over that code can:
+//   4-wide trees  one triangle, then (if that ended the leaf) the next thing off the stack, an
+//                 instance entry and a node.  A ray's steps are its nodes plus the triangles after
+//                 the first of a leaf.  Postponing triangles or instances until more lanes
+//                 of the wave hold one made every workload slower (13-60%): a wave lasts as long
+//                 as its longest ray.
+//   BVH2          an instance entry, then one triangle or one node, whose records are loaded
+//                 together.  Nodes are cheap here and twice as many, so a second load latency in
+//                 the step costs more than the steps it saves (1M primary rays over 65K triangles:
+//                 440 us against 553 us).
+// MI355X, us per launch before (an instance entry and a pop in three places, one node or
+// triangle per step) -> now: 1M primary rays, 65K triangles, quantized 551 -> 360, BVH2 590 ->
+// 438; 300K diffuse rays, 250K triangles, quantized 537 -> 385; 200K rays over masked, rotated
+// instances, quantized 1,216 -> 809; any hit, 1M shadow rays, BVH2 820 -> 653.
+template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, bool STATS, int TREE>
+__device__ __forceinline__ bool advance(const TraceArgs& a, TraceState& s, LaneStack<BLOCK, STACK_LDS>& st) {
+    if constexpr (TREE != 0) {
+        if (s.kind == kTri) {
+            bool end = true;
+            if (s.item < a.n_tris4 - 2) {
+                const auto* p = gview(reinterpret_cast<const uint4*>(a.tris)) + (size_t)(uint32_t)s.item;
+                const uint4 r0 = p[0], r1 = p[1], r2 = p[2];
+                const bool better = tri_step<ANY, MASKED, STATS>(a, s, r0, r1, r2);
+                if (ANY && better) return true;
+                end = r2.w == kLeafEnd;
             } else {
-                const bool better = th < s.best_t ||
-                    (th == s.best_t && ((unsigned)tid < (unsigned)s.best_tri ||
-                                        (tid == s.best_tri && (unsigned)s.inst_id < (unsigned)s.best_inst)));
-                if (better) {
-                    int op = 1;
-                    if (MASKED) {
-                        op = texel_opaque(a, tid, uh, vh);
-                        if (op & 2) s.flags |= kBad;
-                    }
-                    if (op & 1) {
-                        s.best_t = th; s.best_u = uh; s.best_tri = tid; s.best_inst = s.inst_id;
-                    }
-                }
+                s.bad = 1;
             }
+            s.item += 3;
+            s.kind = end ? kNone : kTri;
+        }
+        if (s.kind == kNone && !resume(s, st.sp, [&] { return st.pop(); })) return true;
+        if (s.kind == kInst) inst_step<STATS>(a, s, st.sp);
+        if (s.kind == kNode) {
+            int next = kNoNode;
+            if ((uint32_t)s.item < (uint32_t)a.n_nodes) {
+                const auto* p = gview(reinterpret_cast<const uint4*>(a.nodes)) +
+                                (TREE == 1 ? 8u : 4u) * (size_t)(uint32_t)s.item;
+                const uint4 r0 = p[0], r1 = p[1], r2 = p[2], r3 = p[3];
+                if constexpr (TREE == 2) next = node_step4q<BLOCK, STACK_LDS, STATS>(s, st, r0, r1, r2, r3);
+                else next = node_step4<BLOCK, STACK_LDS, STATS>(a, s, st, r0, r1, r2, r3);
+            } else {
+                s.bad = 1;
+            }
+            follow(s, next);
         }
         return false;
+    } else {
+        if (s.kind == kInst) inst_step<STATS>(a, s, st.sp);
+        const int kind = s.kind;
+        const char* base = (const char*)(kind == kNode ? a.nodes : a.tris);
+        const uint32_t limit = (uint32_t)(kind == kNode ? a.n_nodes : max(a.n_tris4 - 2, 0));
+        const int shift = kind == kTri ? 4 : 6;
+        const bool ok = (uint32_t)s.item < limit;
+        uint4 r0, r1, r2, r3;
+        if (ok) {
+            const auto* p = gview(reinterpret_cast<const uint4*>(base + ((uint64_t)(uint32_t)s.item << shift)));
+            r0 = p[0]; r1 = p[1]; r2 = p[2];
+            if (kind == kNode) r3 = p[3];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        int next = kNoNode;  // link to go on with, or
+        bool list = false;   // the next triangle of the leaf
+        if (!ok) {
+            s.bad = 1;
+        } else if (kind == kTri) {
+            const bool better = tri_step<ANY, MASKED, STATS>(a, s, r0, r1, r2);
+            if (ANY && better) return true;
+            list = r2.w != kLeafEnd;
+        } else {
+            next = node_step2<BLOCK, STACK_LDS, STATS>(s, st, r0, r1, r2, r3);
+        }
+        const int item = s.item + 3;
+        follow(s, next);
+        s.kind = list ? kTri : s.kind;
+        s.item = list ? item : s.item;
+        return s.kind == kNone && !resume(s, st.sp, [&] { return st.pop(); });
     }
-    if (s.node >= 0) {
-        if (TREE == 2) node_step4q<BLOCK, STACK_LDS, STATS, TLK>(a, s, st);
-        else if (TREE == 1) node_step4<BLOCK, STACK_LDS, STATS>(a, s, st);
-        else node_step2<BLOCK, STACK_LDS, STATS>(a, s, st);
-    }
-    return false;
 }
 
 template <int BLOCK, int STACK_LDS>
@@ -584,22 +611,6 @@ __device__ __forceinline__ void stack_init(LaneStack<BLOCK, STACK_LDS>& st, int*
     st.spill_slot = blockIdx.x * BLOCK + threadIdx.x;
     st.spill_stride = gridDim.x * BLOCK;
     st.sp = 0;
-    st.tl = nullptr;
-}
-
-// Copies the treelet nodes of a quantized-tree launch into the block's dynamic LDS (sized by
-// the host for a.tl_nodes nodes).  a.tl_nodes is the same for every thread of the grid.  The
-// copy keeps the node layout: a word-major copy (fewer LDS bank conflicts between lanes
-// reading different nodes) needs a runtime stride that costs the kernel 7 VGPRs and one wave
-// per SIMD, more than the conflicts cost.
-template <int BLOCK, int STACK_LDS, int TREE>
-__device__ __forceinline__ void treelet_init(const TraceArgs& a, LaneStack<BLOCK, STACK_LDS>& st) {
-    extern __shared__ uint4 treelet_lds[];
-    if (TREE != 2 || a.tl_nodes <= 0) return;
-    const uint4* src = reinterpret_cast<const uint4*>(a.nodes) + 4 * (size_t)a.tl_base;
-    for (int i = threadIdx.x; i < 4 * a.tl_nodes; i += BLOCK) treelet_lds[i] = src[i];
-    __syncthreads();
-    st.tl = treelet_lds;
 }
 
 template <bool STATS>
@@ -611,23 +622,18 @@ __device__ __forceinline__ void write_result(const TraceArgs& a, const TraceStat
         a.counts[3 * (size_t)id + 2] = s.ci;
     }
     if (STATS && a.depth_hist) atomicAdd(&a.depth_hist[min(s.cd, 63u)], 1u);
-    if (s.flags & kBad) atomicAdd(a.err, 1);
+    if (s.bad) atomicAdd(a.err, 1);
 }
 
-// One ray per thread (rays strided over the grid when it is smaller than the ray count).
-// The 4-wide variants are held to 7 waves per SIMD (72 VGPRs, a few bytes of scratch per
-// lane): faster than their natural 6 (77 VGPRs; PT frames 4% faster with the any-hit variant
-// held too) and, for closest hit, than 8 (64 VGPRs, more spills: 9% slower).
+// One ray per thread (rays strided over the grid when it is smaller than the ray count).  The 4-wide variants are held to 7 waves per SIMD
+// (72 VGPRs), the BVH2 ones to 8 (64).
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, bool STATS, int TREE>
-__global__ __launch_bounds__(BLOCK, (MASKED || STATS || TREE == 0) ? 1 : 7) void k_trace(TraceArgs a) {
+__global__ __launch_bounds__(BLOCK, STATS ? 1 : TREE == 0 ? 8 : 7) void k_trace(TraceArgs a) {
     __shared__ int lds_stack[STACK_LDS * BLOCK];
     const int count = launch_count(a);
-    // a block past the rays (a launch sized for the capacity of a queue whose size is read on
-    // the device) leaves before it copies the treelet: block-uniform, before any barrier
-    if ((int)(blockIdx.x * BLOCK) >= count) return;
+    if ((int)(blockIdx.x * BLOCK) >= count) return;  // sized for the capacity of a device-side count
     LaneStack<BLOCK, STACK_LDS> st;
     stack_init(st, lds_stack, a);
-    treelet_init<BLOCK, STACK_LDS, TREE>(a, st);
     const int stride = gridDim.x * BLOCK;
     for (int id = blockIdx.x * BLOCK + threadIdx.x; id < count; id += stride) {
         TraceState s;
@@ -649,7 +655,6 @@ __global__ __launch_bounds__(BLOCK) void k_trace_dyn(TraceArgs a, int refill) {
     __shared__ int lds_stack[STACK_LDS * BLOCK];
     LaneStack<BLOCK, STACK_LDS> st;
     stack_init(st, lds_stack, a);
-    treelet_init<BLOCK, STACK_LDS, TREE>(a, st);
     const int lane = __lane_id();
     int* counter = a.work_counter;
     int id = -1;             // ray of this lane, -1 = none
@@ -759,16 +764,11 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchGr
     }
 }
 
-// TL (quantized tree, tl_max > 0): every wave keeps its own LDS copy of the first
-// min(tl_max, a.tl_nodes) treelet nodes of the scene of its current chunk (tl_max x 64 B per
-// wave of dynamic LDS), reloaded when a chunk of another scene comes.  The 4-wide variants
-// are held to 7 waves per SIMD (72 VGPRs, a few bytes of scratch per lane), faster than their
-// natural 6.
-template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE, bool TL>
-__global__ __launch_bounds__(BLOCK, MASKED ? 1 : (TREE == 0 && !ANY ? 8 : 7)) void k_trace_batch(const BatchItem* __restrict__ items, int first, int n_items,
-                                                       const int* __restrict__ total_chunks, int* counter, int* spill,
-                                                       int spill_depth, int tl_max) {
-    extern __shared__ uint4 treelet_lds[];
+// The 4-wide variants are held to 7 waves per SIMD (72 VGPRs), the BVH2 ones to 8.
+template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE>
+__global__ __launch_bounds__(BLOCK, TREE == 0 ? 8 : 7) void k_trace_batch(
+    const BatchItem* __restrict__ items, int first, int n_items, const int* __restrict__ total_chunks, int* counter,
+    int* spill, int spill_depth) {
     __shared__ int lds_stack[STACK_LDS * BLOCK];
     LaneStack<BLOCK, STACK_LDS> st;
     st.lds = lds_stack;
@@ -778,9 +778,6 @@ __global__ __launch_bounds__(BLOCK, MASKED ? 1 : (TREE == 0 && !ANY ? 8 : 7)) vo
     st.spill_slot = blockIdx.x * BLOCK + threadIdx.x;
     st.spill_stride = gridDim.x * BLOCK;
     st.sp = 0;
-    st.tl = TL ? treelet_lds + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6) * 4 * tl_max) : nullptr;
-    const float4* tl_nodes_of = nullptr;  // scene (node array) whose treelet this wave holds
-    int tl_base_of = -1;
     const int lane = __lane_id();
     const int total = __builtin_amdgcn_readfirstlane(*total_chunks);
     for (;;) {
@@ -797,30 +794,13 @@ __global__ __launch_bounds__(BLOCK, MASKED ? 1 : (TREE == 0 && !ANY ? 8 : 7)) vo
             else hi = mid - 1;
         }
         lo = __builtin_amdgcn_readfirstlane(lo);
-        TraceArgs a = items[lo].a;
-        if (TL) {
-            a.tl_nodes = min(a.tl_nodes, tl_max);
-            if (a.nodes != tl_nodes_of || a.tl_base != tl_base_of) {  // wave-uniform
-                // the wave's earlier LDS reads are complete before the copy is overwritten
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                uint4* w = const_cast<uint4*>(st.tl);
-                const uint4* src = reinterpret_cast<const uint4*>(a.nodes) + 4 * (size_t)a.tl_base;
-                for (int i = lane; i < 4 * a.tl_nodes; i += 64) w[i] = src[i];
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                tl_nodes_of = a.nodes;
-                tl_base_of = a.tl_base;
-            }
-        } else {
-            a.tl_nodes = 0;
-        }
+        const TraceArgs a = items[lo].a;
         const int id = (c - items[lo].chunk_begin) * 64 + lane;
         if (id < a.count) {
             TraceState s;
             state_init(s, gview(a.rays)[2 * (size_t)id], gview(a.rays)[2 * (size_t)id + 1], a.root);
             st.sp = 0;
-            while (!advance<BLOCK, STACK_LDS, ANY, MASKED, false, TREE, TL>(a, s, st)) {
+            while (!advance<BLOCK, STACK_LDS, ANY, MASKED, false, TREE>(a, s, st)) {
             }
             write_result<false>(a, s, id);
         }

@@ -78,23 +78,22 @@ int launch_one(const TraceArgs& args_in, int max_stack, int blocks_per_cu, int r
     const bool dyn = refill > 0;
     void (*kern)(TraceArgs) = k_trace<BLOCK, STACK_LDS, ANY, MASKED, STATS, TREE>;
     void (*kern_dyn)(TraceArgs, int) = k_trace_dyn<BLOCK, STACK_LDS, ANY, MASKED, STATS, TREE>;
-    const size_t tl_bytes = TREE == 2 ? (size_t)a.tl_nodes * 64 : 0;  // dynamic LDS: the treelet copy
-    if (TREE != 2) a.tl_nodes = 0;
-    int resident = 0;
-    if (dyn)
-        IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern_dyn, BLOCK, tl_bytes));
-    else
-        IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, BLOCK, tl_bytes));
-    if (resident <= 0) resident = 1;
-    if (blocks_per_cu > 0) resident = std::min(resident, blocks_per_cu);
     const int needed = ceil_div(a.count, BLOCK);
-    // One thread per ray, so that the dispatcher starts a new block wherever one finishes (the
-    // rays of a wave end at very different times); a grid capped at the resident blocks, each
-    // thread striding over several rays, left the SIMDs a quarter occupied on average and was
-    // 4% slower on the path-tracing queues.  The persistent variant and an explicit
-    // blocks_per_cu keep the resident-sized grid.
-    const int grid = (dyn || blocks_per_cu > 0) ? std::max(1, std::min(needed, resident * p->cu_count))
-                                                : std::max(1, needed);
+    int grid = std::max(1, needed);
+    if (dyn || blocks_per_cu > 0) {
+        // The persistent variant and an explicit blocks_per_cu take a grid of resident blocks.
+        int resident = 0;
+        if (dyn)
+            IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern_dyn, BLOCK, 0));
+        else
+            IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, BLOCK, 0));
+        if (resident <= 0) resident = 1;
+        if (blocks_per_cu > 0) resident = std::min(resident, blocks_per_cu);
+        grid = std::max(1, std::min(needed, resident * p->cu_count));
+    }  // else one thread per ray, so that the dispatcher starts a new block wherever one finishes (the
+       // rays of a wave end at very different times); a grid capped at the resident blocks, each
+       // thread striding over several rays, left the SIMDs a quarter occupied on average and was
+       // 4% slower on the path-tracing queues
     a.spill = nullptr;
     a.spill_depth = 0;
     if (max_stack > STACK_LDS) {
@@ -118,19 +117,19 @@ int launch_one(const TraceArgs& args_in, int max_stack, int blocks_per_cu, int r
         }
         int r = counter_slot(p->device & 63, is_capturing(s), &a.work_counter);
         if (r) return r;
-        hipLaunchKernelGGL(kern_dyn, dim3(grid), dim3(BLOCK), tl_bytes, s, a, std::min(refill, 64));
+        hipLaunchKernelGGL(kern_dyn, dim3(grid), dim3(BLOCK), 0, s, a, std::min(refill, 64));
     } else {
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), tl_bytes, s, a);
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), 0, s, a);
     }
     IMBA_HIP_TRY(hipGetLastError());
     return IMBA_OK;
 }
 
 // Default launch: 256 threads, 16 LDS stack entries per lane, one ray per thread (measured
-// fastest on both the 65K-triangle and the 21M-triangle workloads; see DESIGN.md).
+// fastest on both the 65K-triangle and the 21M-triangle workloads).
 constexpr int kDefaultBlock = 256;
-constexpr int kBatchTreeletMax = 64;  // batches: nodes per wave's LDS treelet copy (larger requests clamp)
 constexpr int kDefaultStack = 16;
+
 constexpr int kDefaultWidth = 2;
 
 // Tree a configuration asks for: 0 the BVH2, 1 the 4-wide tree, 2 its quantized form; -1 if
@@ -141,9 +140,15 @@ int tree_code(const ImbaTraceConfig* cfg) {
     if (w == 4) return (cfg && cfg->quantized) ? 2 : 1;
     return -1;
 }
-int width_of(const ImbaTraceConfig* cfg) {
-    const int t = tree_code(cfg);
-    return t < 0 ? 0 : (t == 0 ? 2 : 4);
+
+// The treelet size of a configuration (accepted for the quantized tree, without effect: every
+// node is read through the caches, which hold the top levels anyway).
+int check_treelet(const ImbaTraceConfig* cfg) {
+    if (!cfg || !cfg->treelet) return IMBA_OK;
+    if (cfg->treelet < 0 || cfg->treelet > kTreeletMaxNodes)
+        return fail(IMBA_ERR_INVALID_ARG, "treelet must be 0..%d nodes", kTreeletMaxNodes);
+    if (tree_code(cfg) != 2) return fail(IMBA_ERR_INVALID_ARG, "treelet needs the quantized 4-wide tree");
+    return IMBA_OK;
 }
 
 template <bool ANY, bool MASKED, bool STATS, int TREE>
@@ -211,14 +216,9 @@ int launch_trace(const TreeView& t, int* d_err, const ImbaRay* rays, ImbaHit* hi
     a.depth_hist = depth_hist;
     a.err = d_err;
     const bool stats = counts || depth_hist;
-    if (cfg && cfg->treelet) {
-        if (cfg->treelet < 0 || cfg->treelet > kTreeletMaxNodes)
-            return fail(IMBA_ERR_INVALID_ARG, "treelet must be 0..%d nodes", kTreeletMaxNodes);
-        if (t.tree != 2) return fail(IMBA_ERR_INVALID_ARG, "treelet needs the quantized 4-wide tree");
-        if (!stats) {  // visit counts do not depend on where a node is read from
-            a.tl_base = t.info->treelet_base;
-            a.tl_nodes = std::min(cfg->treelet, t.info->treelet_nodes);
-        }
+    {
+        const int r = check_treelet(cfg);
+        if (r) return r;
     }
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
@@ -239,8 +239,8 @@ int launch_trace(const TreeView& t, int* d_err, const ImbaRay* rays, ImbaHit* hi
 }
 
 // The tree of `s` that `cfg` asks for.
-int pick_tree(const ImbaTraceConfig* cfg, const ImbaSceneDesc* d2, const SceneInfo* i2, const ImbaSceneDesc* d4,
-              const ImbaSceneDesc* d4q, const SceneInfo* i4, TreeView* t) {
+int pick_tree(const ImbaTraceConfig* cfg, const ImbaSceneDesc* d2, const SceneInfo* i2,
+              const ImbaSceneDesc* d4, const ImbaSceneDesc* d4q, const SceneInfo* i4, TreeView* t) {
     const int code = tree_code(cfg);
     if (code < 0) return fail(IMBA_ERR_INVALID_ARG, "bvh_width must be 0, 2 or 4 (quantized only with 4)");
     if (code == 2 && !d4q->nodes) return fail(IMBA_ERR_INVALID_ARG, "the scene has no quantized 4-wide tree");
@@ -378,19 +378,13 @@ namespace imba {
 namespace {
 
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE>
-int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, int tl_max, hipStream_t s) {
+int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, hipStream_t s) {
     const DeviceProps* p = device_props();
     if (!p) return fail(IMBA_ERR_NO_DEVICE, "no HIP device");
-    auto kern = k_trace_batch<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>;
-    if constexpr (TREE == 2) {
-        if (tl_max > 0) kern = k_trace_batch<BLOCK, STACK_LDS, ANY, MASKED, TREE, true>;
-    } else {
-        tl_max = 0;
-    }
+    auto kern = k_trace_batch<BLOCK, STACK_LDS, ANY, MASKED, TREE>;
     const int max_stack = b->max_stack[TREE ? 1 : 0][g];
-    const size_t tl_bytes = (size_t)(BLOCK / 64) * tl_max * 64;  // one treelet copy per wave
     int resident = 0;
-    IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, BLOCK, tl_bytes));
+    IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, BLOCK, 0));
     if (resident <= 0) resident = 1;
     if (blocks_per_cu > 0) resident = std::min(resident, blocks_per_cu);
     const long long needed = (b->capacity_chunks[g] * 64 + BLOCK - 1) / BLOCK;
@@ -408,9 +402,9 @@ int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, int tl_max, 
         }
         spill = (int*)b->spill[g].ptr;
     }
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), tl_bytes, s, b->d_items[TREE], b->groups.first[g],
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), 0, s, b->d_items[TREE], b->groups.first[g],
                        b->groups.first[g + 1] - b->groups.first[g], b->d_group_chunks + g, b->d_counters + 2 * g,
-                       spill, spill_depth, tl_max);
+                       spill, spill_depth);
     IMBA_HIP_TRY(hipGetLastError());
     return IMBA_OK;
 }
@@ -420,9 +414,8 @@ int dispatch_batch(ImbaTraceBatch* b, int g, const ImbaTraceConfig* cfg, hipStre
     const int block = cfg && cfg->block_size ? cfg->block_size : kDefaultBlock;
     const int stack = cfg && cfg->stack_lds ? cfg->stack_lds : kDefaultStack;
     const int bpc = cfg ? cfg->blocks_per_cu : 0;
-    const int tl = cfg ? std::min(cfg->treelet, kBatchTreeletMax) : 0;
 #define IMBA_SHAPE(B, S) \
-    if (block == B && stack == S) return launch_batch_group<B, S, ANY, MASKED, TREE>(b, g, bpc, tl, s);
+    if (block == B && stack == S) return launch_batch_group<B, S, ANY, MASKED, TREE>(b, g, bpc, s);
     IMBA_SHAPE(256, 16)
     IMBA_SHAPE(256, 8)
     IMBA_SHAPE(256, 32)
@@ -492,8 +485,6 @@ int set_tables(ImbaTraceBatch* b, const ImbaTraceItem* items, int n_items, hipSt
             table4.push_back(e);
             if (it.scene->dev4q.nodes) e.a.nodes = (const float4*)it.scene->dev4q.nodes;
             else quantized_ok = false;
-            e.a.tl_base = it.scene->info4.treelet_base;
-            e.a.tl_nodes = it.scene->info4.treelet_nodes;
             table4q.push_back(e);
         }
     }
@@ -611,11 +602,8 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
     const int tree = tree_code(cfg);
     if (tree < 0) return fail(IMBA_ERR_INVALID_ARG, "bvh_width must be 0, 2 or 4 (quantized only with 4)");
     if (tree == 2 && !b->quantized_ok) return fail(IMBA_ERR_INVALID_ARG, "a queue's scene has no quantized tree");
-    if (cfg && cfg->treelet) {
-        if (cfg->treelet < 0 || cfg->treelet > kTreeletMaxNodes)
-            return fail(IMBA_ERR_INVALID_ARG, "treelet must be 0..%d nodes", kTreeletMaxNodes);
-        if (tree != 2) return fail(IMBA_ERR_INVALID_ARG, "treelet needs the quantized 4-wide tree");
-    }
+    int r = check_treelet(cfg);
+    if (r) return r;
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
     if (is_capturing(s)) {
@@ -626,7 +614,6 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
     IMBA_HIP_TRY(hipGetLastError());
     for (int g = 0; g < 4; g++) {
         if (b->groups.first[g + 1] == b->groups.first[g] || b->capacity_chunks[g] == 0) continue;
-        int r;
         switch (g + 4 * tree) {
             case 0: r = dispatch_batch<false, false, 0>(b, g, cfg, s); break;
             case 1: r = dispatch_batch<false, true, 0>(b, g, cfg, s); break;
@@ -653,8 +640,8 @@ int imba_autotune(const ImbaScene* sc, const ImbaRay* rays, ImbaHit* hits, int c
     IMBA_CHECK_ARG(count > 0 && reps > 0, "count and reps must be positive");
     static const int kShapes[][2] = {{256, 16}, {256, 8}, {256, 32}, {128, 16}, {128, 32}, {64, 32}, {64, 64}};
     static const int kRefill[] = {0, 32};
-    // bvh_width, quantized, treelet nodes staged in LDS
-    static const int kTree[][3] = {{2, 0, 0}, {4, 0, 0}, {4, 1, 0}, {4, 1, 64}, {4, 1, 256}};
+    // bvh_width, quantized
+    static const int kTree[][2] = {{2, 0}, {4, 0}, {4, 1}};
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -665,9 +652,8 @@ int imba_autotune(const ImbaScene* sc, const ImbaRay* rays, ImbaHit* hits, int c
     for (const auto& tree : kTree)
     for (const auto& shape : kShapes) {
         for (int refill : kRefill) {
-            ImbaTraceConfig cfg{shape[0], shape[1], refill, 0, tree[0], tree[1], tree[2]};
+            ImbaTraceConfig cfg{shape[0], shape[1], refill, 0, tree[0], tree[1], 0};
             if (tree[1] && !sc->dev4q.nodes) continue;
-            if (tree[2] && sc->info4.treelet_nodes <= 0) continue;
             TreeView t{};
             r = tree_of(sc, &cfg, &t);
             if (!r)

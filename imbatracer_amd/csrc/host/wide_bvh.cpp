@@ -8,7 +8,7 @@
 // the absorbed inner nodes are no longer tested, and each step tests four boxes instead of
 // two.  Node layout: ImbaNode4 (box j of child j as min/max per axis, children[j]: > 0 node,
 // < 0 leaf link as in the BVH2, 0 unused slot).  The first kTreeletMaxNodes nodes of a tree
-// are its top levels in breadth-first order, the rest follow in preorder (a child always
+// are its top levels in breadth-first order (together in the caches), the rest follow in preorder (a child always
 // follows its parent); mesh trees come first (in increasing BVH2 root order), then the top
 // level.  Instance records are copied with `next` pointing at the mesh's 4-wide root.
 #include <algorithm>
@@ -149,17 +149,6 @@ int collapse_scene4(const ImbaSceneDesc& d, WideScene& out) {
     int top_pushes = 0;
     out.root = collapse_tree(d, d.root, out.nodes, &top_pushes);
     if (out.root < 0) return fail(IMBA_ERR_BAD_BVH, "top level has links out of range");
-    // the treelet: the top level, or the mesh when the top level reaches one instance only
-    int reached = 0, only = -1;
-    for (int i = 0; i < d.instance_count; i++)
-        if (used[i]) { reached++; only = i; }
-    int base = out.root, end = (int)out.nodes.size();
-    if (reached == 1) {  // the only mesh tree spans the nodes before the top level
-        base = root_map[d.instances[only].next];
-        end = out.root;
-    }
-    out.treelet_base = base;
-    out.treelet_nodes = std::min(kTreeletMaxNodes, end - base);
     out.instances.assign(d.instances, d.instances + d.instance_count);
     for (int i = 0; i < d.instance_count; i++) out.instances[i].next = used[i] ? root_map[d.instances[i].next] : -1;
     // stack entries of the top level stay while a ray is inside a mesh tree
@@ -218,8 +207,19 @@ bool quantize_nodes(WideScene& w) {
         while (k < 4 && n.children[k] != 0) k++;
         q.count = (uint8_t)k;
         for (int j = 0; j < 4; j++) q.children[j] = n.children[j];
-        const float* lo[3] = {n.min_x, n.min_y, n.min_z};
-        const float* hi[3] = {n.max_x, n.max_y, n.max_z};
+        // a box given with its bounds the wrong way round is the slab between them to every
+        // traversal; the kernel takes the near bound by the ray's direction, so the bytes are ordered
+        float lo[3][4], hi[3][4];
+        for (int j = 0; j < k; j++) {
+            for (float v : {n.min_x[j], n.max_x[j], n.min_y[j], n.max_y[j], n.min_z[j], n.max_z[j]})
+                if (!std::isfinite(v)) {
+                    w.qnodes.clear();
+                    return false;
+                }
+            lo[0][j] = std::min(n.min_x[j], n.max_x[j]), hi[0][j] = std::max(n.min_x[j], n.max_x[j]);
+            lo[1][j] = std::min(n.min_y[j], n.max_y[j]), hi[1][j] = std::max(n.min_y[j], n.max_y[j]);
+            lo[2][j] = std::min(n.min_z[j], n.max_z[j]), hi[2][j] = std::max(n.min_z[j], n.max_z[j]);
+        }
         uint8_t* qlo[3] = {q.lo_x, q.lo_y, q.lo_z};
         uint8_t* qhi[3] = {q.hi_x, q.hi_y, q.hi_z};
         for (int a = 0; a < 3; a++) {

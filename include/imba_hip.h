@@ -289,9 +289,8 @@ typedef struct ImbaTraceConfig {
                               it at upload (same leaves); 0 = default                      */
     int quantized;         /* with bvh_width 4: 64-byte nodes whose child boxes are 8-bit
                               offsets from the node box, rounded outward                  */
-    int treelet;           /* quantized tree only: nodes of its top levels (0..256) each
-                              block copies into LDS and reads from there (0 = none);
-                              batches keep one copy per wave, of at most 64 nodes        */
+    int treelet;           /* quantized tree only, 0..256: accepted, without effect (every node
+                              is read through the caches)                                  */
 } ImbaTraceConfig;
 
 int imba_intersect(const ImbaScene* s, const ImbaRay* rays, ImbaHit* hits, int count,
@@ -362,7 +361,7 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
 int imba_trace_batch_release(ImbaTraceBatch* b);
 
 /* Launch shape autotuning: times every supported shape (static and persistent) of every tree
- * (BVH2, 4-wide, quantized with LDS treelets of 0 / 64 / 256 nodes) on the given device queue
+ * (BVH2, 4-wide, quantized) on the given device queue
  * with HIP events, `reps` launches each after one warm-up, and returns the fastest in *best
  * (and its mean time per launch in *best_ms, nullable).  Results do not depend on the shape. */
 int imba_autotune(const ImbaScene* s, const ImbaRay* rays, ImbaHit* hits, int count, int any_hit, int reps,

@@ -176,3 +176,17 @@ def test_top_levels_breadth_first(name, build):
             order.append(k)
             queue += [int(c) for c in nodes[k]["children"] if c > 0]
         assert order == list(range(root, root + len(order)))
+
+
+def test_quantized_bytes_are_ordered():
+    """A child box given with its bounds the wrong way round is the slab between them: its
+    quantized bytes are those of the box with the bounds in order."""
+    b, _, _ = T.random_tri_scene(500)
+    a = b.arrays()
+    want = S.wide_tree(a)["qnodes"]
+    swapped = {k: (v.copy() if isinstance(v, np.ndarray) else v) for k, v in a.items()}
+    bb = swapped["nodes"]["left_bb"]
+    leaf = swapped["nodes"]["left"] < 0
+    assert leaf.sum() > 50
+    bb["lo_x"][leaf], bb["hi_x"][leaf] = a["nodes"]["left_bb"]["hi_x"][leaf], a["nodes"]["left_bb"]["lo_x"][leaf]
+    assert np.array_equal(S.wide_tree(swapped)["qnodes"], want)
