@@ -47,6 +47,7 @@ struct TraceArgs {
     int spill_depth;      // spill entries per thread
     int* work_counter;    // persistent variant: next ray to fetch
     const int* count_dev; // device ray count read when the launch runs (<= count), or null
+    int quad;             // quantized tree: a launch of at most this many rays gives each ray four lanes
 };
 
 // Rays of this launch: count, or the device count clamped to [0, count].
@@ -613,6 +614,141 @@ __device__ __forceinline__ void stack_init(LaneStack<BLOCK, STACK_LDS>& st, int*
     st.sp = 0;
 }
 
+// ---------------------------------------------------------------------------------------
+// Four lanes per ray (quantized tree, small queues).  The lanes of a quad hold the same ray and
+// go through the same steps; lane j tests child box j of a node and triangle j of a leaf, and
+// the quad sorts with DPP exchanges.  A step is then about half the instructions, a wave lasts
+// as long as the longest of 16 rays instead of 64, and a queue that would leave SIMDs with one
+// wave or none spreads over four times the waves.  Visiting order, and so every hit, is that
+// of `advance`.  The stack of a quad has the LDS of its four lanes (4 * STACK_LDS entries).
+// MI355X, us per launch, one lane -> four lanes per ray, quantized tree, 65K triangles: 1,000
+// diffuse rays 186 -> 111, 16,000: 209 -> 116, 65,000: 216 -> 153, 130,000: 203 -> 243; primary
+// rays 16,000: 167 -> 95, 130,000: 162 -> 133; shadow rays 65,000: 156 -> 122, 130,000: 161 ->
+// 187; 1M primary rays 360 -> 694 (the chip is full and four lanes do more work per ray).
+// Lane (4 q + k) receives the value of lane 4 q + {A, B, C, D}[k].
+template <int A, int B, int C, int D>
+__device__ __forceinline__ uint32_t quad_u(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, A | (B << 2) | (C << 4) | (D << 6), 0xF, 0xF, false);
+}
+template <int A, int B, int C, int D>
+__device__ __forceinline__ float quad_f(float v) {
+    return __uint_as_float(quad_u<A, B, C, D>(__float_as_uint(v)));
+}
+
+// Compare-exchange of (distance, link) between the lanes of a pair, as order2: the pair's low lane
+// keeps the nearer, its own on a tie.
+template <int A, int B, int C, int D>
+__device__ __forceinline__ void quad_order(float& d, uint32_t& c, bool low) {
+    const float od = quad_f<A, B, C, D>(d);
+    const uint32_t oc = quad_u<A, B, C, D>(c);
+    const bool take = low ? od < d : d < od;
+    d = take ? od : d;
+    c = take ? oc : c;
+}
+
+// A candidate hit of the lane against that of another lane of the quad: the smaller (t, triangle
+// id), or for any hit the earlier one of the list (from = lane + 1, 0: no candidate).
+struct Candidate {
+    float t, u;
+    uint32_t tri, from;
+};
+template <bool ANY, int A, int B, int C, int D>
+__device__ __forceinline__ void quad_best(Candidate& c) {
+    const float t = quad_f<A, B, C, D>(c.t), u = quad_f<A, B, C, D>(c.u);
+    const uint32_t tri = quad_u<A, B, C, D>(c.tri), from = quad_u<A, B, C, D>(c.from);
+    const bool nearer = ANY ? from < c.from : t < c.t || (t == c.t && (tri < c.tri || (tri == c.tri && from < c.from)));
+    const bool take = from != 0 && (c.from == 0 || nearer);
+    c.t = take ? t : c.t;
+    c.u = take ? u : c.u;
+    c.tri = take ? tri : c.tri;
+    c.from = take ? from : c.from;
+}
+
+// One step of a quad's ray, as `advance` for the quantized tree; stack is the quad's column
+// ([depth][BLOCK / 4]), j the lane's place in the quad.
+template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED>
+__device__ __forceinline__ bool advance_quad(const TraceArgs& a, TraceState& s, int* stack, int& sp, int j) {
+    constexpr int kQuads = BLOCK / 4;
+    if (s.kind == kTri) {
+        const int t = s.item + 3 * j;
+        const bool in = t < a.n_tris4 - 2;
+        uint4 r0 = {}, r1 = {}, r2 = {};
+        r2.w = kLeafEnd;
+        if (in) {
+            const auto* p = gview(reinterpret_cast<const uint4*>(a.tris)) + (size_t)(uint32_t)t;
+            r0 = p[0]; r1 = p[1]; r2 = p[2];
+        }
+        // the triangles after the leaf's last one belong to another leaf
+        const uint32_t e = r2.w == kLeafEnd ? 1u : 0u;
+        const uint32_t e0 = quad_u<0, 0, 0, 0>(e), e1 = quad_u<1, 1, 1, 1>(e), e2 = quad_u<2, 2, 2, 2>(e),
+                       e3 = quad_u<3, 3, 3, 3>(e);
+        const bool mine = !((j > 0 && e0) || (j > 1 && e1) || (j > 2 && e2));
+        if (mine && !in) s.bad = 1;
+        float th = 0.0f, uh = 0.0f, vh = 0.0f;
+        const uint32_t tid = r1.w;
+        bool better = mine && in && tri_hit(s.cs, as_float4(r0), as_float4(r1), as_float4(r2), th, uh, vh) &&
+                      th >= s.tmin;
+        better = better && is_better<ANY>(s, th, (int)tid);
+        if (MASKED && better) {
+            const int op = texel_opaque(a, (int)tid, uh, vh);
+            if (op & 2) s.bad = 1;
+            better = op & 1;
+        }
+        if (__ballot(better)) {
+            Candidate c{th, uh, tid, better ? (uint32_t)j + 1u : 0u};
+            quad_best<ANY, 1, 0, 3, 2>(c);
+            quad_best<ANY, 2, 3, 0, 1>(c);
+            const bool hit = c.from != 0;
+            s.best_t = hit ? c.t : s.best_t;
+            s.best_u = hit ? c.u : s.best_u;
+            s.best_tri = hit ? (int)c.tri : s.best_tri;
+            s.best_inst = hit ? s.inst_id : s.best_inst;
+            if (ANY && hit) return true;
+        }
+        s.item += 12;
+        s.kind = (e0 | e1 | e2 | e3) ? kNone : kTri;
+    }
+    if (s.kind == kNone && !resume(s, sp, [&] { return lds_view(stack)[--sp * kQuads]; })) return true;
+    if (s.kind == kInst) inst_step<false>(a, s, sp);
+    if (s.kind == kNode) {
+        int next = kNoNode;
+        const uint32_t n = (uint32_t)s.item;
+        if (n < (uint32_t)a.n_nodes) {
+            const auto* p = gview(reinterpret_cast<const uint4*>(a.nodes)) + 4u * (size_t)n;
+            const uint4 w0 = p[0], w2 = p[2];
+            const uint2 w3 = gview(reinterpret_cast<const uint2*>(a.nodes))[8u * (size_t)n + 6];
+            uint32_t c = gview(reinterpret_cast<const uint32_t*>(a.nodes))[16u * (size_t)n + 4 + j];
+            // byte j of the low and of the high word of an axis, near one first (see node_step4q)
+            const uint32_t lo_hi = (uint32_t)(j | (4 + j) << 8), hi_lo = (uint32_t)((4 + j) | j << 8);
+            const uint32_t bx = __builtin_amdgcn_perm(w2.y, w2.x, s.cs.idx >= 0.0f ? lo_hi : hi_lo);
+            const uint32_t by = __builtin_amdgcn_perm(w2.w, w2.z, s.cs.idy >= 0.0f ? lo_hi : hi_lo);
+            const uint32_t bz = __builtin_amdgcn_perm(w3.y, w3.x, s.cs.idz >= 0.0f ? lo_hi : hi_lo);
+            float d;
+            const bool h = quant_box_hit(s, QuantFrame(w0), bx, 0, bx, 1, by, 0, by, 1, bz, 0, bz, 1, d) && c > n;
+            d = h ? d : __int_as_float(0x7f800000);
+            const uint32_t one = h ? 1u : 0u;
+            uint32_t cnt = one + quad_u<1, 0, 3, 2>(one);
+            cnt += quad_u<2, 3, 0, 1>(cnt);
+            // the sorting network of descend4
+            quad_order<1, 0, 3, 2>(d, c, !(j & 1));
+            quad_order<2, 3, 0, 1>(d, c, j < 2);
+            quad_order<0, 2, 1, 3>(d, c, j < 2);
+            const int top = sp + max((int)cnt - 1, 0);
+            if (top <= 4 * STACK_LDS) {
+                if (j > 0 && (uint32_t)j < cnt) lds_view(stack)[(top - j) * kQuads] = (int)c;
+                sp = top;
+            } else {
+                s.bad = 1;  // not for the trees the launch was checked for
+            }
+            next = cnt ? (int)quad_u<0, 0, 0, 0>(c) : kNoNode;
+        } else {
+            s.bad = 1;
+        }
+        follow(s, next);
+    }
+    return false;
+}
+
 template <bool STATS>
 __device__ __forceinline__ void write_result(const TraceArgs& a, const TraceState& s, int id) {
     gview_w(a.hits)[id] = make_int4(s.best_tri, s.best_inst, __float_as_int(s.best_t), __float_as_int(s.best_u));
@@ -625,12 +761,35 @@ __device__ __forceinline__ void write_result(const TraceArgs& a, const TraceStat
     if (s.bad) atomicAdd(a.err, 1);
 }
 
-// One ray per thread (rays strided over the grid when it is smaller than the ray count).  The 4-wide variants are held to 7 waves per SIMD
+// Traces ray `id` with this thread's quad.
+template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED>
+__device__ __forceinline__ void quad_trace(const TraceArgs& a, int* lds_stack, int id) {
+    const int j = threadIdx.x & 3;
+    TraceState s;
+    state_init(s, gview(a.rays)[2 * (size_t)id], gview(a.rays)[2 * (size_t)id + 1], a.root);
+    int sp = 0;
+    while (!advance_quad<BLOCK, STACK_LDS, ANY, MASKED>(a, s, lds_stack + (threadIdx.x >> 2), sp, j)) {
+    }
+    s.bad |= (int)quad_u<1, 0, 3, 2>((uint32_t)s.bad);
+    s.bad |= (int)quad_u<2, 3, 0, 1>((uint32_t)s.bad);
+    if (j == 0) write_result<false>(a, s, id);
+}
+
+// One ray per thread (rays strided over the grid when it is smaller than the ray count), or four
+// lanes per ray when the launch holds at most a.quad rays (the host then sizes the grid for four
+// threads per ray and has checked the stack).  The 4-wide variants are held to 7 waves per SIMD
 // (72 VGPRs), the BVH2 ones to 8 (64).
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, bool STATS, int TREE>
 __global__ __launch_bounds__(BLOCK, STATS ? 1 : TREE == 0 ? 8 : 7) void k_trace(TraceArgs a) {
     __shared__ int lds_stack[STACK_LDS * BLOCK];
     const int count = launch_count(a);
+    if constexpr (TREE == 2 && !STATS) {
+        if (count <= a.quad) {
+            const int id = (int)(blockIdx.x * BLOCK + threadIdx.x) >> 2;
+            if (id < count) quad_trace<BLOCK, STACK_LDS, ANY, MASKED>(a, lds_stack, id);
+            return;
+        }
+    }
     if ((int)(blockIdx.x * BLOCK) >= count) return;  // sized for the capacity of a device-side count
     LaneStack<BLOCK, STACK_LDS> st;
     stack_init(st, lds_stack, a);
@@ -719,7 +878,9 @@ struct BatchGroups {
 };
 
 // One block of 1024 threads: ray counts of this launch, each queue's first chunk, chunks per group.
-__global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchGroups groups, int* group_chunks) {
+// `also` (or null): another table of the same queues that gets the same numbers.
+__global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchItem* also, BatchGroups groups,
+                                                       int* group_chunks) {
     // thread t owns the queues [b0, b1); items are ordered by group, so a queue's chunk_begin is
     // its exclusive chunk prefix over all queues minus that of its group's first queue
     __shared__ int part[1024];
@@ -733,6 +894,7 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchGr
         int n = items[i].capacity;
         if (items[i].count_dev) n = min(max(*items[i].count_dev, 0), n);
         items[i].a.count = n;
+        if (also) also[i].a.count = n;
         sum += (n + 63) >> 6;
     }
     part[t] = sum;
@@ -756,6 +918,7 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchGr
     for (int i = b0; i < b1; i++) {
         while (g < 3 && groups.first[g + 1] <= i) g++;
         items[i].chunk_begin = run - base[g];
+        if (also) also[i].chunk_begin = run - base[g];
         run += (items[i].a.count + 63) >> 6;
     }
     if (t < 4) {
@@ -765,10 +928,15 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchGr
 }
 
 // The 4-wide variants are held to 7 waves per SIMD (72 VGPRs), the BVH2 ones to 8.
-template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE>
+// QUADS (quantized tree): four lanes per ray, a wave taking a quarter of a chunk at a time.  A
+// kernel of its own: both mappings in one kernel cost the one-lane mapping 7% (48 queues, 1.3M
+// rays: 1,157 us against 1,082).  Where the queue sizes are only known on the device both kernels
+// are launched and `limit` chunks decide which of them works: the one-lane kernel above it, the
+// other up to it (limit < 0: the one-lane kernel always).
+template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE, bool QUADS>
 __global__ __launch_bounds__(BLOCK, TREE == 0 ? 8 : 7) void k_trace_batch(
     const BatchItem* __restrict__ items, int first, int n_items, const int* __restrict__ total_chunks, int* counter,
-    int* spill, int spill_depth) {
+    int* spill, int spill_depth, int limit) {
     __shared__ int lds_stack[STACK_LDS * BLOCK];
     LaneStack<BLOCK, STACK_LDS> st;
     st.lds = lds_stack;
@@ -779,12 +947,15 @@ __global__ __launch_bounds__(BLOCK, TREE == 0 ? 8 : 7) void k_trace_batch(
     st.spill_stride = gridDim.x * BLOCK;
     st.sp = 0;
     const int lane = __lane_id();
-    const int total = __builtin_amdgcn_readfirstlane(*total_chunks);
+    const int chunks = __builtin_amdgcn_readfirstlane(*total_chunks);
+    if (QUADS ? chunks > limit : chunks <= limit) return;  // the same for the whole grid: counters untouched
+    const int total = QUADS ? 4 * chunks : chunks;  // pieces of 16 or 64 rays
     for (;;) {
-        int c = 0;
-        if (lane == 0) c = atomicAdd(&counter[0], 1);
-        c = __builtin_amdgcn_readfirstlane(__shfl(c, 0, 64));
-        if (c >= total) break;
+        int piece = 0;
+        if (lane == 0) piece = atomicAdd(&counter[0], 1);
+        piece = __builtin_amdgcn_readfirstlane(__shfl(piece, 0, 64));
+        if (piece >= total) break;
+        const int c = QUADS ? piece >> 2 : piece;
         // the queue owning chunk c: the last one whose first chunk is <= c (queues without
         // rays share their first chunk with the next queue and are skipped)
         int lo = first, hi = first + n_items - 1;
@@ -795,14 +966,20 @@ __global__ __launch_bounds__(BLOCK, TREE == 0 ? 8 : 7) void k_trace_batch(
         }
         lo = __builtin_amdgcn_readfirstlane(lo);
         const TraceArgs a = items[lo].a;
-        const int id = (c - items[lo].chunk_begin) * 64 + lane;
-        if (id < a.count) {
-            TraceState s;
-            state_init(s, gview(a.rays)[2 * (size_t)id], gview(a.rays)[2 * (size_t)id + 1], a.root);
-            st.sp = 0;
-            while (!advance<BLOCK, STACK_LDS, ANY, MASKED, false, TREE>(a, s, st)) {
+        const int begin = (c - items[lo].chunk_begin) * 64;
+        if constexpr (QUADS) {
+            const int id = begin + (piece & 3) * 16 + (lane >> 2);
+            if (id < a.count) quad_trace<BLOCK, STACK_LDS, ANY, MASKED>(a, lds_stack, id);
+        } else {
+            const int id = begin + lane;
+            if (id < a.count) {
+                TraceState s;
+                state_init(s, gview(a.rays)[2 * (size_t)id], gview(a.rays)[2 * (size_t)id + 1], a.root);
+                st.sp = 0;
+                while (!advance<BLOCK, STACK_LDS, ANY, MASKED, false, TREE>(a, s, st)) {
+                }
+                write_result<false>(a, s, id);
             }
-            write_result<false>(a, s, id);
         }
     }
     if (lane == 0) {

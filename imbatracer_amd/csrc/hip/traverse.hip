@@ -70,6 +70,14 @@ int not_capturing(hipStream_t s, const char* what) {
     return IMBA_OK;
 }
 
+// Most rays a launch over the quantized tree traces with four lanes each: six waves of 16 rays
+// per SIMD (98,304 on 256 CUs).  Around there the chip is full with either mapping and one lane
+// per ray, which does less work in all, overtakes (trace_kernels.h has both sides, between 65,000
+// and 130,000 rays).  A quad's stack is the LDS of its four lanes, without a spill buffer.
+int quad_rays(const DeviceProps* p, int max_stack, int stack_lds) {
+    return max_stack <= 4 * stack_lds ? p->cu_count * 4 * 6 * 16 : 0;
+}
+
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, bool STATS, int TREE>
 int launch_one(const TraceArgs& args_in, int max_stack, int blocks_per_cu, int refill, hipStream_t s) {
     TraceArgs a = args_in;
@@ -90,10 +98,15 @@ int launch_one(const TraceArgs& args_in, int max_stack, int blocks_per_cu, int r
         if (resident <= 0) resident = 1;
         if (blocks_per_cu > 0) resident = std::min(resident, blocks_per_cu);
         grid = std::max(1, std::min(needed, resident * p->cu_count));
-    }  // else one thread per ray, so that the dispatcher starts a new block wherever one finishes (the
-       // rays of a wave end at very different times); a grid capped at the resident blocks, each
-       // thread striding over several rays, left the SIMDs a quarter occupied on average and was
-       // 4% slower on the path-tracing queues
+    } else {
+        // One thread per ray, so that the dispatcher starts a new block wherever one finishes (the
+        // rays of a wave end at very different times); a grid capped at the resident blocks, each
+        // thread striding over several rays, left the SIMDs a quarter occupied on average and was
+        // 4% slower on the path-tracing queues.  A small queue (its size may only be known on the
+        // device) gets four threads per ray.
+        a.quad = TREE == 2 && !STATS ? quad_rays(p, max_stack, STACK_LDS) : 0;
+        grid = std::max(grid, ceil_div(4 * std::min(a.quad, a.count), BLOCK));
+    }
     a.spill = nullptr;
     a.spill_depth = 0;
     if (max_stack > STACK_LDS) {
@@ -130,16 +143,18 @@ int launch_one(const TraceArgs& args_in, int max_stack, int blocks_per_cu, int r
 constexpr int kDefaultBlock = 256;
 constexpr int kDefaultStack = 16;
 
-constexpr int kDefaultWidth = 2;
-
 // Tree a configuration asks for: 0 the BVH2, 1 the 4-wide tree, 2 its quantized form; -1 if
-// the configuration is invalid.
-int tree_code(const ImbaTraceConfig* cfg) {
-    const int w = cfg && cfg->bvh_width ? cfg->bvh_width : kDefaultWidth;
-    if (w == 2) return (cfg && cfg->quantized) ? -1 : 0;
-    if (w == 4) return (cfg && cfg->quantized) ? 2 : 1;
+// the configuration is invalid; `otherwise` when it leaves the choice open.
+int tree_code(const ImbaTraceConfig* cfg, int otherwise) {
+    const int w = cfg ? cfg->bvh_width : 0;
+    if (w == 0) return (cfg && cfg->quantized) ? -1 : otherwise;
+    if (w == 2) return cfg->quantized ? -1 : 0;
+    if (w == 4) return cfg->quantized ? 2 : 1;
     return -1;
 }
+
+// The tree when the configuration leaves it open.
+int default_tree(bool, bool) { return 0; }
 
 // The treelet size of a configuration (accepted for the quantized tree, without effect: every
 // node is read through the caches, which hold the top levels anyway).
@@ -147,7 +162,7 @@ int check_treelet(const ImbaTraceConfig* cfg) {
     if (!cfg || !cfg->treelet) return IMBA_OK;
     if (cfg->treelet < 0 || cfg->treelet > kTreeletMaxNodes)
         return fail(IMBA_ERR_INVALID_ARG, "treelet must be 0..%d nodes", kTreeletMaxNodes);
-    if (tree_code(cfg) != 2) return fail(IMBA_ERR_INVALID_ARG, "treelet needs the quantized 4-wide tree");
+    if (tree_code(cfg, 0) != 2) return fail(IMBA_ERR_INVALID_ARG, "treelet needs the quantized 4-wide tree");
     return IMBA_OK;
 }
 
@@ -239,17 +254,17 @@ int launch_trace(const TreeView& t, int* d_err, const ImbaRay* rays, ImbaHit* hi
 }
 
 // The tree of `s` that `cfg` asks for.
-int pick_tree(const ImbaTraceConfig* cfg, const ImbaSceneDesc* d2, const SceneInfo* i2,
+int pick_tree(const ImbaTraceConfig* cfg, int otherwise, const ImbaSceneDesc* d2, const SceneInfo* i2,
               const ImbaSceneDesc* d4, const ImbaSceneDesc* d4q, const SceneInfo* i4, TreeView* t) {
-    const int code = tree_code(cfg);
+    const int code = tree_code(cfg, otherwise);
     if (code < 0) return fail(IMBA_ERR_INVALID_ARG, "bvh_width must be 0, 2 or 4 (quantized only with 4)");
     if (code == 2 && !d4q->nodes) return fail(IMBA_ERR_INVALID_ARG, "the scene has no quantized 4-wide tree");
     *t = code == 0 ? TreeView{d2, i2, 0} : code == 1 ? TreeView{d4, i4, 1} : TreeView{d4q, i4, 2};
     return IMBA_OK;
 }
 
-int tree_of(const ImbaScene* s, const ImbaTraceConfig* cfg, TreeView* t) {
-    return pick_tree(cfg, &s->dev, &s->info, &s->dev4, &s->dev4q, &s->info4, t);
+int tree_of(const ImbaScene* s, const ImbaTraceConfig* cfg, int otherwise, TreeView* t) {
+    return pick_tree(cfg, otherwise, &s->dev, &s->info, &s->dev4, &s->dev4q, &s->info4, t);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -360,6 +375,7 @@ struct ImbaTraceBatch {
     imba::BatchGroups groups{};
     int max_stack[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};  // per tree width (2, 4) and group
     long long capacity_chunks[4] = {0, 0, 0, 0};
+    bool device_counts[4] = {false, false, false, false};  // a queue's size is read on the device
     imba::BatchItem* d_items[3] = {nullptr, nullptr, nullptr};  // queue tables per tree (BVH2, 4-wide, quantized)
     bool quantized_ok = true;                              // every queue's scene has the quantized tree
     int cap = 0;                                           // queues the tables hold room for
@@ -377,21 +393,25 @@ struct ImbaTraceBatch {
 namespace imba {
 namespace {
 
-template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE>
-int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, hipStream_t s) {
+// One launch of group g: chunks of 64 rays with one lane each, or (QUADS) quarters of chunks with
+// four lanes per ray; `limit` as in k_trace_batch.  With `reserve` only the spill stack the launch
+// would need is allocated (for a later launch that is recorded into a graph).
+template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE, bool QUADS>
+int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, bool reserve, hipStream_t s) {
     const DeviceProps* p = device_props();
-    if (!p) return fail(IMBA_ERR_NO_DEVICE, "no HIP device");
-    auto kern = k_trace_batch<BLOCK, STACK_LDS, ANY, MASKED, TREE>;
+    auto kern = k_trace_batch<BLOCK, STACK_LDS, ANY, MASKED, TREE, QUADS>;
     const int max_stack = b->max_stack[TREE ? 1 : 0][g];
     int resident = 0;
     IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, BLOCK, 0));
     if (resident <= 0) resident = 1;
     if (blocks_per_cu > 0) resident = std::min(resident, blocks_per_cu);
-    const long long needed = (b->capacity_chunks[g] * 64 + BLOCK - 1) / BLOCK;
+    const long long chunks = b->capacity_chunks[g];
+    const long long pieces = QUADS ? 4 * std::min<long long>(chunks, limit) : chunks;  // 64 threads each
+    const long long needed = (pieces * 64 + BLOCK - 1) / BLOCK;
     const int grid = (int)std::max<long long>(1, std::min<long long>(needed, (long long)resident * p->cu_count));
     int* spill = nullptr;
     int spill_depth = 0;
-    if (max_stack > STACK_LDS) {
+    if (!QUADS && max_stack > STACK_LDS) {
         spill_depth = max_stack - STACK_LDS;
         const size_t need = (size_t)spill_depth * grid * BLOCK * sizeof(int);
         if (b->spill[g].bytes < need) {
@@ -402,20 +422,40 @@ int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, hipStream_t 
         }
         spill = (int*)b->spill[g].ptr;
     }
+    if (reserve) return IMBA_OK;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), 0, s, b->d_items[TREE], b->groups.first[g],
                        b->groups.first[g + 1] - b->groups.first[g], b->d_group_chunks + g, b->d_counters + 2 * g,
-                       spill, spill_depth);
+                       spill, spill_depth, limit);
     IMBA_HIP_TRY(hipGetLastError());
     return IMBA_OK;
 }
 
+template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE>
+int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, bool reserve, hipStream_t s) {
+    const DeviceProps* p = device_props();
+    if (!p) return fail(IMBA_ERR_NO_DEVICE, "no HIP device");
+    if constexpr (TREE == 2) {
+        const int limit = blocks_per_cu <= 0 ? quad_rays(p, b->max_stack[1][g], STACK_LDS) / 64 : 0;
+        if (limit > 0 && !reserve) {
+            // a graph replays its launches with whatever sizes a later update brings
+            const bool small = b->capacity_chunks[g] <= limit && !b->captured;
+            if (small || b->device_counts[g] || b->captured) {
+                const int r = launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, true>(b, g, 0, limit, false, s);
+                if (r) return r;
+                return launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, 0, limit, small, s);
+            }
+        }
+    }
+    return launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, blocks_per_cu, -1, reserve, s);
+}
+
 template <bool ANY, bool MASKED, int TREE>
-int dispatch_batch(ImbaTraceBatch* b, int g, const ImbaTraceConfig* cfg, hipStream_t s) {
+int dispatch_batch(ImbaTraceBatch* b, int g, const ImbaTraceConfig* cfg, hipStream_t s, bool reserve = false) {
     const int block = cfg && cfg->block_size ? cfg->block_size : kDefaultBlock;
     const int stack = cfg && cfg->stack_lds ? cfg->stack_lds : kDefaultStack;
     const int bpc = cfg ? cfg->blocks_per_cu : 0;
 #define IMBA_SHAPE(B, S) \
-    if (block == B && stack == S) return launch_batch_group<B, S, ANY, MASKED, TREE>(b, g, bpc, s);
+    if (block == B && stack == S) return launch_batch_group<B, S, ANY, MASKED, TREE>(b, g, bpc, reserve, s);
     IMBA_SHAPE(256, 16)
     IMBA_SHAPE(256, 8)
     IMBA_SHAPE(256, 32)
@@ -453,6 +493,7 @@ int set_tables(ImbaTraceBatch* b, const ImbaTraceItem* items, int n_items, hipSt
     BatchGroups groups{};
     int max_stack[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
     long long chunks[4] = {0, 0, 0, 0};
+    bool device_counts[4] = {false, false, false, false};
     for (int g = 0; g < 4; g++) {
         groups.first[g] = (int)table.size();
         for (int i = 0; i < n_items; i++) {
@@ -475,6 +516,7 @@ int set_tables(ImbaTraceBatch* b, const ImbaTraceItem* items, int n_items, hipSt
             max_stack[0][g] = std::max(max_stack[0][g], it.scene->info.max_stack);
             max_stack[1][g] = std::max(max_stack[1][g], it.scene->info4.max_stack);
             chunks[g] += ceil_div(it.count, 64);
+            device_counts[g] |= it.count_dev != nullptr;
             table.push_back(e);
             const TraceArgs a4 = scene_args(it.scene->dev4, it.scene->d_error);
             e.a.nodes = a4.nodes;
@@ -544,6 +586,7 @@ int set_tables(ImbaTraceBatch* b, const ImbaTraceItem* items, int n_items, hipSt
     b->quantized_ok = quantized_ok;
     std::memcpy(b->max_stack, max_stack, sizeof(max_stack));
     std::memcpy(b->capacity_chunks, chunks, sizeof(chunks));
+    std::memcpy(b->device_counts, device_counts, sizeof(device_counts));
     return IMBA_OK;
 }
 
@@ -599,22 +642,34 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
     IMBA_HIP_TRY(hipGetDevice(&dev));
     if (dev != b->device) return fail(IMBA_ERR_INVALID_ARG, "batch belongs to device %d, current is %d", b->device, dev);
     if (b->n == 0) return IMBA_OK;
-    const int tree = tree_code(cfg);
-    if (tree < 0) return fail(IMBA_ERR_INVALID_ARG, "bvh_width must be 0, 2 or 4 (quantized only with 4)");
-    if (tree == 2 && !b->quantized_ok) return fail(IMBA_ERR_INVALID_ARG, "a queue's scene has no quantized tree");
-    int r = check_treelet(cfg);
-    if (r) return r;
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
-    if (is_capturing(s)) {
+    const bool capturing = is_capturing(s);
+    // Closest-hit and any-hit queues may take different trees.  A launch recorded into a graph
+    // must do for every queue a later update brings, so there the open choice is the BVH2.
+    const int closest = tree_code(cfg, default_tree(false, b->quantized_ok && !capturing));
+    const int any = tree_code(cfg, default_tree(true, false));
+    if (closest < 0) return fail(IMBA_ERR_INVALID_ARG, "bvh_width must be 0, 2 or 4 (quantized only with 4)");
+    if (closest == 2 && !b->quantized_ok) return fail(IMBA_ERR_INVALID_ARG, "a queue's scene has no quantized tree");
+    int r = check_treelet(cfg);
+    if (r) return r;
+    if (capturing) {
         b->captured = true;
         b->captured_groups = b->groups;
     }
-    hipLaunchKernelGGL(k_batch_prefix, dim3(1), dim3(1024), 0, s, b->d_items[tree], b->groups, b->d_group_chunks);
+    hipLaunchKernelGGL(k_batch_prefix, dim3(1), dim3(1024), 0, s, b->d_items[closest],
+                       any == closest ? (BatchItem*)nullptr : b->d_items[any], b->groups, b->d_group_chunks);
     IMBA_HIP_TRY(hipGetLastError());
+    // the tree an open choice takes in a graph
+    const bool other = closest == 2 && tree_code(cfg, 0) == 0;
     for (int g = 0; g < 4; g++) {
         if (b->groups.first[g + 1] == b->groups.first[g] || b->capacity_chunks[g] == 0) continue;
-        switch (g + 4 * tree) {
+        if (other && g < 2) {
+            r = g == 0 ? dispatch_batch<false, false, 0>(b, g, cfg, s, true)
+                       : dispatch_batch<false, true, 0>(b, g, cfg, s, true);
+            if (r) return r;
+        }
+        switch (g + 4 * (g >= 2 ? any : closest)) {
             case 0: r = dispatch_batch<false, false, 0>(b, g, cfg, s); break;
             case 1: r = dispatch_batch<false, true, 0>(b, g, cfg, s); break;
             case 2: r = dispatch_batch<true, false, 0>(b, g, cfg, s); break;
@@ -655,7 +710,7 @@ int imba_autotune(const ImbaScene* sc, const ImbaRay* rays, ImbaHit* hits, int c
             ImbaTraceConfig cfg{shape[0], shape[1], refill, 0, tree[0], tree[1], 0};
             if (tree[1] && !sc->dev4q.nodes) continue;
             TreeView t{};
-            r = tree_of(sc, &cfg, &t);
+            r = tree_of(sc, &cfg, 0, &t);
             if (!r)
                 r = launch_trace(t, sc->d_error, rays, hits, nullptr, count, any_hit != 0, !sc->info.all_opaque, &cfg,
                                  s);
@@ -699,7 +754,8 @@ static int trace_entry(const ImbaScene* s, const ImbaRay* rays, ImbaHit* hits, u
                        uint32_t* depth_hist = nullptr) {
     IMBA_CHECK_ARG(s, "scene is NULL");
     TreeView t{};
-    int r = tree_of(s, cfg, &t);
+    const bool stats = counts || depth_hist;
+    int r = tree_of(s, cfg, stats ? 0 : default_tree(any, s->dev4q.nodes != nullptr), &t);
     if (r) return r;
     return launch_trace(t, s->d_error, rays, hits, counts, count, any, !s->info.all_opaque, cfg, stream, count_dev,
                         depth_hist);

@@ -1,0 +1,118 @@
+"""Small queues over the quantized tree are traced with four lanes per ray: hits equal the
+one-lane-per-ray launch's bit for bit (closest and any hit) and the oracle's closest hits, at the
+edges of quads, waves and the largest queue that takes this path, over leaves longer than a quad,
+instances and masks, for device-side counts and batches; closest hits of the default launch
+equal the BVH2's.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from imbatracer_amd import native as N
+from imbatracer_amd import scene as S
+from tests import scenes as T
+
+pytestmark = pytest.mark.gpu
+
+Q4 = N.TraceConfig(256, 16, 0, 0, 4, 1, 0)
+ONE_LANE = N.TraceConfig(256, 16, 0, 64, 4, 1, 0)  # an explicit grid: one lane per ray at any size
+BVH2 = N.TraceConfig(256, 16, 0, 0, 2, 0, 0)
+LARGEST = 98304  # on 256 CUs
+
+
+def _same(a, b):
+    return np.array_equal(np.ascontiguousarray(a).view(np.int32), np.ascontiguousarray(b).view(np.int32))
+
+
+def _stacked():
+    """Leaves of up to 13 coincident triangles (equal distances: the smallest id wins)."""
+    v, i = S.random_triangles(300, 31)
+    tri = v.reshape(-1, 3, 4)
+    rng = np.random.default_rng(7)
+    tri = np.concatenate([np.repeat(tri[k:k + 1], rng.integers(1, 14), 0) for k in range(len(tri))])
+    b = S.SceneBuild()
+    b.add_mesh(tri.reshape(-1, 4), np.arange(3 * len(tri), dtype=np.uint32).reshape(-1, 3))
+    b.run(N.BUILDER_BINNED_SAH, 1)
+    return b
+
+
+SCENES = {"random": lambda: T.random_tri_scene(20000, N.BUILDER_SBVH)[0], "instanced": T.instanced_scene,
+          "masked": T.masked_scene, "stacked": _stacked}
+
+
+@pytest.mark.parametrize("name", sorted(SCENES))
+def test_sizes(gpu, name):
+    b = SCENES[name]()
+    sc = S.Scene(b.desc())
+    box = (-2.0, 2.0) if name == "instanced" else (-0.2, 1.2)
+    rays = T.random_rays(LARGEST + 1, seed=8, box=box)
+    want, _ = oracle.trace(b.arrays(), rays, threads=8)
+    want_any = sc.trace_host(rays, any_hit=True, cfg=ONE_LANE)
+    assert (want["tri_id"] >= 0).sum() > 100
+    for n in (1, 3, 15, 16, 17, 63, 64, 65, 1000, LARGEST, LARGEST + 1):
+        assert _same(sc.trace_host(rays[:n], cfg=Q4), want[:n]), n
+        assert _same(sc.trace_host(rays[:n]), want[:n]), n
+        assert _same(sc.trace_host(rays[:n], any_hit=True, cfg=Q4), want_any[:n]), n
+    assert _same(sc.trace_host(rays, cfg=BVH2), want)
+    assert sc.error_count() == 0
+
+
+def test_device_counts_and_batches(gpu):
+    b = T.instanced_scene()
+    sc = S.Scene(b.desc())
+    rays = T.random_rays(200000, seed=9, box=(-2.0, 2.0))
+    want, _ = oracle.trace(b.arrays(), rays, threads=8)
+    want_any = sc.trace_host(rays, any_hit=True, cfg=BVH2)
+    rb = N.DeviceBuffer.from_array(rays)
+    hb, ha = N.DeviceBuffer(16 * len(rays)), N.DeviceBuffer(16 * len(rays))
+    untouched = np.full(4 * len(rays), 7, np.int32)
+    for n in (0, 1, 61, 5000, LARGEST, LARGEST + 5, len(rays)):
+        cnt = N.DeviceBuffer.from_array(np.array([n], np.int32))
+        hb.upload(untouched)
+        N.check(N.lib.imba_intersect_dev(sc.h, rb.ptr, hb.ptr, len(rays), cnt.ptr, None, None), "intersect_dev")
+        got = hb.download(N.HIT_DTYPE, len(rays))
+        assert _same(got[:n], want[:n]) and (np.ascontiguousarray(got[n:]).view(np.int32) == 7).all(), n
+        # two closest queues and an any-hit queue of the same rays, default trees per kind
+        k = n // 3
+        batch = S.TraceBatch([(sc, rb, hb, k, None, False), (sc, rb.at(32 * k), hb.at(16 * k), len(rays) - k, cnt, False),
+                              (sc, rb, ha, n, None, True)])
+        left = min(n, len(rays) - k)
+        for cfg in (None, Q4):
+            hb.upload(untouched)
+            batch.launch(cfg)
+            got = hb.download(N.HIT_DTYPE, len(rays))
+            assert _same(got[:k + left], want[:k + left]), (n, cfg)
+            got_any = ha.download(N.HIT_DTYPE, len(rays))[:n]
+            if cfg is None:
+                assert _same(got_any, want_any[:n]), n
+            else:
+                assert np.array_equal(got_any["tri_id"] >= 0, want_any[:n]["tri_id"] >= 0), n
+    assert sc.error_count() == 0
+
+
+def test_recorded_batch(gpu):
+    """A batch recorded into a graph after one plain launch, with the open choice of tree and with
+    the quantized one: replays follow the queue sizes of later updates on both sides of the
+    largest small queue.  The scene's stack is deeper than the LDS part."""
+    b = T.random_tri_scene(200000, N.BUILDER_BINNED_SAH)[0]
+    sc = S.Scene(b.desc())
+    rays = T.random_rays(LARGEST + 3000, seed=10)
+    want = sc.trace_host(rays, cfg=BVH2)
+    rb, hb = N.DeviceBuffer.from_array(rays), N.DeviceBuffer(16 * len(rays))
+    for cfg in (None, Q4):
+        st = N.Stream()
+        batch = S.TraceBatch([(sc, rb, hb, 500, None, False)])
+        batch.launch(cfg, st)
+        st.sync()
+        S.Graph.begin(st)
+        try:
+            batch.launch(cfg, st)
+        finally:
+            g = S.Graph.end(st)
+        for n in (500, len(rays), 77, LARGEST):
+            batch.update([(sc, rb, hb, n, None, False)], st)
+            hb.upload(np.full(4 * len(rays), 7, np.int32), st)
+            g.launch(st)
+            st.sync()
+            got = hb.download(N.HIT_DTYPE, len(rays))
+            assert _same(got[:n], want[:n]) and (np.ascontiguousarray(got[n:]).view(np.int32) == 7).all(), (n, cfg)
