@@ -286,7 +286,10 @@ typedef struct ImbaTraceConfig {
                               rays (0 = default: persistent launches fill the resident
                               blocks, others launch one thread per ray)                 */
     int bvh_width;         /* 2: the scene's BVH2 as given; 4: the 4-wide tree derived from
-                              it at upload (same leaves); 0 = default                      */
+                              it at upload (same leaves); 0 = default: any hits, visit counts,
+                              stack depths and batches recorded into a graph take the BVH2,
+                              closest hits (which do not depend on the tree) the quantized
+                              4-wide tree where the scene has one                          */
     int quantized;         /* with bvh_width 4: 64-byte nodes whose child boxes are 8-bit
                               offsets from the node box, rounded outward                  */
     int treelet;           /* quantized tree only, 0..256: accepted, without effect (every node
