@@ -1,4 +1,4 @@
-// Photon hash grid: parameters, device-side state and the one-query-per-wave scan shared by
+// Photon hash grid: parameters, device-side state and the wave's query scan shared by
 // the index query (hashgrid.hip, HashGrid::query of rangesearch/rangesearch.h:79-129) and the
 // fused vertex-merging launch (vcm.hip).
 #pragma once
@@ -77,96 +77,163 @@ __device__ __forceinline__ float box_dist2(const uint32_t* box, int b, float qx,
     return gx * gx + gy * gy + gz * gz;
 }
 
-// One query per wave.  The eight probed buckets are visited in the reference's order, each
-// bucket's photons scanned 64 at a time (lane l takes photon base + l, so loads are contiguous
-// across the wave).  Candidates within the limit at the start of the chunk (the radius, or the
-// current k-th distance once the list is full) are then inserted one at a time in visiting
-// order with the reference's rule; the list itself lives in lanes 0..k-1 (squared distance and
-// id per lane), so any k up to 64 fits.  The limit only shrinks, so the candidates it rejects
-// would be rejected by the exact test as well: the results are those of the one-at-a-time
-// scan.  For the same reason a bucket whose photon box lies beyond the limit when its turn
-// comes is skipped whole (none of its photons would pass).  The id is the photon index, or with
-// SLOTS the photon's slot in the grid order (pos4[slot]).  Returns the list length
-// (wave-uniform); lanes >= count hold (0, -1).  Every lane of the wave must call it.
-template <bool SLOTS>
-__device__ __forceinline__ int query_wave_list(const GridParams& g, const int* ends, const float4* pos4,
-                                               const uint32_t* box, float qx, float qy, float qz, int k,
-                                               float& my_dist, int& my_id) {
-    const int lane = (int)(threadIdx.x & 63);
-    my_dist = 0.0f;
-    my_id = -1;
-    int count = 0;
+// The value lane `lane` holds (wave-uniform).
+__device__ __forceinline__ float lane_value(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+
+// The probes of a query: lane 8 q + j holds probe j's bucket range and the squared distance to its
+// photons' box for the q-th of the wave's queries.
+struct GridProbes {
+    int begin, size;
+    float lb;
+};
+
+// (qx, qy, qz): the position of the lane's query; `active`: it has one.  A query outside the grid
+// has eight empty ranges.  All loads of a lane are independent of each other, and those of eight
+// queries are in flight together.
+__device__ __forceinline__ GridProbes grid_probes(const GridParams& g, const int* ends, const uint32_t* box, float qx,
+                                                  float qy, float qz, bool active) {
+    GridProbes r{0, 0, 0.0f};
     const bool inside = qx >= g.bmin[0] && qy >= g.bmin[1] && qz >= g.bmin[2] &&
                         qx <= g.bmax[0] && qy <= g.bmax[1] && qz <= g.bmax[2];
-    if (!(inside && g.count > 0)) return 0;
+    if (!(active && inside && g.count > 0)) return r;
+    const int probe = (int)(threadIdx.x & 7);
     const float cx = g.inv_cell_size * (qx - g.bmin[0]);
     const float cy = g.inv_cell_size * (qy - g.bmin[1]);
     const float cz = g.inv_cell_size * (qz - g.bmin[2]);
     const float fx = floorf(cx), fy = floorf(cy), fz = floorf(cz);
-    const int px = (int)fx, py = (int)fy, pz = (int)fz;
-    const int pxo = px + ((cx - fx) < 0.5f ? -1 : 1);
-    const int pyo = py + ((cy - fy) < 0.5f ? -1 : 1);
-    const int pzo = pz + ((cz - fz) < 0.5f ? -1 : 1);
-    // lane j < 8: probe j's bucket range and the squared distance to its photons' box
-    int begin = 0, size = 0;
-    float lb = 0.0f;
-    if (lane < 8) {
-        const int x = (lane & 4) ? pxo : px;
-        const int y = (lane & 2) ? pyo : py;
-        const int z = (lane & 1) ? pzo : pz;
-        const int b = bucket_of((uint32_t)x, (uint32_t)y, (uint32_t)z, g.table_size);
-        begin = b == 0 ? 0 : ends[b - 1];
-        size = ends[b] - begin;
-        lb = box && size > 0 ? box_dist2(box, b, qx, qy, qz) : 0.0f;
-    }
-    float kth = 0.0f;  // dist[k - 1] once the list is full (wave-uniform)
+    const int x = (int)fx + ((probe & 4) ? ((cx - fx) < 0.5f ? -1 : 1) : 0);
+    const int y = (int)fy + ((probe & 2) ? ((cy - fy) < 0.5f ? -1 : 1) : 0);
+    const int z = (int)fz + ((probe & 1) ? ((cz - fz) < 0.5f ? -1 : 1) : 0);
+    const int b = bucket_of((uint32_t)x, (uint32_t)y, (uint32_t)z, g.table_size);
+    r.lb = box_dist2(box, b, qx, qy, qz);  // (an empty bucket's entry holds anything: not used)
+    r.begin = ends[b > 0 ? b - 1 : 0];
+    r.begin = b > 0 ? r.begin : 0;
+    r.size = ends[b] - r.begin;
+    return r;
+}
+
+// Queries per wave: they share the wave's probing (the hash, the table reads and their latency),
+// as long as every SIMD still gets its waves.  600,000 queries, k = 10 / 200,000 queries, k = 64, with
+// 1, 2, 4, 8 per wave: 838, 801, 798, 880 us / 632, 636, 679, 850 us.
+constexpr int kQueriesPerWave = 2;
+inline int queries_per_wave(int nq, int cu_count) {
+    int per = kQueriesPerWave;
+    while (per > 1 && nq < per * cu_count * 4 * 8) per >>= 1;
+    return per;
+}
+
+// One query by a whole wave, its probes in lanes `first`..`first` + 7.  The eight probed buckets are
+// visited in the reference's order, each bucket's photons scanned in groups of four chunks of 64
+// (lane l takes photon base + l of a chunk, so loads are contiguous across the wave and a group's
+// are in flight together).
+// Candidates within the limit are then inserted one at a time in visiting order with the
+// reference's rule; the list itself lives in lanes 0..k-1 (squared distance and id per lane), so
+// any k up to 64 fits.  The limit is the radius, or the current k-th distance once the list is
+// full, or, where a group holds many candidates, a bound that at least k of the list's entries
+// and the group's per-lane minima do not exceed, found by halving.  A candidate beyond any of them
+// is beyond the final k-th distance: such a candidate never stays in the list and never
+// moves one that does (an insertion only looks at the entries up to it), so the results are those
+// of the one-at-a-time scan, equal distances included.  For the same reason a bucket whose photon
+// box lies beyond the limit when its turn comes is skipped whole.  The id is the photon index, or
+// with SLOTS the photon's slot in the grid order (pos4[slot]).  Returns the list length
+// (wave-uniform); lanes >= count hold (0, -1).  Every lane of the wave must call it.
+//
+// Bound by instruction issue: 720 vector and 540 scalar instructions per query at k = 10 over
+// 1,000 probed photons, 70% of the kernel's time.  Before the bound (which leaves 11-15 insertions
+// of 45), 600,000 queries over 2M photons took 1,557 us, now 785; 200,000 with k = 64 860, now 636;
+// with k = 1 265, now 137.  Groups of 2 or 8 chunks and testing a bucket's end per chunk were slower.
+template <bool SLOTS>
+__device__ __forceinline__ int query_wave_list(const GridParams& g, const float4* pos4, const GridProbes& probes,
+                                               int first, float qx, float qy, float qz, int k, float& my_dist,
+                                               int& my_id) {
+    constexpr int kGroup = 4;    // chunks of 64 photons in flight
+    constexpr int kMany = 10;    // candidates of a group above which the bound is worth finding
+    constexpr int kHalvings = 7;
+    constexpr uint32_t kOctaves = 6;  // the bound is sought down to limit / 64
+    const float inf = __int_as_float(0x7f800000);
+    const int lane = (int)(threadIdx.x & 63);
+    my_id = -1;
+    int count = 0;
+    // Distances are compared as their bits where they are wave-uniform (squares' sums are never
+    // negative, so the order is the same), which keeps that work on the scalar unit.
+    const uint32_t radius_bits = __float_as_uint(g.radius_sqr);
+    uint32_t kth = 0x7f800000u;  // dist[k - 1], infinity until the list is full
+    my_dist = inf;               // lanes past the list's end
     for (int j = 0; j < 8; j++) {
-        const int beg = __builtin_amdgcn_readlane(begin, j);
-        const int n = __builtin_amdgcn_readlane(size, j);
-        const float lbj = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lb), j));
-        if (n == 0 || lbj > (count == k ? kth : g.radius_sqr)) continue;
-        // photon c of this bucket (x = +inf past its end, which no test accepts); the next
-        // chunk's load is issued before the current chunk's insertions
-        auto fetch = [&](int c) {
-            if (c >= n) return make_float4(__int_as_float(0x7f800000), 0.0f, 0.0f, 0.0f);
-            return pos4[beg + c];
-        };
-        float4 p_next = fetch(lane);
-        for (int base = 0; base < n; base += 64) {
-            const bool valid = base + lane < n;
-            const float4 p = p_next;
-            if (base + 64 < n) p_next = fetch(base + 64 + lane);
-            float d2 = 0.0f;
-            int pid = -1;
-            if (valid) {
-                const float dx = qx - p.x, dy = qy - p.y, dz = qz - p.z;
-                d2 = dx * dx + dy * dy + dz * dz;
-                pid = SLOTS ? beg + base + lane : __float_as_int(p.w);
+        const int beg = __builtin_amdgcn_readlane(probes.begin, first + j);
+        const int n = __builtin_amdgcn_readlane(probes.size, first + j);
+        const float lbj = lane_value(probes.lb, first + j);
+        if (n == 0 || __float_as_uint(lbj) > min(kth, radius_bits)) continue;
+        for (int base = 0; base < n; base += 64 * kGroup) {
+            float4 p[kGroup];
+#pragma unroll
+            for (int i = 0; i < kGroup; i++) {
+                // past the bucket's end: x = +inf, which no limit admits
+                p[i] = make_float4(inf, 0.0f, 0.0f, 0.0f);
+                if (base + 64 * i < n && base + 64 * i + lane < n) p[i] = pos4[beg + base + 64 * i + lane];
             }
-            const float lim = count == k ? kth : g.radius_sqr;
-            unsigned long long m = __ballot(valid && d2 <= lim && d2 <= g.radius_sqr);
-            while (m) {
-                const int src = __builtin_ctzll(m);
-                m &= m - 1;
-                const float dd = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(d2), src));
-                const int id = __builtin_amdgcn_readlane(pid, src);
-                if (count == k) {
-                    if (kth < dd) continue;
-                } else {
-                    count++;
+            float d2[kGroup];
+            unsigned long long m[kGroup];
+            uint32_t lim = min(kth, radius_bits);
+            int candidates = 0;
+#pragma unroll
+            for (int i = 0; i < kGroup; i++) {
+                const float dx = qx - p[i].x, dy = qy - p[i].y, dz = qz - p[i].z;
+                d2[i] = dx * dx + dy * dy + dz * dz;
+                m[i] = __ballot(d2[i] <= __uint_as_float(lim));
+                candidates += __popcll(m[i]);
+            }
+            if (candidates > kMany) {
+                float least = d2[0];
+#pragma unroll
+                for (int i = 1; i < kGroup; i++) least = fminf(least, d2[i]);
+                const float listed = lane < k ? my_dist : inf;
+                if (__popcll(__ballot(least <= __uint_as_float(lim))) + count >= k) {
+                    // lim: always a distance that at least k values do not exceed
+                    uint32_t lo = max(lim, kOctaves << 23) - (kOctaves << 23);
+                    for (int h = 0; h < kHalvings; h++) {
+                        const uint32_t mid = (lo + lim) >> 1;
+                        const float f = __uint_as_float(mid);
+                        const bool enough = __popcll(__ballot(least <= f)) + __popcll(__ballot(listed <= f)) >= k;
+                        lo = enough ? lo : mid;
+                        lim = enough ? mid : lim;
+                    }
+#pragma unroll
+                    for (int i = 0; i < kGroup; i++) m[i] = __ballot(d2[i] <= __uint_as_float(lim));
                 }
-                // keep the first count-1 entries, insert dd after every entry <= dd
-                const int keep = count - 1;
-                const int pos = __popcll(__ballot(lane < keep && my_dist <= dd));
-                // the entries one lane down (wave shift right by one lane, DPP)
-                const float up_d = __int_as_float(__builtin_amdgcn_update_dpp(
-                    __float_as_int(my_dist), __float_as_int(my_dist), kDppWaveShr1, 0xF, 0xF, false));
-                const int up_i = __builtin_amdgcn_update_dpp(my_id, my_id, kDppWaveShr1, 0xF, 0xF, false);
-                if (lane > pos && lane <= keep) { my_dist = up_d; my_id = up_i; }
-                if (lane == pos) { my_dist = dd; my_id = id; }
-                if (count == k) kth = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_dist), k - 1));
+            }
+#pragma unroll
+            for (int i = 0; i < kGroup; i++) {
+                while (m[i]) {
+                    const int src = __builtin_ctzll(m[i]);
+                    m[i] &= m[i] - 1;
+                    const uint32_t dd = (uint32_t)__builtin_amdgcn_readlane(__float_as_int(d2[i]), src);
+                    const int id = SLOTS ? beg + base + 64 * i + src
+                                         : __builtin_amdgcn_readlane(__float_as_int(p[i].w), src);
+                    if (kth < dd) continue;
+                    // dd goes after every entry <= dd, but into the last place at the latest (the
+                    // reference drops the last entry of a full list first); lanes from k on hold
+                    // what was dropped, nothing nearer than the k-th
+                    const int pos = min((int)__popcll(__ballot(my_dist <= __uint_as_float(dd))), k - 1);
+                    int my_bits = __float_as_int(my_dist);
+                    if (lane >= pos) {  // the entries one lane down (wave shift right by one lane, DPP)
+                        my_bits = __builtin_amdgcn_update_dpp(my_bits, my_bits, kDppWaveShr1, 0xF, 0xF, false);
+                        my_id = __builtin_amdgcn_update_dpp(my_id, my_id, kDppWaveShr1, 0xF, 0xF, false);
+                    }
+                    my_bits = lane == pos ? (int)dd : my_bits;
+                    my_id = lane == pos ? id : my_id;
+                    my_dist = __int_as_float(my_bits);
+                    count = min(count + 1, k);
+                    kth = (uint32_t)__builtin_amdgcn_readlane(my_bits, k - 1);
+                }
             }
         }
+    }
+    if (lane >= count) {
+        my_dist = 0.0f;
+        my_id = -1;
     }
     return count;
 }

@@ -257,24 +257,31 @@ __global__ __launch_bounds__(kBlock) void k_bucket_box(const int* keys_sorted, i
     }
 }
 
-// One query per wave (the scan and insertion of query_wave_list); the list goes to out_idx /
-// out_dist.
+// `per` queries per wave (query_wave_list); the lists go to out_idx / out_dist.
 __global__ __launch_bounds__(kBlock) void k_query_wave(const GridParams* gp, const int* ends, const float4* pos4,
                                                        const uint32_t* box, const unsigned char* qs, int qstride,
-                                                       int qoff, int nq, int k, int* out_idx, float* out_dist,
+                                                       int qoff, int nq, int per, int k, int* out_idx, float* out_dist,
                                                        int* out_count) {
-    const int q = blockIdx.x * (kBlock / 64) + (int)(threadIdx.x >> 6);
-    if (q >= nq) return;  // whole waves leave together
     const int lane = (int)(threadIdx.x & 63);
-    const float* qp = photon_pos(qs, qstride, qoff, q);
-    float my_dist;
-    int my_idx;
-    const int count = query_wave_list<false>(*gp, ends, pos4, box, qp[0], qp[1], qp[2], k, my_dist, my_idx);
-    if (lane < count) {
-        out_idx[(size_t)q * k + lane] = my_idx;
-        if (out_dist) out_dist[(size_t)q * k + lane] = my_dist;
+    const int q0 = (blockIdx.x * (kBlock / 64) + (int)(threadIdx.x >> 6)) * per;
+    const int n = min(per, nq - q0);
+    if (n <= 0) return;  // whole waves leave together
+    const GridParams g = *gp;
+    const float* qp = photon_pos(qs, qstride, qoff, q0 + min(lane >> 3, n - 1));
+    const float x = qp[0], y = qp[1], z = qp[2];
+    const GridProbes probes = grid_probes(g, ends, box, x, y, z, (lane >> 3) < n);
+    for (int i = 0; i < n; i++) {
+        float my_dist;
+        int my_idx;
+        const int count = query_wave_list<false>(g, pos4, probes, 8 * i, lane_value(x, 8 * i), lane_value(y, 8 * i),
+                                                 lane_value(z, 8 * i), k, my_dist, my_idx);
+        const size_t q = (size_t)(q0 + i);
+        if (lane < count) {
+            out_idx[q * k + lane] = my_idx;
+            if (out_dist) out_dist[q * k + lane] = my_dist;
+        }
+        if (lane == 0) out_count[q] = count;
     }
-    if (lane == 0) out_count[q] = count;
 }
 
 // k > 64: the same scan and insertion rule with the k-capped list in LDS, one query per wave
@@ -532,11 +539,14 @@ int imba_hashgrid_query(const ImbaHashGrid* g, const void* queries, int query_st
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
     const unsigned char* qs = (const unsigned char*)queries;
-    if (k <= 64)
-        hipLaunchKernelGGL(k_query_wave, dim3(ceil_div(nq, kBlock / 64)), dim3(kBlock), 0, s, g->d_params,
-                           g->cell_ends, g->pos4, g->bucket_box, qs, query_stride, query_offset, nq, k, out_idx,
-                           out_dist, out_count);
-    else
+    if (k <= 64) {
+        const DeviceProps* p = device_props();
+        if (!p) return fail(IMBA_ERR_NO_DEVICE, "no HIP device");
+        const int per = queries_per_wave(nq, p->cu_count);
+        hipLaunchKernelGGL(k_query_wave, dim3(ceil_div(ceil_div(nq, per), kBlock / 64)), dim3(kBlock), 0, s,
+                           g->d_params, g->cell_ends, g->pos4, g->bucket_box, qs, query_stride, query_offset, nq, per,
+                           k, out_idx, out_dist, out_count);
+    } else
         hipLaunchKernelGGL(k_query_lds, dim3(nq), dim3(64), (size_t)k * 8, s, g->d_params, g->cell_ends, g->pos4, qs,
                            query_stride, query_offset, nq, k, out_idx, out_dist, out_count);
     IMBA_HIP_TRY(hipGetLastError());

@@ -328,21 +328,11 @@ struct GridMergeArgs {
     float* image;
 };
 
-// The grid query and k_merge's sum in one launch, one query per wave: the wave's k-capped list
-// keeps each photon's grid slot, lane j weighs list entry j, and the wave adds the lanes'
-// terms in list order (k_merge's loop order).
-__global__ __launch_bounds__(256) void k_merge_grid(GridMergeArgs a) {
-    const int q = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-    if (q >= a.nq) return;  // whole waves leave together
-    const float4 q0 = a.queries[4 * (size_t)q];
-    const int pixel = __float_as_int(q0.w);
-    if (pixel < 0) return;
-    float my_dist;
-    int my_slot;
-    const int c = query_wave_list<true>(*a.gp, a.ends, a.pos4, a.box, q0.x, q0.y, q0.z, a.k, my_dist, my_slot);
-    if (c <= 0) return;
-    const float kd = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_dist), a.k - 1));
-    const float rs = c == a.k ? kd : a.radius_sqr;
+// k_merge's sum for query q, whose list holds c photons: lane j weighs list entry j, and the wave
+// adds the lanes' terms in list order (k_merge's loop order).
+__device__ __forceinline__ void merge_query(const GridMergeArgs& a, int q, int pixel, int c, float my_dist,
+                                            int my_slot) {
+    const float rs = c == a.k ? lane_value(my_dist, a.k - 1) : a.radius_sqr;
     if (!(rs > 0.0f)) return;
     const float4 qn = a.queries[4 * (size_t)q + 1];
     const float4 qo = a.queries[4 * (size_t)q + 2];
@@ -372,6 +362,28 @@ __global__ __launch_bounds__(256) void k_merge_grid(GridMergeArgs a) {
         atomicAdd(&a.image[3 * (size_t)pixel + 0], qw.x * sr * scale);
         atomicAdd(&a.image[3 * (size_t)pixel + 1], qw.y * sg * scale);
         atomicAdd(&a.image[3 * (size_t)pixel + 2], qw.z * sb * scale);
+    }
+}
+
+// The grid query and the merge in one launch, `per` queries per wave; the lists keep each photon's
+// grid slot.
+__global__ __launch_bounds__(256) void k_merge_grid(GridMergeArgs a, int per) {
+    const int lane = (int)(threadIdx.x & 63);
+    const int q0 = (blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * per;
+    const int n = min(per, a.nq - q0);
+    if (n <= 0) return;  // whole waves leave together
+    const GridParams g = *a.gp;
+    const float4 q = a.queries[4 * (size_t)(q0 + min(lane >> 3, n - 1))];
+    const bool used = (lane >> 3) < n && __float_as_int(q.w) >= 0;
+    const GridProbes probes = grid_probes(g, a.ends, a.box, q.x, q.y, q.z, used);
+    const unsigned long long found = __ballot(probes.size > 0);
+    for (int i = 0; i < n; i++) {
+        if (((found >> (8 * i)) & 0xff) == 0) continue;
+        float my_dist;
+        int my_slot;
+        const int c = query_wave_list<true>(g, a.pos4, probes, 8 * i, lane_value(q.x, 8 * i), lane_value(q.y, 8 * i),
+                                            lane_value(q.z, 8 * i), a.k, my_dist, my_slot);
+        if (c > 0) merge_query(a, q0 + i, __float_as_int(lane_value(q.w, 8 * i)), c, my_dist, my_slot);
     }
 }
 
@@ -540,7 +552,10 @@ int imba_ppm_merge_grid(const ImbaHashGrid* grid, const void* records, const voi
     a.image = image;
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
-    hipLaunchKernelGGL(k_merge_grid, dim3(ceil_div(nq, 4)), dim3(256), 0, s, a);
+    const DeviceProps* p = device_props();
+    if (!p) return fail(IMBA_ERR_NO_DEVICE, "no HIP device");
+    const int per = queries_per_wave(nq, p->cu_count);
+    hipLaunchKernelGGL(k_merge_grid, dim3(ceil_div(ceil_div(nq, per), 4)), dim3(256), 0, s, a, per);
     IMBA_HIP_TRY(hipGetLastError());
     if (sync) IMBA_HIP_TRY(hipStreamSynchronize(s));
     return IMBA_OK;

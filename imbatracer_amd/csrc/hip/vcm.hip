@@ -737,20 +737,28 @@ __device__ __forceinline__ void merge_epilogue(const Frame& f, const MergeArgs& 
     }
 }
 
-// Grid query and merge in one launch, one query per wave: the k-capped list keeps each
+// Grid query and merge in one launch, `per` query slots per wave: the k-capped list keeps each
 // photon's grid slot, and the merge reads the slot-ordered records next to the positions the
 // scan just read.
-__global__ __launch_bounds__(256) void k_vcm_merge(Frame f, MergeArgs a) {
-    const int q = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-    if (q >= entries(a.capacity, a.count_dev)) return;  // whole waves leave together
-    const float4 q0 = a.queries[4 * (size_t)q];
-    if (__float_as_int(q0.w) < 0) return;
-    float my_dist;
-    int my_slot;
-    const int count = query_wave_list<true>(*a.gp, a.ends, a.pos4, a.box, q0.x, q0.y, q0.z, a.k, my_dist, my_slot);
-    if (count == 0) return;
-    const float kd = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_dist), a.k - 1));
-    merge_epilogue(f, a, q, count, my_dist, my_slot, kd);
+__global__ __launch_bounds__(256) void k_vcm_merge(Frame f, MergeArgs a, int per) {
+    const int lane = (int)(threadIdx.x & 63);
+    const int q0 = (blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * per;
+    const int n = min(per, entries(a.capacity, a.count_dev) - q0);
+    if (n <= 0) return;  // whole waves leave together
+    const GridParams g = *a.gp;
+    const float4 q = a.queries[4 * (size_t)(q0 + min(lane >> 3, n - 1))];
+    const bool used = (lane >> 3) < n && __float_as_int(q.w) >= 0;
+    const GridProbes probes = grid_probes(g, a.ends, a.box, q.x, q.y, q.z, used);
+    const unsigned long long found = __ballot(probes.size > 0);
+    for (int i = 0; i < n; i++) {
+        if (((found >> (8 * i)) & 0xff) == 0) continue;
+        float my_dist;
+        int my_slot;
+        const int count = query_wave_list<true>(g, a.pos4, probes, 8 * i, lane_value(q.x, 8 * i), lane_value(q.y, 8 * i),
+                                                lane_value(q.z, 8 * i), a.k, my_dist, my_slot);
+        if (count == 0) continue;
+        merge_epilogue(f, a, q0 + i, count, my_dist, my_slot, lane_value(my_dist, a.k - 1));
+    }
 }
 
 int check_frame(const ImbaVcmFrame* p, Frame* f) {
@@ -938,7 +946,10 @@ int imba_vcm_merge(const ImbaVcmFrame* frame, const ImbaHashGrid* grid, const vo
     a.image = image;
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
-    hipLaunchKernelGGL(k_vcm_merge, dim3(ceil_div(capacity, 4)), dim3(256), 0, s, f, a);
+    const DeviceProps* p = device_props();
+    if (!p) return fail(IMBA_ERR_NO_DEVICE, "no HIP device");
+    const int per = queries_per_wave(capacity, p->cu_count);
+    hipLaunchKernelGGL(k_vcm_merge, dim3(ceil_div(ceil_div(capacity, per), 4)), dim3(256), 0, s, f, a, per);
     IMBA_HIP_TRY(hipGetLastError());
     if (sync) IMBA_HIP_TRY(hipStreamSynchronize(s));
     return IMBA_OK;

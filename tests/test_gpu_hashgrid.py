@@ -170,3 +170,35 @@ def test_reset_forgets_the_table_history(gpu):
     for j in range(len(q)):
         assert np.array_equal(ia[j, :ca[j]], ib[j, :cb[j]])
         assert np.array_equal(da[j, :ca[j]].view(np.int32), db[j, :cb[j]].view(np.int32))
+
+
+@pytest.mark.parametrize("k", [1, 2, 10, 63, 64])
+def test_query_ties_and_edges(gpu, k):
+    """Photons on a lattice, many of them several times, so that many distances are equal, also at
+    the k-th place (where the reference keeps the latest of the equal ones); bucket sizes around
+    the 64-photon chunks and the groups of four of them; query counts around a wave's and a
+    block's share, and enough queries that every wave takes more than one."""
+    rng = np.random.default_rng(k)
+    lattice = rng.integers(0, 5, (3000, 3)).astype(np.float32) * np.float32(0.02)
+    heaps = [np.repeat(rng.random((1, 3), dtype=np.float32) + 2.0, n, 0) for n in (63, 64, 65, 255, 256, 257, 511)]
+    heaps = [h + rng.integers(0, 3, h.shape).astype(np.float32) * np.float32(0.004) for h in heaps]
+    p = np.concatenate([lattice] + heaps)
+    photons = np.zeros((len(p), 4), np.float32)
+    photons[:, :3] = p[rng.permutation(len(p))]
+    g, _ = _grid(photons, 0.03)
+    og = oracle.Grid()
+    og.build(photons[:, :3], 0.03)
+    near = photons[rng.integers(0, len(p), 70000), :3]
+    near[::2] += rng.integers(-1, 2, near[::2].shape).astype(np.float32) * np.float32(0.01)
+    near[::97] = np.float32(np.inf)
+    idx, dist, cnt = _query(g, near, k)
+    for q in list(range(600)) + list(range(69700, 70000)):
+        want_i, want_d = og.query(near[q], k)
+        assert cnt[q] == len(want_i), q
+        assert np.array_equal(idx[q, :cnt[q]], want_i), q
+        assert np.array_equal(dist[q, :cnt[q]].view(np.int32), want_d.view(np.int32)), q
+    for n in (1, 2, 3, 4, 5, 7, 8, 9):
+        i2, d2, c2 = _query(g, near[:n], k)
+        assert np.array_equal(c2, cnt[:n])
+        for q in range(n):
+            assert np.array_equal(i2[q, :c2[q]], idx[q, :c2[q]])
