@@ -6,6 +6,8 @@ reference loop's exactly; the miss suffix must be the same multiset (the referen
 permutes it) and, for this library, the misses in their original order.
 compact_rays: survivors, their order and the new size must equal the reference loop's.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -107,3 +109,57 @@ def test_sort_by_material_matches_oracle(gpu, count, num_mats):
             assert np.array_equal(ob.download(np.int32, count), want_order)
             got_rays = rb.download(N.RAY_DTYPE, count)
             assert np.array_equal(got_rays.view(np.int32), want_rays.view(np.int32))
+
+
+@pytest.mark.parametrize("words,offset", [(1, 0), (2, 0), (2, 4), (3, 0), (4, 0), (4, 8), (5, 0), (10, 0), (12, 0),
+                                          (12, 4), (16, 0), (67, 0)])
+def test_state_sizes_and_alignment(gpu, words, offset):
+    """States are moved in units of 16, 8 or 4 bytes as their size and addresses allow; queue
+    sizes around waves, chunks and tiles.  Entries past the outputs' ends stay as they were."""
+    for n in (1, 63, 64, 65, 255, 257, 511, 512, 513, 5000):
+        rays, hits, states = _queue(n, 0.6, seed=n * 100 + words, state_words=words)
+        sb = N.DeviceBuffer(states.nbytes + 16)
+        sb.upload(states, offset=offset)
+        rb, hb = N.DeviceBuffer.from_array(rays), N.DeviceBuffer.from_array(hits)
+        ro, ho = N.DeviceBuffer(rays.nbytes + 32), N.DeviceBuffer(hits.nbytes + 16)
+        so = N.DeviceBuffer.from_array(np.full(states.nbytes + 16, 0x5A, np.uint8))
+        k = C.c_int()
+        N.check(N.lib.imba_compact_hits(rb.ptr, hb.ptr, sb.at(offset), 4 * words, n, ro.ptr, ho.ptr, so.at(offset),
+                                        C.byref(k), None), "compact_hits")
+        kept = np.concatenate([np.nonzero(hits["tri_id"] >= 0)[0], np.nonzero(hits["tri_id"] < 0)[0]])
+        assert k.value == (hits["tri_id"] >= 0).sum()
+        assert np.array_equal(ro.download(N.RAY_DTYPE, n).view(np.int32), rays[kept].view(np.int32))
+        assert np.array_equal(ho.download(N.HIT_DTYPE, n).view(np.int32), hits[kept].view(np.int32))
+        assert np.array_equal(so.download(np.int32, n * words, offset=offset).reshape(n, words), states[kept])
+        out = so.download(np.uint8, states.nbytes + 16)
+        assert (out[:offset] == 0x5A).all() and (out[offset + states.nbytes:] == 0x5A).all()
+
+
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 1, 4096 * 2048, 4096 * 2048 + 1])
+def test_tile_and_offset_rules(gpu, n):
+    """Both sides of the sizes where the tile and the way a block gets its offset change, with the
+    size on the device and a workspace of exactly the promised size."""
+    rng = np.random.default_rng(n & 0xffff)
+    states = rng.integers(0, 1 << 30, (n, 1)).astype(np.int32)
+    states[rng.random(n) < 0.4] = -1
+    rays = np.zeros(n, N.RAY_DTYPE)
+    rays["org"][:, 0] = np.arange(n) % (1 << 24)
+    rb, sb = N.DeviceBuffer.from_array(rays), N.DeviceBuffer.from_array(states)
+    ro, so = N.DeviceBuffer(rays.nbytes), N.DeviceBuffer(states.nbytes)
+    size = int(N.lib.imba_compact_workspace_size(n))
+    for count in (0, 700, 600000, n):
+        cnt = N.DeviceBuffer.from_array(np.array([count, -5], np.int32))
+        ws = N.DeviceBuffer.from_array(np.full(size + 64, 0x77, np.uint8))
+        N.check(N.lib.imba_compact_rays_dev(rb.ptr, sb.ptr, 4, n, cnt.ptr, ro.ptr, so.ptr, cnt.at(4), ws.ptr, None),
+                "compact_rays_dev")
+        keep = np.nonzero(states[:count, 0] >= 0)[0]
+        assert cnt.download(np.int32, 2)[1] == len(keep)
+        assert np.array_equal(so.download(np.int32, len(keep)), states[keep, 0])
+        assert np.array_equal(ro.download(N.RAY_DTYPE, len(keep))["org"][:, 0], rays["org"][keep, 0])
+        assert (ws.download(np.uint8, size + 64)[size:] == 0x77).all()
+        # a smaller capacity takes another tile and still fits the workspace
+        cap = min(n, 1 << 20)
+        N.check(N.lib.imba_compact_rays_dev(rb.ptr, sb.ptr, 4, cap, cnt.ptr, ro.ptr, so.ptr, cnt.at(4), ws.ptr, None),
+                "compact_rays_dev")
+        assert cnt.download(np.int32, 2)[1] == (states[:min(count, cap), 0] >= 0).sum()
+        assert (ws.download(np.uint8, size + 64)[size:] == 0x77).all()
