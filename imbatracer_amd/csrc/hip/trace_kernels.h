@@ -217,6 +217,24 @@ struct LaneStack {
         if (sp < STACK_LDS) return lds_view(lds)[sp * BLOCK + lane_slot];
         return spill[(size_t)(sp - STACK_LDS) * spill_stride + spill_slot];
     }
+    // For a quad working on this stack (advance_quad): whether it can hold `top` entries, and a
+    // write of entry e.
+    __device__ __forceinline__ bool holds(int top) const { return top <= STACK_LDS || top - STACK_LDS <= spill_depth; }
+    __device__ __forceinline__ void put(int e, int v) {
+        if (e < STACK_LDS) lds_view(lds)[e * BLOCK + lane_slot] = v;
+        else spill[(size_t)(e - STACK_LDS) * spill_stride + spill_slot] = v;
+    }
+};
+
+// The stack of a ray that has a quad of lanes from the start: the LDS of its four lanes.
+template <int BLOCK, int STACK_LDS>
+struct QuadStack {
+    int* lds;  // [4 * STACK_LDS][BLOCK / 4], the quad's column
+    int sp;
+
+    __device__ __forceinline__ int pop() { return lds_view(lds)[--sp * (BLOCK / 4)]; }
+    __device__ __forceinline__ bool holds(int top) const { return top <= 4 * STACK_LDS; }
+    __device__ __forceinline__ void put(int e, int v) { lds_view(lds)[e * (BLOCK / 4)] = v; }
 };
 
 __device__ __forceinline__ float4 as_float4(const uint4& u) {
@@ -615,16 +633,26 @@ __device__ __forceinline__ void stack_init(LaneStack<BLOCK, STACK_LDS>& st, int*
 }
 
 // ---------------------------------------------------------------------------------------
-// Four lanes per ray (quantized tree, small queues).  The lanes of a quad hold the same ray and
-// go through the same steps; lane j tests child box j of a node and triangle j of a leaf, and
-// the quad sorts with DPP exchanges.  A step is then about half the instructions, a wave lasts
-// as long as the longest of 16 rays instead of 64, and a queue that would leave SIMDs with one
-// wave or none spreads over four times the waves.  Visiting order, and so every hit, is that
-// of `advance`.  The stack of a quad has the LDS of its four lanes (4 * STACK_LDS entries).
+// Four lanes per ray (quantized tree).  The lanes of a quad hold the same ray and go through the
+// same steps; lane j tests child box j of a node and triangle j of a leaf, and the quad sorts with
+// DPP exchanges.  A step is then about half the instructions of one with a lane per ray.
+// Visiting order, and so every hit, is that of `advance`.
+//
+// Small queues start that way (quad_trace): a wave lasts as long as the longest of 16 rays
+// instead of 64, and a queue that would leave SIMDs with one wave or none spreads over four times
+// the waves.  The stack of such a quad has the LDS of its four lanes.
 // MI355X, us per launch, one lane -> four lanes per ray, quantized tree, 65K triangles: 1,000
 // diffuse rays 186 -> 111, 16,000: 209 -> 116, 65,000: 216 -> 153, 130,000: 203 -> 243; primary
 // rays 16,000: 167 -> 95, 130,000: 162 -> 133; shadow rays 65,000: 156 -> 122, 130,000: 161 ->
 // 187; 1M primary rays 360 -> 694 (the chip is full and four lanes do more work per ray).
+//
+// Waves of larger queues start with a lane per ray and go over to it (wave_trace): with 37% (1M
+// primary rays) to 23% (diffuse rays) of the lanes busy on average, most steps of a wave serve few
+// rays.  Moving the state costs about one step.  us per launch before -> now: 1M primary rays
+// 361 -> 353, 1M shadow rays 534 -> 486, 300K diffuse rays over 250K triangles 397 -> 334, 200K rays
+// over masked instances 790 -> 743, 48 queues in a batch 1,040 -> 917; path-traced frame 640x480
+// 4,261 -> 4,002.
+
 // Lane (4 q + k) receives the value of lane 4 q + {A, B, C, D}[k].
 template <int A, int B, int C, int D>
 __device__ __forceinline__ uint32_t quad_u(uint32_t v) {
@@ -664,11 +692,9 @@ __device__ __forceinline__ void quad_best(Candidate& c) {
     c.from = take ? from : c.from;
 }
 
-// One step of a quad's ray, as `advance` for the quantized tree; stack is the quad's column
-// ([depth][BLOCK / 4]), j the lane's place in the quad.
-template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED>
-__device__ __forceinline__ bool advance_quad(const TraceArgs& a, TraceState& s, int* stack, int& sp, int j) {
-    constexpr int kQuads = BLOCK / 4;
+// One step of a quad's ray, as `advance` for the quantized tree; j is the lane's place in the quad.
+template <bool ANY, bool MASKED, typename STACK>
+__device__ __forceinline__ bool advance_quad(const TraceArgs& a, TraceState& s, STACK& st, int j) {
     if (s.kind == kTri) {
         const int t = s.item + 3 * j;
         const bool in = t < a.n_tris4 - 2;
@@ -708,8 +734,8 @@ __device__ __forceinline__ bool advance_quad(const TraceArgs& a, TraceState& s, 
         s.item += 12;
         s.kind = (e0 | e1 | e2 | e3) ? kNone : kTri;
     }
-    if (s.kind == kNone && !resume(s, sp, [&] { return lds_view(stack)[--sp * kQuads]; })) return true;
-    if (s.kind == kInst) inst_step<false>(a, s, sp);
+    if (s.kind == kNone && !resume(s, st.sp, [&] { return st.pop(); })) return true;
+    if (s.kind == kInst) inst_step<false>(a, s, st.sp);
     if (s.kind == kNode) {
         int next = kNoNode;
         const uint32_t n = (uint32_t)s.item;
@@ -733,10 +759,10 @@ __device__ __forceinline__ bool advance_quad(const TraceArgs& a, TraceState& s, 
             quad_order<1, 0, 3, 2>(d, c, !(j & 1));
             quad_order<2, 3, 0, 1>(d, c, j < 2);
             quad_order<0, 2, 1, 3>(d, c, j < 2);
-            const int top = sp + max((int)cnt - 1, 0);
-            if (top <= 4 * STACK_LDS) {
-                if (j > 0 && (uint32_t)j < cnt) lds_view(stack)[(top - j) * kQuads] = (int)c;
-                sp = top;
+            const int top = st.sp + max((int)cnt - 1, 0);
+            if (st.holds(top)) {
+                if (j > 0 && (uint32_t)j < cnt) st.put(top - j, (int)c);
+                st.sp = top;
             } else {
                 s.bad = 1;  // not for the trees the launch was checked for
             }
@@ -761,26 +787,88 @@ __device__ __forceinline__ void write_result(const TraceArgs& a, const TraceStat
     if (s.bad) atomicAdd(a.err, 1);
 }
 
+// Writes the result of a quad's ray.
+__device__ __forceinline__ void write_quad(const TraceArgs& a, TraceState& s, int id, int j) {
+    s.bad |= (int)quad_u<1, 0, 3, 2>((uint32_t)s.bad);
+    s.bad |= (int)quad_u<2, 3, 0, 1>((uint32_t)s.bad);
+    if (j == 0) write_result<false>(a, s, id);
+}
+
 // Traces ray `id` with this thread's quad.
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED>
 __device__ __forceinline__ void quad_trace(const TraceArgs& a, int* lds_stack, int id) {
     const int j = threadIdx.x & 3;
     TraceState s;
     state_init(s, gview(a.rays)[2 * (size_t)id], gview(a.rays)[2 * (size_t)id + 1], a.root);
-    int sp = 0;
-    while (!advance_quad<BLOCK, STACK_LDS, ANY, MASKED>(a, s, lds_stack + (threadIdx.x >> 2), sp, j)) {
+    QuadStack<BLOCK, STACK_LDS> st{lds_stack + (threadIdx.x >> 2), 0};
+    while (!advance_quad<ANY, MASKED>(a, s, st, j)) {
     }
-    s.bad |= (int)quad_u<1, 0, 3, 2>((uint32_t)s.bad);
-    s.bad |= (int)quad_u<2, 3, 0, 1>((uint32_t)s.bad);
-    if (j == 0) write_result<false>(a, s, id);
+    write_quad(a, s, id, j);
 }
+
+__device__ __forceinline__ void from_lane(int& v, int lane) { v = __builtin_amdgcn_ds_bpermute(4 * lane, v); }
+__device__ __forceinline__ void from_lane(float& v, int lane) {
+    v = __int_as_float(__builtin_amdgcn_ds_bpermute(4 * lane, __float_as_int(v)));
+}
+
+// Traces the wave's rays (ray `id` of every lane with `valid`; whole waves call it), one per lane
+// until at most 16 are left, those with a quad of lanes each.
+template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED>
+__device__ __forceinline__ void wave_trace(const TraceArgs& a, LaneStack<BLOCK, STACK_LDS>& st, int id, bool valid) {
+    const int lane = threadIdx.x & 63;
+    TraceState s;
+    const int at = valid ? id : 0;
+    state_init(s, gview(a.rays)[2 * (size_t)at], gview(a.rays)[2 * (size_t)at + 1], a.root);
+    st.sp = 0;
+    bool live = valid;
+    unsigned long long left = __ballot(live);
+    while (__popcll(left) > 16) {
+        if (live && advance<BLOCK, STACK_LDS, ANY, MASKED, false, 2>(a, s, st)) {
+            write_result<false>(a, s, id);
+            live = false;
+        }
+        left = __ballot(live);
+    }
+    if (!left) return;
+    // the r-th ray left goes to quad r: its lane's number to lane 4 r (the other lanes' to a lane
+    // that no one asks), then to the quad, which takes over its state and its stack
+    const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(left >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)left, 0u));
+    const int from = (int)quad_u<0, 0, 0, 0>((uint32_t)__builtin_amdgcn_ds_permute(4 * (live ? 4 * rank : 1), lane));
+    const int j = lane & 3;
+    live = (lane >> 2) < __popcll(left);
+    from_lane(s.world.ox, from); from_lane(s.world.oy, from); from_lane(s.world.oz, from);
+    from_lane(s.world.dx, from); from_lane(s.world.dy, from); from_lane(s.world.dz, from);
+    from_lane(s.world.idx, from); from_lane(s.world.idy, from); from_lane(s.world.idz, from);
+    from_lane(s.cs.ox, from); from_lane(s.cs.oy, from); from_lane(s.cs.oz, from);
+    from_lane(s.cs.dx, from); from_lane(s.cs.dy, from); from_lane(s.cs.dz, from);
+    from_lane(s.cs.idx, from); from_lane(s.cs.idy, from); from_lane(s.cs.idz, from);
+    s.cs.oidx = s.cs.ox * s.cs.idx; s.cs.oidy = s.cs.oy * s.cs.idy; s.cs.oidz = s.cs.oz * s.cs.idz;
+    from_lane(s.tmin, from); from_lane(s.best_t, from); from_lane(s.best_u, from);
+    from_lane(s.best_tri, from); from_lane(s.best_inst, from);
+    from_lane(s.kind, from); from_lane(s.item, from);
+    from_lane(s.inst_id, from); from_lane(s.inst_next, from); from_lane(s.inst_sp, from);
+    from_lane(s.bad, from); from_lane(st.sp, from); from_lane(id, from);
+    LaneStack<BLOCK, STACK_LDS> theirs = st;
+    theirs.lane_slot += from - lane;
+    theirs.spill_slot += from - lane;
+    while (__ballot(live)) {
+        if (live && advance_quad<ANY, MASKED>(a, s, theirs, j)) {
+            write_quad(a, s, id, j);
+            live = false;
+        }
+    }
+}
+
+// Waves per SIMD a traversal kernel is held to: 8 over the BVH2 (64 VGPRs), 7 over the 4-wide tree
+// (72), 6 over the quantized one (80: both mappings of rays to lanes without scratch; held to 7 its
+// 24 bytes of scratch per lane cost batches 5% and frames 1.5%).
+constexpr int min_waves(int tree) { return tree == 0 ? 8 : tree == 1 ? 7 : 6; }
 
 // One ray per thread (rays strided over the grid when it is smaller than the ray count), or four
 // lanes per ray when the launch holds at most a.quad rays (the host then sizes the grid for four
-// threads per ray and has checked the stack).  The 4-wide variants are held to 7 waves per SIMD
-// (72 VGPRs), the BVH2 ones to 8 (64).
+// threads per ray and has checked the stack).
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, bool STATS, int TREE>
-__global__ __launch_bounds__(BLOCK, STATS ? 1 : TREE == 0 ? 8 : 7) void k_trace(TraceArgs a) {
+__global__ __launch_bounds__(BLOCK, STATS ? 1 : min_waves(TREE)) void k_trace(TraceArgs a) {
     __shared__ int lds_stack[STACK_LDS * BLOCK];
     const int count = launch_count(a);
     if constexpr (TREE == 2 && !STATS) {
@@ -794,6 +882,13 @@ __global__ __launch_bounds__(BLOCK, STATS ? 1 : TREE == 0 ? 8 : 7) void k_trace(
     LaneStack<BLOCK, STACK_LDS> st;
     stack_init(st, lds_stack, a);
     const int stride = gridDim.x * BLOCK;
+    if constexpr (TREE == 2 && !STATS) {
+        for (int first = blockIdx.x * BLOCK + (threadIdx.x & ~63); first < count; first += stride) {
+            const int id = first + (threadIdx.x & 63);
+            wave_trace<BLOCK, STACK_LDS, ANY, MASKED>(a, st, id, id < count);
+        }
+        return;
+    }
     for (int id = blockIdx.x * BLOCK + threadIdx.x; id < count; id += stride) {
         TraceState s;
         state_init(s, a.rays[2 * (size_t)id], a.rays[2 * (size_t)id + 1], a.root);
@@ -927,14 +1022,13 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchIt
     }
 }
 
-// The 4-wide variants are held to 7 waves per SIMD (72 VGPRs), the BVH2 ones to 8.
 // QUADS (quantized tree): four lanes per ray, a wave taking a quarter of a chunk at a time.  A
 // kernel of its own: both mappings in one kernel cost the one-lane mapping 7% (48 queues, 1.3M
 // rays: 1,157 us against 1,082).  Where the queue sizes are only known on the device both kernels
 // are launched and `limit` chunks decide which of them works: the one-lane kernel above it, the
 // other up to it (limit < 0: the one-lane kernel always).
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE, bool QUADS>
-__global__ __launch_bounds__(BLOCK, TREE == 0 ? 8 : 7) void k_trace_batch(
+__global__ __launch_bounds__(BLOCK, min_waves(TREE)) void k_trace_batch(
     const BatchItem* __restrict__ items, int first, int n_items, const int* __restrict__ total_chunks, int* counter,
     int* spill, int spill_depth, int limit) {
     __shared__ int lds_stack[STACK_LDS * BLOCK];
@@ -972,7 +1066,9 @@ __global__ __launch_bounds__(BLOCK, TREE == 0 ? 8 : 7) void k_trace_batch(
             if (id < a.count) quad_trace<BLOCK, STACK_LDS, ANY, MASKED>(a, lds_stack, id);
         } else {
             const int id = begin + lane;
-            if (id < a.count) {
+            if constexpr (TREE == 2) {
+                wave_trace<BLOCK, STACK_LDS, ANY, MASKED>(a, st, id, id < a.count);
+            } else if (id < a.count) {
                 TraceState s;
                 state_init(s, gview(a.rays)[2 * (size_t)id], gview(a.rays)[2 * (size_t)id + 1], a.root);
                 st.sp = 0;

@@ -70,12 +70,13 @@ int not_capturing(hipStream_t s, const char* what) {
     return IMBA_OK;
 }
 
-// Most rays a launch over the quantized tree traces with four lanes each: six waves of 16 rays
-// per SIMD (98,304 on 256 CUs).  Around there the chip is full with either mapping and one lane
-// per ray, which does less work in all, overtakes (trace_kernels.h has both sides, between 65,000
-// and 130,000 rays).  A quad's stack is the LDS of its four lanes, without a spill buffer.
+// Most rays a launch over the quantized tree traces with four lanes each from the start: five
+// waves of 16 rays per SIMD (81,920 on 256 CUs).  us with four lanes -> with waves that start with
+// one: 65,000 diffuse / primary / shadow rays 152 / 103 / 131 -> 159 / 132 / 137, 80,000: 171 /
+// 118 / 141 -> 167 / 138 / 134, 96,000: 195 / 124 / 152 -> 168 / 141 / 141.  A quad's stack is the
+// LDS of its four lanes, without a spill buffer.
 int quad_rays(const DeviceProps* p, int max_stack, int stack_lds) {
-    return max_stack <= 4 * stack_lds ? p->cu_count * 4 * 6 * 16 : 0;
+    return max_stack <= 4 * stack_lds ? p->cu_count * 4 * 5 * 16 : 0;
 }
 
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, bool STATS, int TREE>

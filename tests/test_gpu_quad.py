@@ -1,8 +1,9 @@
-"""Small queues over the quantized tree are traced with four lanes per ray: hits equal the
-one-lane-per-ray launch's bit for bit (closest and any hit) and the oracle's closest hits, at the
-edges of quads, waves and the largest queue that takes this path, over leaves longer than a quad,
-instances and masks, for device-side counts and batches; closest hits of the default launch
-equal the BVH2's.
+"""Small queues over the quantized tree are traced with four lanes per ray, and waves of larger ones
+go over to that when 16 rays are left: hits equal those of the persistent kernel (one lane per
+ray throughout) bit for bit, closest and any hit, and the oracle's closest hits, at the edges of
+quads, waves and the largest queue that starts this way, over leaves longer than a quad, stacks
+deeper than the LDS part, instances and masks, for device-side counts and batches; closest hits
+of the default launch equal the BVH2's.
 """
 import numpy as np
 import pytest
@@ -15,9 +16,10 @@ from tests import scenes as T
 pytestmark = pytest.mark.gpu
 
 Q4 = N.TraceConfig(256, 16, 0, 0, 4, 1, 0)
-ONE_LANE = N.TraceConfig(256, 16, 0, 64, 4, 1, 0)  # an explicit grid: one lane per ray at any size
+STRIDED = N.TraceConfig(256, 8, 0, 1, 4, 1, 0)  # one block per CU, rays strided, 8 stack entries in LDS
+ONE_LANE = N.TraceConfig(256, 16, 1, 0, 4, 1, 0)  # the persistent kernel
 BVH2 = N.TraceConfig(256, 16, 0, 0, 2, 0, 0)
-LARGEST = 98304  # on 256 CUs
+LARGEST = 81920  # on 256 CUs
 
 
 def _same(a, b):
@@ -53,6 +55,8 @@ def test_sizes(gpu, name):
         assert _same(sc.trace_host(rays[:n], cfg=Q4), want[:n]), n
         assert _same(sc.trace_host(rays[:n]), want[:n]), n
         assert _same(sc.trace_host(rays[:n], any_hit=True, cfg=Q4), want_any[:n]), n
+        assert _same(sc.trace_host(rays[:n], cfg=STRIDED), want[:n]), n
+        assert _same(sc.trace_host(rays[:n], any_hit=True, cfg=STRIDED), want_any[:n]), n
     assert _same(sc.trace_host(rays, cfg=BVH2), want)
     assert sc.error_count() == 0
 
@@ -98,6 +102,7 @@ def test_recorded_batch(gpu):
     sc = S.Scene(b.desc())
     rays = T.random_rays(LARGEST + 3000, seed=10)
     want = sc.trace_host(rays, cfg=BVH2)
+    assert sc.stack_depths(rays, cfg=Q4)[17:].sum() > 0
     rb, hb = N.DeviceBuffer.from_array(rays), N.DeviceBuffer(16 * len(rays))
     for cfg in (None, Q4):
         st = N.Stream()
