@@ -37,9 +37,7 @@ struct ImbaHashGrid {
     int box_cap = 0;
     imba::GridParams* d_params = nullptr;
     float* partial = nullptr;  // 6 per bounds block
-    int* scan_tmp = nullptr;   // tile maxima of the ends scan
-    int scan_cap = 0;
-    int* digits = nullptr;     // radix digit counts
+    int* digits = nullptr;     // the sort's tile counts
     int digits_cap = 0;
 };
 

@@ -2,14 +2,19 @@
 //
 // HashGrid (rangesearch/rangesearch.h:21-158) builds on the host with TBB: bounds reduce,
 // atomic count per bucket, serial exclusive scan, atomic scatter.  Here:
-//   bounds   k_bounds (per-block min/max) + k_params (combine, grow by 0.1%, derived values)
-//   keys     k_grid_keys: bucket of each photon, paired with the photon index
-//   sort     stable LSD radix sort of the pairs by bucket (radix.h): the slot order is by
+//   bounds   k_bounds (per-block min/max; it also clears the bucket ends)
+//   keys     k_grid_keys combines the bounds (grown by 0.1%, derived values) and writes the
+//            bucket of each photon and the sort's first tile counts
+//   sort     stable LSD radix sort of the photon indices by bucket (radix.h): the slot order is by
 //            bucket, then by photon index, which is deterministic and equals a serial run of
 //            the reference's scatter
-//   ends     k_mark_ends writes slot + 1 at the last slot of each bucket, an inclusive max-scan
-//            (k_max_tiles / k_max_top / k_max_apply) carries it over the empty buckets
-//   gather   positions copied to slot order as float4 (x, y, z, index bits)
+//   slots    k_slots: positions copied to slot order as float4 (x, y, z, index bits), slot + 1 at
+//            the last slot of each bucket into its end
+//   boxes    k_bucket_box: bounds of each bucket's photons
+//   ends     k_ends carries the ends over the empty buckets (an inclusive max-scan; what comes
+//            before a tile of buckets is found by searching the sorted keys)
+// 4M photons, 8M buckets: 444 us in 26 launches before the sort was rewritten and the smaller
+// launches were merged, now 331 in 13.
 // The query visits the same 8 buckets in the same order as the reference (duplicates
 // included), one query per wave, and keeps the k-capped, distance-sorted list in lanes 0..k-1
 // with the reference's insertion rule.  Squared distances are computed without fused
@@ -26,162 +31,217 @@
 namespace imba {
 namespace {
 
-constexpr int kBoundsBlocks = 1024;
+constexpr int kBoundsBlocks = 512;
 constexpr int kBlock = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kBlock * kScanItems;
-constexpr int kSortItems = 16;  // radix tiles of 4096 pairs
+constexpr int kSortItems = 16;  // radix tiles of 4096 entries
 
 __device__ __forceinline__ const float* photon_pos(const unsigned char* base, int stride, int off, int i) {
     return reinterpret_cast<const float*>(base + (size_t)i * stride + off);
 }
 
-__global__ __launch_bounds__(kBlock) void k_bounds(const unsigned char* ph, int stride, int off, int n, float* partial) {
-    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
-        const float* p = photon_pos(ph, stride, off, i);
-        for (int k = 0; k < 3; k++) {
-            const float v = p[k];
-            lo[k] = lo[k] < v ? lo[k] : v;
-            hi[k] = hi[k] > v ? hi[k] : v;
+__device__ __forceinline__ float pick_min(float a, float b) { return a < b ? a : b; }
+__device__ __forceinline__ float pick_max(float a, float b) { return a > b ? a : b; }
+
+// Block-wide bounds of the threads' bounds (min / max are exact in any order), in every thread.
+__device__ __forceinline__ void block_bounds(float* lo, float* hi) {
+    __shared__ float red[6][kBlock / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        for (int o = 32; o > 0; o >>= 1) {
+            lo[k] = pick_min(lo[k], __shfl_xor(lo[k], o, 64));
+            hi[k] = pick_max(hi[k], __shfl_xor(hi[k], o, 64));
+        }
+        if (lane == 0) {
+            red[k][wave] = lo[k];
+            red[3 + k][wave] = hi[k];
         }
     }
-    __shared__ float red[6][kBlock];
-    for (int k = 0; k < 3; k++) { red[k][threadIdx.x] = lo[k]; red[3 + k][threadIdx.x] = hi[k]; }
     __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            for (int k = 0; k < 3; k++) {
-                const float a = red[k][threadIdx.x], b = red[k][threadIdx.x + s];
-                red[k][threadIdx.x] = a < b ? a : b;
-                const float c = red[3 + k][threadIdx.x], d = red[3 + k][threadIdx.x + s];
-                red[3 + k][threadIdx.x] = c > d ? c : d;
-            }
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+        for (int w = 0; w < kBlock / 64; w++) {
+            lo[k] = pick_min(lo[k], red[k][w]);
+            hi[k] = pick_max(hi[k], red[3 + k][w]);
         }
-        __syncthreads();
-    }
-    if (threadIdx.x < 6) partial[6 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
 }
 
-// One block: the per-block bounds reduced to the photon bounds (min / max are exact in any
-// order), then the grid parameters.
-__global__ __launch_bounds__(kBlock) void k_params(const float* partial, int nparts, GridParams* gp, float radius,
-                                                   int table_size, int count) {
+// Bounds of the photons, one box per block, and the bucket ends cleared (a kernel's stores rather
+// than a memset node, so the build can be captured in a graph).
+__global__ __launch_bounds__(kBlock) void k_bounds(const unsigned char* ph, int stride, int off, int n, float* partial,
+                                                   int* ends, int table) {
+    float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
+    const int step = gridDim.x * kBlock;
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += step) {
+        const float* p = photon_pos(ph, stride, off, i);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            const float v = p[k];
+            lo[k] = pick_min(lo[k], v);
+            hi[k] = pick_max(hi[k], v);
+        }
+    }
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < table; i += step) ends[i] = 0;
+    block_bounds(lo, hi);
+    if (threadIdx.x < 6) partial[6 * blockIdx.x + threadIdx.x] = threadIdx.x < 3 ? lo[threadIdx.x] : hi[threadIdx.x - 3];
+}
+
+// Every block combines the bounds of all (a few KB from L2) into the grid parameters; block 0 stores
+// them for the later kernels.  Then the bucket of each photon of the block's tile, and the tile's
+// counts of the keys' lowest digit.
+__global__ __launch_bounds__(kBlock) void k_grid_keys(const unsigned char* ph, int stride, int off, int n,
+                                                      const float* partial, int nparts, GridParams* gp, float radius,
+                                                      int table, int* keys, int n_tiles, int* counts) {
+    __shared__ RadixTile<kSortItems> tile;
     float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     for (int b = threadIdx.x; b < nparts; b += kBlock)
         for (int k = 0; k < 3; k++) {
-            const float a = partial[6 * b + k], c = partial[6 * b + 3 + k];
-            lo[k] = lo[k] < a ? lo[k] : a;
-            hi[k] = hi[k] > c ? hi[k] : c;
+            lo[k] = pick_min(lo[k], partial[6 * b + k]);
+            hi[k] = pick_max(hi[k], partial[6 * b + 3 + k]);
         }
-    __shared__ float red[6][kBlock];
-    for (int k = 0; k < 3; k++) { red[k][threadIdx.x] = lo[k]; red[3 + k][threadIdx.x] = hi[k]; }
-    __syncthreads();
-    for (int s = kBlock / 2; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) {
-            for (int k = 0; k < 3; k++) {
-                const float a = red[k][threadIdx.x], b = red[k][threadIdx.x + s];
-                red[k][threadIdx.x] = a < b ? a : b;
-                const float c = red[3 + k][threadIdx.x], d = red[3 + k][threadIdx.x + s];
-                red[3 + k][threadIdx.x] = c > d ? c : d;
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x != 0) return;
-    for (int k = 0; k < 3; k++) { lo[k] = red[k][0]; hi[k] = red[3 + k][0]; }
+    block_bounds(lo, hi);
+    GridParams g;
     for (int k = 0; k < 3; k++) {
         const float e = hi[k] - lo[k];
-        gp->bmax[k] = hi[k] + e * 0.001f;
-        gp->bmin[k] = lo[k] - e * 0.001f;
+        g.bmax[k] = hi[k] + e * 0.001f;
+        g.bmin[k] = lo[k] - e * 0.001f;
     }
-    gp->radius = radius;
-    gp->radius_sqr = radius * radius;
-    gp->cell_size = radius * 2.0f;
-    gp->inv_cell_size = 1.0f / gp->cell_size;
-    gp->table_size = table_size;
-    gp->count = count;
+    g.radius = radius;
+    g.radius_sqr = radius * radius;
+    g.cell_size = radius * 2.0f;
+    g.inv_cell_size = 1.0f / g.cell_size;
+    g.table_size = table;
+    g.count = n;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *gp = g;
+    if (n == 0) return;
+    tile.clear();
+    float p[kSortItems][3];
+#pragma unroll
+    for (int it = 0; it < kSortItems; it++) {
+        const float* q = photon_pos(ph, stride, off, min(tile.index(it), n - 1));
+        for (int k = 0; k < 3; k++) p[it][k] = q[k];
+    }
+#pragma unroll
+    for (int it = 0; it < kSortItems; it++) {
+        const int i = tile.index(it);
+        if (i < n) {
+            const int cx = (int)floorf(g.inv_cell_size * (p[it][0] - g.bmin[0]));
+            const int cy = (int)floorf(g.inv_cell_size * (p[it][1] - g.bmin[1]));
+            const int cz = (int)floorf(g.inv_cell_size * (p[it][2] - g.bmin[2]));
+            const int key = bucket_of((uint32_t)cx, (uint32_t)cy, (uint32_t)cz, table);
+            keys[i] = key;
+            tile.add(key & 255);
+        }
+    }
+    tile.store(counts, n_tiles);
 }
 
-// Zero fill (a kernel rather than a memset node, so the build can be captured in a graph).
-__global__ __launch_bounds__(kBlock) void k_zero(int* p, int n) {
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) p[i] = 0;
+// Slot order: the photons' positions (four scattered reads of a thread in flight together), and at
+// a bucket's first slot its box cleared, at its last slot its end (the empty buckets' ends were
+// cleared before).
+constexpr int kSlotItems = 4;
+__global__ __launch_bounds__(kBlock) void k_slots(const unsigned char* ph, int stride, int off, int n, const int* order,
+                                                  const int* keys_sorted, float4* pos4, int* ends, uint32_t* box) {
+    const int base = blockIdx.x * kBlock * kSlotItems + (int)threadIdx.x;
+    float p[kSlotItems][3];
+    int idx[kSlotItems];
+#pragma unroll
+    for (int it = 0; it < kSlotItems; it++) idx[it] = order[min(base + it * kBlock, n - 1)];
+#pragma unroll
+    for (int it = 0; it < kSlotItems; it++) {
+        const float* q = photon_pos(ph, stride, off, idx[it]);
+        for (int k = 0; k < 3; k++) p[it][k] = q[k];
+    }
+#pragma unroll
+    for (int it = 0; it < kSlotItems; it++) {
+        const int s = base + it * kBlock;
+        if (s >= n) break;
+        pos4[s] = make_float4(p[it][0], p[it][1], p[it][2], __int_as_float(idx[it]));
+        const int b = keys_sorted[s];
+        if (s == n - 1 || keys_sorted[s + 1] != b) ends[b] = s + 1;
+        if (s == 0 || keys_sorted[s - 1] != b) {
+            uint32_t* e = box + 6 * (size_t)b;
+            e[0] = e[1] = e[2] = 0xFFFFFFFFu;  // min over nothing
+            e[3] = e[4] = e[5] = 0u;           // max over nothing
+        }
+    }
 }
 
-
-__global__ __launch_bounds__(kBlock) void k_grid_keys(const unsigned char* ph, int stride, int off, int n,
-                                                      const GridParams* gp, int* keys, int* vals) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const float* p = photon_pos(ph, stride, off, i);
-    const float inv = gp->inv_cell_size;
-    const int cx = (int)floorf(inv * (p[0] - gp->bmin[0]));
-    const int cy = (int)floorf(inv * (p[1] - gp->bmin[1]));
-    const int cz = (int)floorf(inv * (p[2] - gp->bmin[2]));
-    keys[i] = bucket_of((uint32_t)cx, (uint32_t)cy, (uint32_t)cz, gp->table_size);
-    vals[i] = i;
+// One step of a scan over the wave's runs of equal keys: the bounds of the lane that the DPP control
+// names (in the rows of the mask) join this lane's if its key is the same.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ void join_bounds(int key, uint32_t* lo, uint32_t* hi) {
+    const bool same = __builtin_amdgcn_update_dpp(~key, key, CTRL, ROWS, 0xF, false) == key;
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp((int)lo[a], (int)lo[a], CTRL, ROWS, 0xF, false);
+        const uint32_t h = (uint32_t)__builtin_amdgcn_update_dpp((int)hi[a], (int)hi[a], CTRL, ROWS, 0xF, false);
+        lo[a] = same ? min(lo[a], l) : lo[a];
+        hi[a] = same ? max(hi[a], h) : hi[a];
+    }
 }
 
-// ends[b] = 1 + the last slot of bucket b, for the buckets that hold photons (the others
-// were zeroed).
-__global__ __launch_bounds__(kBlock) void k_mark_ends(const int* keys, int n, int* ends) {
+// Bounds of every non-empty bucket's photons (the queries skip buckets that lie beyond their
+// limit; an empty bucket's entry is never used), in the order-preserving integer form of
+// grid_query.h so that atomic min / max can combine them.  Every wave takes 64 consecutive slots
+// and reduces the runs of equal keys with DPP row shifts and broadcasts (the keys are sorted, so
+// equal keys are contiguous; with shuffles through LDS this took 39 us for 4M photons); the last lane
+// of each run combines the run's bounds into the bucket's entry with six atomics.  Hot buckets
+// thus cost one atomic per 64 photons.
+__global__ __launch_bounds__(kBlock) void k_bucket_box(const int* keys_sorted, int n, const float4* pos4, uint32_t* box) {
     const int s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= n) return;
-    const int b = keys[s];
-    if (s == n - 1 || keys[s + 1] != b) ends[b] = s + 1;
-}
-
-// Inclusive max-scan of `n` ints in place: per-tile maxima, a one-block exclusive max-scan of
-// the maxima, then each tile is scanned again from its offset.  Values are >= 0.
-__global__ __launch_bounds__(kBlock) void k_max_tiles(const int* in, int n, int* tile_max) {
-    __shared__ int ws[kBlock / 64];
-    const int base = blockIdx.x * kScanTile;
-    int m = 0;
-    for (int it = 0; it < kScanItems; it++) {
-        const int i = base + it * kBlock + threadIdx.x;
-        if (i < n) m = max(m, in[i]);
-    }
-    for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_down(m, o, 64));
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int w = 0; w < kBlock / 64; w++) t = max(t, ws[w]);
-        tile_max[blockIdx.x] = t;
+    const int lane = threadIdx.x & 63;
+    const bool valid = s < n;
+    const int key = valid ? keys_sorted[s] : -1;
+    const float4 p = pos4[min(s, n - 1)];
+    uint32_t lo[3], hi[3];
+    lo[0] = hi[0] = ordered_bits(p.x);
+    lo[1] = hi[1] = ordered_bits(p.y);
+    lo[2] = hi[2] = ordered_bits(p.z);
+    join_bounds<0x111, 0xF>(key, lo, hi);  // row_shr:1, 2, 4, 8: the 16 lanes of a row
+    join_bounds<0x112, 0xF>(key, lo, hi);
+    join_bounds<0x114, 0xF>(key, lo, hi);
+    join_bounds<0x118, 0xF>(key, lo, hi);
+    join_bounds<0x142, 0xA>(key, lo, hi);  // row_bcast:15: the last lane of rows 0, 2 to rows 1, 3
+    join_bounds<0x143, 0xC>(key, lo, hi);  // row_bcast:31: lane 31 to rows 2 and 3
+    const int next = __shfl_down(key, 1, 64);
+    if (!valid || (lane < 63 && next == key)) return;  // not the last lane of its run
+    uint32_t* e = box + 6 * (size_t)key;
+    for (int a = 0; a < 3; a++) {
+        atomicMin(e + a, lo[a]);
+        atomicMax(e + 3 + a, hi[a]);
     }
 }
 
-__global__ __launch_bounds__(1024) void k_max_top(int* v, int nt) {
-    __shared__ int part[1024];
-    const int t = threadIdx.x;
-    const int per = (nt + 1023) / 1024;
-    const int b0 = min(nt, t * per), b1 = min(nt, b0 + per);
-    int m = 0;
-    for (int b = b0; b < b1; b++) m = max(m, v[b]);
-    part[t] = m;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        const int x = t >= d ? part[t - d] : 0;
-        __syncthreads();
-        part[t] = max(part[t], x);
-        __syncthreads();
+// Photons in buckets before `bucket`: the first slot whose key is not less, searched 64 places at a
+// time by a wave.
+__device__ __forceinline__ int slots_before(const int* keys_sorted, int n, int bucket) {
+    const int lane = threadIdx.x & 63;
+    int lo = 0, len = n;  // the answer lies in [lo, lo + len]
+    while (len > 0) {
+        const int step = (len + 63) / 64;
+        const int at = lo + lane * step;
+        const bool less = at < lo + len && keys_sorted[at] < bucket;
+        const int k = __popcll(__ballot(less));  // the first k probes are less
+        if (k == 0) return lo;
+        const int end = lo + len;
+        lo += (k - 1) * step + 1;
+        len = min(step - 1, end - lo);
     }
-    int run = t > 0 ? part[t - 1] : 0;
-    for (int b = b0; b < b1; b++) {
-        const int c = v[b];
-        v[b] = run;
-        run = max(run, c);
-    }
+    return lo;
 }
 
-__global__ __launch_bounds__(kBlock) void k_max_apply(int* v, int n, const int* tile_offsets) {
+// Inclusive max-scan of the bucket ends in place, a tile of buckets per block.
+__global__ __launch_bounds__(kBlock) void k_ends(int* v, int table, const int* keys_sorted, int n) {
     __shared__ int wmax[kBlock / 64];
     const int base = blockIdx.x * kScanTile;
-    int run = tile_offsets[blockIdx.x];
+    int run = slots_before(keys_sorted, n, base);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (int it = 0; it < kScanItems; it++) {
         const int i = base + it * kBlock + threadIdx.x;
-        int x = i < n ? v[i] : 0;
+        int x = i < table ? v[i] : 0;
         for (int o = 1; o < 64; o <<= 1) {
             const int y = __shfl_up(x, o, 64);
             if (lane >= o) x = max(x, y);
@@ -193,67 +253,9 @@ __global__ __launch_bounds__(kBlock) void k_max_apply(int* v, int n, const int* 
             if (w < wave) wm = max(wm, wmax[w]);
             total = max(total, wmax[w]);
         }
-        if (i < n) v[i] = max(run, max(wm, x));
+        if (i < table) v[i] = max(run, max(wm, x));
         run = max(run, total);
         __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_gather_pos(const unsigned char* ph, int stride, int off, int n, const int* order,
-                                                       float4* pos4) {
-    const int s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= n) return;
-    const int i = order[s];
-    const float* p = photon_pos(ph, stride, off, i);
-    pos4[s] = make_float4(p[0], p[1], p[2], __int_as_float(i));
-}
-
-// Bounds of every non-empty bucket's photons (the queries skip buckets that lie beyond their
-// limit; an empty bucket's entry is never read), in the order-preserving integer form of
-// grid_query.h so that atomic min / max can combine them.  First the first slot of every bucket
-// run in the sorted keys resets its bucket's entry; then every wave takes 64 consecutive slots,
-// reduces the runs of equal keys within the wave (shift-down doubling: keys are sorted, so equal
-// keys are contiguous) and the first lane of each run combines the run's bounds into the bucket's
-// entry with six atomics.  Hot buckets thus cost one atomic per 64 photons.
-__global__ __launch_bounds__(kBlock) void k_bucket_box_reset(const int* keys_sorted, int n, uint32_t* box) {
-    const int s = blockIdx.x * kBlock + threadIdx.x;
-    if (s >= n) return;
-    const int b = keys_sorted[s];
-    if (s > 0 && keys_sorted[s - 1] == b) return;
-    uint32_t* e = box + 6 * (size_t)b;
-    e[0] = e[1] = e[2] = 0xFFFFFFFFu;  // min over nothing
-    e[3] = e[4] = e[5] = 0u;           // max over nothing
-}
-
-__global__ __launch_bounds__(kBlock) void k_bucket_box(const int* keys_sorted, int n, const float4* pos4, uint32_t* box) {
-    const int s = blockIdx.x * kBlock + threadIdx.x;
-    const int lane = threadIdx.x & 63;
-    const bool valid = s < n;
-    const int key = valid ? keys_sorted[s] : -1;
-    uint32_t lo[3] = {0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu}, hi[3] = {0u, 0u, 0u};
-    if (valid) {
-        const float4 p = pos4[s];
-        lo[0] = hi[0] = ordered_bits(p.x);
-        lo[1] = hi[1] = ordered_bits(p.y);
-        lo[2] = hi[2] = ordered_bits(p.z);
-    }
-    for (int off = 1; off < 64; off <<= 1) {
-        const int k2 = __shfl_down(key, off, 64);
-        const bool take = lane + off < 64 && k2 == key;
-        for (int a = 0; a < 3; a++) {
-            const uint32_t l2 = __shfl_down(lo[a], off, 64), h2 = __shfl_down(hi[a], off, 64);
-            if (take) {
-                lo[a] = min(lo[a], l2);
-                hi[a] = max(hi[a], h2);
-            }
-        }
-    }
-    const int kprev = __shfl_up(key, 1, 64);
-    if (!valid || (lane > 0 && kprev == key)) return;  // not the first lane of its run
-    uint32_t* e = box + 6 * (size_t)key;
-    for (int a = 0; a < 3; a++) {
-        atomicMin(e + a, lo[a]);
-        atomicMax(e + 3 + a, hi[a]);
     }
 }
 
@@ -441,7 +443,7 @@ int imba_hashgrid_create(ImbaHashGrid** out) {
 int imba_hashgrid_release(ImbaHashGrid* g) {
     if (!g) return IMBA_OK;
     void* ptrs[] = {g->cell_ends, g->order, g->keys_a, g->vals_a, g->keys_b, g->vals_b, g->pos4, g->d_params,
-                    g->partial, g->scan_tmp, g->digits, g->bucket_box};
+                    g->partial, g->digits, g->bucket_box};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     delete g;
@@ -480,11 +482,6 @@ int imba_hashgrid_build(ImbaHashGrid* g, const void* photons, int stride, int po
         c = 0; if ((r = ensure(g->pos4, c, count))) return r;
         g->cap = count;
     }
-    const int ntiles = ceil_div(std::max(table, 1), kScanTile);
-    if (ntiles > g->scan_cap) {
-        int r = ensure(g->scan_tmp, g->scan_cap, ntiles);
-        if (r) return r;
-    }
     const int ndigits = (int)radix_counts_size<kSortItems>(std::max(count, 1));
     if (ndigits > g->digits_cap) {
         int r = ensure(g->digits, g->digits_cap, ndigits);
@@ -492,33 +489,24 @@ int imba_hashgrid_build(ImbaHashGrid* g, const void* photons, int stride, int po
     }
     g->count = count;
     const unsigned char* ph = (const unsigned char*)photons;
-    const int nparts = count > 0 ? std::min(kBoundsBlocks, ceil_div(count, kBlock)) : 0;
-    if (count > 0) hipLaunchKernelGGL(k_bounds, dim3(nparts), dim3(kBlock), 0, s, ph, stride, pos_offset, count, g->partial);
-    hipLaunchKernelGGL(k_params, dim3(1), dim3(kBlock), 0, s, g->partial, nparts, g->d_params, radius, table, count);
-    if (table > 0)
-        hipLaunchKernelGGL(k_zero, dim3(std::min(ceil_div(table, kBlock), 4096)), dim3(kBlock), 0, s, g->cell_ends,
-                           table);
+    const int nparts = std::min(kBoundsBlocks, std::max(1, ceil_div(std::max(count, table / 8), kBlock)));
+    const int n_tiles = radix_tiles<kSortItems>(count);
+    hipLaunchKernelGGL(k_bounds, dim3(nparts), dim3(kBlock), 0, s, ph, stride, pos_offset, count, g->partial,
+                       g->cell_ends, table);
+    hipLaunchKernelGGL(k_grid_keys, dim3(std::max(1, n_tiles)), dim3(kBlock), 0, s, ph, stride, pos_offset, count,
+                       g->partial, nparts, g->d_params, radius, table, g->keys_a, n_tiles, g->digits);
     if (count > 0) {
-        hipLaunchKernelGGL(k_grid_keys, dim3(ceil_div(count, kBlock)), dim3(kBlock), 0, s, ph, stride, pos_offset,
-                           count, g->d_params, g->keys_a, g->vals_a);
         int bits = 1;
         while (bits < 31 && (1 << bits) < table) bits++;  // buckets are < table
         int* keys_sorted = nullptr;
-        radix_sort_pairs<kSortItems>(g->keys_a, g->vals_a, g->keys_b, g->vals_b, count, bits, g->digits, g->order,
-                                     &keys_sorted, s);
-        hipLaunchKernelGGL(k_mark_ends, dim3(ceil_div(count, kBlock)), dim3(kBlock), 0, s, keys_sorted, count,
-                           g->cell_ends);
-        hipLaunchKernelGGL(k_gather_pos, dim3(ceil_div(count, kBlock)), dim3(kBlock), 0, s, ph, stride, pos_offset,
-                           count, g->order, g->pos4);
-        hipLaunchKernelGGL(k_bucket_box_reset, dim3(ceil_div(count, kBlock)), dim3(kBlock), 0, s, keys_sorted, count,
-                           g->bucket_box);
+        radix_sort<kSortItems>(g->keys_a, g->keys_b, g->vals_a, g->vals_b, count, bits, g->digits, g->order,
+                               &keys_sorted, s);
+        hipLaunchKernelGGL(k_slots, dim3(ceil_div(count, kBlock * kSlotItems)), dim3(kBlock), 0, s, ph, stride,
+                           pos_offset, count, g->order, keys_sorted, g->pos4, g->cell_ends, g->bucket_box);
         hipLaunchKernelGGL(k_bucket_box, dim3(ceil_div(count, kBlock)), dim3(kBlock), 0, s, keys_sorted, count, g->pos4,
                            g->bucket_box);
-    }
-    if (table > 0) {
-        hipLaunchKernelGGL(k_max_tiles, dim3(ntiles), dim3(kBlock), 0, s, g->cell_ends, table, g->scan_tmp);
-        hipLaunchKernelGGL(k_max_top, dim3(1), dim3(1024), 0, s, g->scan_tmp, ntiles);
-        hipLaunchKernelGGL(k_max_apply, dim3(ntiles), dim3(kBlock), 0, s, g->cell_ends, table, g->scan_tmp);
+        hipLaunchKernelGGL(k_ends, dim3(ceil_div(table, kScanTile)), dim3(kBlock), 0, s, g->cell_ends, table,
+                           keys_sorted, count);
     }
     IMBA_HIP_TRY(hipGetLastError());
     if (sync) IMBA_HIP_TRY(hipStreamSynchronize(s));

@@ -1,18 +1,22 @@
-// Stable LSD radix sort of (int key, int value) pairs by 8-bit digits, shared by the material
-// sort and the hash-grid build.
+// Stable LSD radix sort of int keys by 8-bit digits, with the entries' original indices as values,
+// shared by the material sort and the hash-grid build.
 //
-// One pass over a digit:
-//   1. k_radix_hist: per tile of 256 x ITEMS entries, a 256-bin histogram (LDS atomics),
-//      stored digit-major so that one exclusive scan gives every (digit, tile) its first
-//      position;
-//   2. k_radix_scan_sums / _top / _apply: exclusive scan of the 256 x tiles counts;
-//   3. k_radix_scatter: per tile, in ITEMS chunks of 256 entries in order, each wave ranks its
-//      lanes among the lanes with the same digit (eight ballots, one per digit bit), the waves'
-//      per-digit counts in LDS give the offsets of the earlier waves, and a running per-digit
-//      count carries over between chunks.
-// Entries with equal digits keep their order, so after the passes over all key bits the pairs
-// are ordered by key and, for equal keys, as they came in.
-// Traffic per entry and pass: key read twice, value once, both written once (20 B).
+// One pass over a digit, in tiles of 256 x ITEMS entries:
+//   1. the tile's 256-bin histogram (LDS atomics, one histogram per wave), stored digit-major;
+//      the first pass's is left by the kernel that writes the keys (RadixTile);
+//   2. k_radix_rows: one block per digit turns its row of tile counts into offsets, the digit's
+//      total beside them;
+//   3. k_radix_scatter: each wave takes 64 x ITEMS consecutive entries, all loaded at once, and ranks
+//      them (eight ballots per 64, one per digit bit, a running count per digit in LDS that only
+//      this wave touches, so without barriers); the tile is put in digit order in LDS and
+//      written out in that order, neighbouring lanes to neighbouring places.
+// Entries with equal digits keep their order, so after the passes over all key bits the entries
+// are ordered by key and, for equal keys, by index.
+// Traffic per entry and pass: key read twice, value once, both written once (20 B; the first pass
+// reads neither values nor, for its counts, keys).  4M entries, 23-bit keys: a pass took 77 us in
+// five launches (49 of them the scatter, with four barriers per 256 entries and every lane writing
+// where its entry goes), now 38 in three: counts 12, rows 5, scatter 21 (64 MB, 3 TB/s; the ballots
+// and LDS work of a tile keep it from the copy rate).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -26,181 +30,193 @@ constexpr int kRadixBlock = 256;
 constexpr int kRadixWaves = kRadixBlock / 64;
 
 template <int ITEMS>
-__global__ __launch_bounds__(kRadixBlock) void k_radix_hist(const int* __restrict__ keys, int n, int shift,
-                                                            int n_tiles, int* counts) {
-    __shared__ int hist[256];
-    hist[threadIdx.x] = 0;
-    __syncthreads();
-    const int base = blockIdx.x * kRadixBlock * ITEMS;
+inline int radix_tiles(int n) {
+    return (n + kRadixBlock * ITEMS - 1) / (kRadixBlock * ITEMS);
+}
+
+// A block's tile: its histogram of one digit.  Entry `it` of a thread is index(it).
+template <int ITEMS>
+struct RadixTile {
+    int hist[kRadixWaves][256];
+
+    __device__ __forceinline__ static int index(int it) {
+        return (int)blockIdx.x * kRadixBlock * ITEMS + it * kRadixBlock + (int)threadIdx.x;
+    }
+    __device__ __forceinline__ void clear() {
 #pragma unroll
-    for (int it = 0; it < ITEMS; it++) {
-        const int i = base + it * kRadixBlock + (int)threadIdx.x;
-        if (i < n) atomicAdd(&hist[(keys[i] >> shift) & 255], 1);
+        for (int w = 0; w < kRadixWaves; w++) hist[w][threadIdx.x] = 0;
+        __syncthreads();
     }
-    __syncthreads();
-    counts[(size_t)threadIdx.x * n_tiles + blockIdx.x] = hist[threadIdx.x];
-}
-
-// Exclusive scan of m ints in place, in three coalesced launches: per-segment sums
-// (kRadixScanSeg ints per block), a one-block scan of the segment sums, then every segment
-// scanned again from its offset.
-constexpr int kRadixScanItems = 8;
-constexpr int kRadixScanSeg = kRadixBlock * kRadixScanItems;
-
-__device__ __forceinline__ int radix_block_sum(int v, int* ws) {
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = v;
-    __syncthreads();
-    int t = 0;
-    for (int w = 0; w < kRadixWaves; w++) t += ws[w];
-    __syncthreads();
-    return t;
-}
-
-__global__ __launch_bounds__(kRadixBlock) void k_radix_scan_sums(const int* v, int m, int* seg_sums) {
-    __shared__ int ws[kRadixWaves];
-    const int base = blockIdx.x * kRadixScanSeg;
-    int s = 0;
+    __device__ __forceinline__ void add(int digit) { atomicAdd(&hist[threadIdx.x >> 6][digit], 1); }
+    // The tile's counts to counts[digit][tile].
+    __device__ __forceinline__ void store(int* counts, int n_tiles) {
+        __syncthreads();
+        int c = 0;
 #pragma unroll
-    for (int it = 0; it < kRadixScanItems; it++) {
-        const int i = base + it * kRadixBlock + (int)threadIdx.x;
-        if (i < m) s += v[i];
+        for (int w = 0; w < kRadixWaves; w++) c += hist[w][threadIdx.x];
+        counts[(size_t)threadIdx.x * n_tiles + blockIdx.x] = c;
     }
-    s = radix_block_sum(s, ws);
-    if (threadIdx.x == 0) seg_sums[blockIdx.x] = s;
-}
-
-// Exclusive scan of the (few) segment sums, one block.
-__global__ __launch_bounds__(1024) void k_radix_scan_top(int* sums, int nseg) {
-    __shared__ int part[1024];
-    const int t = threadIdx.x;
-    const int per = (nseg + 1023) / 1024;
-    const int b0 = min(nseg, t * per), b1 = min(nseg, b0 + per);
-    int s = 0;
-    for (int b = b0; b < b1; b++) s += sums[b];
-    part[t] = s;
-    __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
-        const int x = t >= d ? part[t - d] : 0;
-        __syncthreads();
-        part[t] += x;
-        __syncthreads();
-    }
-    int run = part[t] - s;
-    for (int b = b0; b < b1; b++) {
-        const int c = sums[b];
-        sums[b] = run;
-        run += c;
-    }
-}
-
-__global__ __launch_bounds__(kRadixBlock) void k_radix_scan_apply(int* v, int m, const int* seg_offsets) {
-    __shared__ int wsum[kRadixWaves];
-    const int base = blockIdx.x * kRadixScanSeg;
-    int run = seg_offsets[blockIdx.x];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int it = 0; it < kRadixScanItems; it++) {
-        const int i = base + it * kRadixBlock + (int)threadIdx.x;
-        const int c = i < m ? v[i] : 0;
-        int x = c;  // inclusive wave scan
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
-        if (lane == 63) wsum[wave] = x;
-        __syncthreads();
-        int woff = 0, total = 0;
-        for (int w = 0; w < kRadixWaves; w++) {
-            woff += w < wave ? wsum[w] : 0;
-            total += wsum[w];
-        }
-        if (i < m) v[i] = run + woff + x - c;
-        run += total;
-        __syncthreads();
-    }
-}
+};
 
 template <int ITEMS>
+__global__ __launch_bounds__(kRadixBlock) void k_radix_hist(const int* __restrict__ keys, int n, int shift,
+                                                            int n_tiles, int* counts) {
+    __shared__ RadixTile<ITEMS> tile;
+    tile.clear();
+    int key[ITEMS];
+#pragma unroll
+    for (int it = 0; it < ITEMS; it++) key[it] = tile.index(it) < n ? keys[tile.index(it)] : 0;
+#pragma unroll
+    for (int it = 0; it < ITEMS; it++)
+        if (tile.index(it) < n) tile.add((key[it] >> shift) & 255);
+    tile.store(counts, n_tiles);
+}
+
+// Inclusive sum over the block's threads; `ws` holds an int per wave.
+__device__ __forceinline__ int radix_block_scan(int v, int* ws) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(v, o, 64);
+        if (lane >= o) v += y;
+    }
+    if (lane == 63) ws[wave] = v;
+    __syncthreads();
+    for (int w = 0; w < wave; w++) v += ws[w];
+    __syncthreads();
+    return v;
+}
+
+// Block d: exclusive scan of row d of the counts in place, its sum to totals[d].
+__global__ __launch_bounds__(kRadixBlock) void k_radix_rows(int* counts, int n_tiles, int* totals) {
+    __shared__ int ws[kRadixWaves];
+    __shared__ int last;
+    int* row = counts + (size_t)blockIdx.x * n_tiles;
+    int run = 0;
+    for (int base = 0; base < n_tiles; base += kRadixBlock) {
+        const int i = base + (int)threadIdx.x;
+        const int c = i < n_tiles ? row[i] : 0;
+        const int x = radix_block_scan(c, ws);
+        if (i < n_tiles) row[i] = run + x - c;
+        if (threadIdx.x == kRadixBlock - 1) last = x;
+        __syncthreads();
+        run += last;
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = run;
+}
+
+// FIRST: the values are the entries' indices (vals_in is not read).
+template <int ITEMS, bool FIRST>
 __global__ __launch_bounds__(kRadixBlock) void k_radix_scatter(const int* __restrict__ keys_in,
                                                                const int* __restrict__ vals_in, int n, int shift,
                                                                int n_tiles, const int* __restrict__ offsets,
-                                                               int* keys_out, int* vals_out) {
-    __shared__ int wave_count[kRadixWaves][256];
-    __shared__ int running[256];
-    const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+                                                               const int* __restrict__ totals, int* keys_out,
+                                                               int* vals_out) {
+    constexpr int kTile = kRadixBlock * ITEMS;
+    __shared__ int count[kRadixWaves][256];  // a wave's entries per digit, then the waves' before it
+    __shared__ int start[256];               // the digit's first place in the tile
+    __shared__ int move[256];                // what takes a place in the tile to one in the output
+    __shared__ int ws[kRadixWaves];
+    __shared__ int skey[kTile], sval[kTile];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const unsigned long long lt = lane ? (~0ull >> (64 - lane)) : 0ull;  // lanes below this one
-    running[threadIdx.x] = offsets[(size_t)threadIdx.x * n_tiles + blockIdx.x];
-    const int base = blockIdx.x * kRadixBlock * ITEMS;
+    const int base = blockIdx.x * kTile;
+    const int first = base + wave * 64 * ITEMS + lane;
+    int key[ITEMS], val[ITEMS], rank[ITEMS];
+#pragma unroll
     for (int it = 0; it < ITEMS; it++) {
-        for (int w = 0; w < kRadixWaves; w++) wave_count[w][threadIdx.x] = 0;
-        __syncthreads();
-        const int i = base + it * kRadixBlock + (int)threadIdx.x;
-        const bool valid = i < n;
-        const int key = valid ? keys_in[i] : 0;
-        const int val = valid ? vals_in[i] : 0;
-        const int digit = (key >> shift) & 255;
-        // lanes of this wave with the same digit
-        unsigned long long same = __ballot(valid);
+        const int i = first + it * 64;
+        key[it] = i < n ? keys_in[i] : 0;
+        val[it] = FIRST ? i : i < n ? vals_in[i] : 0;
+    }
+    const int digit_total = totals[t], tile_offset = offsets[(size_t)t * n_tiles + blockIdx.x];
+    for (int k = lane; k < 256; k += 64) count[wave][k] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int it = 0; it < ITEMS; it++) {
+        const bool valid = first + it * 64 < n;
+        const int digit = (key[it] >> shift) & 255;
+        unsigned long long same = __ballot(valid);  // lanes with the same digit
 #pragma unroll
         for (int b = 0; b < 8; b++) {
             const unsigned long long bits = __ballot((digit >> b) & 1);
             same &= ((digit >> b) & 1) ? bits : ~bits;
         }
-        const int rank = __popcll(same & lt);
-        if (valid && rank == 0) wave_count[wave][digit] = __popcll(same);
-        __syncthreads();
-        if (valid) {
-            int before = 0;
-            for (int w = 0; w < wave; w++) before += wave_count[w][digit];
-            const int pos = running[digit] + before + rank;
-            keys_out[pos] = key;
-            vals_out[pos] = val;
+        const int before = __popcll(same & lt);
+        rank[it] = count[wave][digit] + before;  // every lane reads before the first of them adds
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (valid && before == 0) count[wave][digit] = rank[it] + __popcll(same);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    int tile_total = 0;
+#pragma unroll
+    for (int w = 0; w < kRadixWaves; w++) {
+        const int c = count[w][t];
+        count[w][t] = tile_total;
+        tile_total += c;
+    }
+    const int tile_start = radix_block_scan(tile_total, ws) - tile_total;
+    const int digit_start = radix_block_scan(digit_total, ws) - digit_total;
+    start[t] = tile_start;
+    move[t] = digit_start + tile_offset - tile_start;
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < ITEMS; it++) {
+        if (first + it * 64 < n) {
+            const int digit = (key[it] >> shift) & 255;
+            const int at = start[digit] + count[wave][digit] + rank[it];
+            skey[at] = key[it];
+            sval[at] = val[it];
         }
-        __syncthreads();
-        int add = 0;
-        for (int w = 0; w < kRadixWaves; w++) add += wave_count[w][threadIdx.x];
-        running[threadIdx.x] += add;
-        __syncthreads();
+    }
+    __syncthreads();
+    const int left = min(kTile, n - base);
+#pragma unroll
+    for (int it = 0; it < ITEMS; it++) {
+        const int i = it * kRadixBlock + t;
+        if (i < left) {
+            const int k = skey[i];
+            const int to = move[(k >> shift) & 255] + i;
+            keys_out[to] = k;
+            vals_out[to] = sval[i];
+        }
     }
 }
 
-template <int ITEMS>
-inline int radix_tiles(int n) {
-    return (n + kRadixBlock * ITEMS - 1) / (kRadixBlock * ITEMS);
-}
-
-// Ints of the `counts` workspace radix_sort_pairs needs for n pairs: the digit counts, then
-// the scan's segment sums.
+// Ints of the `counts` workspace radix_sort needs for n entries: the tile counts, then the digits'
+// totals.
 template <int ITEMS>
 inline size_t radix_counts_size(int n) {
-    const size_t m = (size_t)256 * radix_tiles<ITEMS>(n);
-    return m + (m + kRadixScanSeg - 1) / kRadixScanSeg + 1;
+    return (size_t)256 * radix_tiles<ITEMS>(n) + 256;
 }
 
-// Sorts n pairs (keys in [0, 2^bits)) from (keys_a, vals_a) using (keys_b, vals_b) as the
-// other buffer; `counts` holds radix_counts_size<ITEMS>(n) ints.  The last pass writes the
-// values to vals_final (may be vals_b); *keys_sorted is set to the buffer holding the sorted
+// Sorts n keys (in [0, 2^bits)) from keys_a using keys_b as the other buffer; vals_a and vals_b
+// hold n ints each for the values of the passes between.  `counts` holds radix_counts_size<ITEMS>(n)
+// ints, the first 256 x tiles of them the tile counts of the lowest digit (RadixTile).  The last
+// pass writes the indices to vals_final; *keys_sorted is set to the buffer holding the sorted
 // keys.  Launch errors are left for the caller's hipGetLastError.
 template <int ITEMS>
-void radix_sort_pairs(int* keys_a, int* vals_a, int* keys_b, int* vals_b, int n, int bits, int* counts,
-                      int* vals_final, int** keys_sorted, hipStream_t s) {
+void radix_sort(int* keys_a, int* keys_b, int* vals_a, int* vals_b, int n, int bits, int* counts, int* vals_final,
+                int** keys_sorted, hipStream_t s) {
     const int passes = bits <= 8 ? 1 : (bits + 7) / 8;
     const int n_tiles = radix_tiles<ITEMS>(n);
-    const int m = 256 * n_tiles;
-    const int nseg = (m + kRadixScanSeg - 1) / kRadixScanSeg;
-    int* seg = counts + m;
+    int* totals = counts + (size_t)256 * n_tiles;
     for (int p = 0; p < passes; p++) {
         const int shift = 8 * p;
-        const bool last = p == passes - 1;
-        int* vo = last ? vals_final : vals_b;
-        hipLaunchKernelGGL(k_radix_hist<ITEMS>, dim3(n_tiles), dim3(kRadixBlock), 0, s, keys_a, n, shift, n_tiles,
-                           counts);
-        hipLaunchKernelGGL(k_radix_scan_sums, dim3(nseg), dim3(kRadixBlock), 0, s, counts, m, seg);
-        hipLaunchKernelGGL(k_radix_scan_top, dim3(1), dim3(1024), 0, s, seg, nseg);
-        hipLaunchKernelGGL(k_radix_scan_apply, dim3(nseg), dim3(kRadixBlock), 0, s, counts, m, seg);
-        hipLaunchKernelGGL(k_radix_scatter<ITEMS>, dim3(n_tiles), dim3(kRadixBlock), 0, s, keys_a, vals_a, n, shift,
-                           n_tiles, counts, keys_b, vo);
+        int* vo = p == passes - 1 ? vals_final : vals_b;
+        if (p > 0)
+            hipLaunchKernelGGL(k_radix_hist<ITEMS>, dim3(n_tiles), dim3(kRadixBlock), 0, s, keys_a, n, shift, n_tiles,
+                               counts);
+        hipLaunchKernelGGL(k_radix_rows, dim3(256), dim3(kRadixBlock), 0, s, counts, n_tiles, totals);
+        if (p == 0)
+            hipLaunchKernelGGL((k_radix_scatter<ITEMS, true>), dim3(n_tiles), dim3(kRadixBlock), 0, s, keys_a,
+                               (const int*)nullptr, n, shift, n_tiles, counts, totals, keys_b, vo);
+        else
+            hipLaunchKernelGGL((k_radix_scatter<ITEMS, false>), dim3(n_tiles), dim3(kRadixBlock), 0, s, keys_a, vals_a,
+                               n, shift, n_tiles, counts, totals, keys_b, vo);
         std::swap(keys_a, keys_b);
         std::swap(vals_a, vals_b);
     }

@@ -9,9 +9,9 @@
 // valid material (a miss, a triangle id or material out of range) get key num_mats and end up
 // after all materials.
 //
-// The sort is radix_sort_pairs (radix.h) with tiles of 1024 entries.
-// Traffic per entry and pass: key and index read twice, written once (16 B), plus the hit
-// (16 B), the index record (4 B) and the ray's dir.w (4 B) once for the keys.
+// The sort is radix_sort (radix.h) with tiles of 2048 entries; the key kernel leaves the first
+// pass's tile counts.  Traffic per entry: 20 B per pass, plus the hit (16 B), the index record (4 B)
+// and the ray's dir.w (4 B) once for the keys.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,20 +23,31 @@ namespace imba {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kItems = 4;
+constexpr int kItems = 8;
+
+static_assert(kBlock == kRadixBlock, "the key kernel's tiles are the sort's");
 
 __global__ __launch_bounds__(kBlock) void k_mat_keys(const int4* __restrict__ hits, const int* __restrict__ indices,
                                                      int n_tris, float4* rays, int count, int num_mats, int* keys,
-                                                     int* vals) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= count) return;
-    const int tri = hits[i].x;
-    int mat = -1;
-    if (tri >= 0 && tri < n_tris) mat = indices[4 * (size_t)tri + 3];
-    const int key = (mat >= 0 && mat < num_mats) ? mat : num_mats;
-    reinterpret_cast<float*>(rays)[8 * (size_t)i + 7] = __int_as_float(key);  // ray.dir.w
-    keys[i] = key;
-    vals[i] = i;
+                                                     int n_tiles, int* counts) {
+    __shared__ RadixTile<kItems> tile;
+    tile.clear();
+    int tri[kItems], mat[kItems];
+#pragma unroll
+    for (int it = 0; it < kItems; it++) tri[it] = tile.index(it) < count ? hits[tile.index(it)].x : -1;
+#pragma unroll
+    for (int it = 0; it < kItems; it++) mat[it] = tri[it] >= 0 && tri[it] < n_tris ? indices[4 * (size_t)tri[it] + 3] : -1;
+#pragma unroll
+    for (int it = 0; it < kItems; it++) {
+        const int i = tile.index(it);
+        if (i < count) {
+            const int key = (mat[it] >= 0 && mat[it] < num_mats) ? mat[it] : num_mats;
+            reinterpret_cast<float*>(rays)[8 * (size_t)i + 7] = __int_as_float(key);  // ray.dir.w
+            keys[i] = key;
+            tile.add(key & 255);
+        }
+    }
+    tile.store(counts, n_tiles);
 }
 
 // bucket_start[k] = first position whose key is >= k, for k = 0..num_mats.
@@ -92,9 +103,10 @@ int imba_sort_by_material(const int* indices, int tri_count, ImbaRay* rays, cons
     int* vals_a = keys_b + count;
     int* vals_b = vals_a + count;
     int* counts = vals_b + count;
-    hipLaunchKernelGGL(k_mat_keys, dim3(ceil_div(count, kBlock)), dim3(kBlock), 0, s, (const int4*)hits, indices,
-                       tri_count, (float4*)rays, count, num_mats, keys_a, vals_a);
-    radix_sort_pairs<kItems>(keys_a, vals_a, keys_b, vals_b, count, bits, counts, sorted, &keys_a, s);
+    const int n_tiles = radix_tiles<kItems>(count);
+    hipLaunchKernelGGL(k_mat_keys, dim3(n_tiles), dim3(kBlock), 0, s, (const int4*)hits, indices, tri_count,
+                       (float4*)rays, count, num_mats, keys_a, n_tiles, counts);
+    radix_sort<kItems>(keys_a, keys_b, vals_a, vals_b, count, bits, counts, sorted, &keys_a, s);
     if (bucket_start)
         hipLaunchKernelGGL(k_bucket_starts, dim3(ceil_div(num_mats + 1, 256)), dim3(256), 0, s, keys_a, count,
                            num_mats, bucket_start);

@@ -163,3 +163,11 @@ def test_tile_and_offset_rules(gpu, n):
                 "compact_rays_dev")
         assert cnt.download(np.int32, 2)[1] == (states[:min(count, cap), 0] >= 0).sum()
         assert (ws.download(np.uint8, size + 64)[size:] == 0x77).all()
+
+
+@pytest.mark.parametrize("count", [63, 2047, 2048, 2049, 256 * 2048 + 1])
+@pytest.mark.parametrize("num_mats", [1, 255, 65536])
+def test_sort_tile_and_digit_edges(gpu, count, num_mats):
+    """The sort at the edges of its tiles (2048 entries), of the scan over tiles (256 of them) and of
+    its digits (keys up to 1, 255 and 65536: one, one and three passes)."""
+    test_sort_by_material_matches_oracle(gpu, count, num_mats)

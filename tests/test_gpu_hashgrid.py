@@ -202,3 +202,20 @@ def test_query_ties_and_edges(gpu, k):
         assert np.array_equal(c2, cnt[:n])
         for q in range(n):
             assert np.array_equal(i2[q, :c2[q]], idx[q, :c2[q]])
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 127, 1023, 1024, 1025, 4095, 4096, 4097, 33000])
+@pytest.mark.parametrize("spread", [0.0, 0.02, 1.0])
+def test_build_tile_edges(gpu, n, spread):
+    """The build at the edges of its waves (64 slots), blocks and sort tiles (4096), with all photons
+    in one bucket, in a few crowded ones, and spread over the table; 33000 photons in one bucket
+    make its run of slots longer than any block's share."""
+    photons = np.zeros((n, 4), np.float32)
+    photons[:, :3] = 0.5 + spread * np.random.default_rng(n).random((n, 3), dtype=np.float32)
+    radius = 0.01 if spread else 1.0
+    g, _ = _grid(photons, radius)
+    og = oracle.Grid()
+    og.build(photons[:, :3], radius)
+    _check_build(g, og, n)
+    queries = photons[:: max(1, n // 8), :3] + np.float32(0.3 * radius)
+    _check_queries(g, og, np.ascontiguousarray(queries), 10)
