@@ -2,19 +2,18 @@
 //
 // HashGrid (rangesearch/rangesearch.h:21-158) builds on the host with TBB: bounds reduce,
 // atomic count per bucket, serial exclusive scan, atomic scatter.  Here:
-//   bounds   k_bounds (per-block min/max; it also clears the bucket ends)
+//   bounds   k_bounds: per-block min/max
 //   keys     k_grid_keys combines the bounds (grown by 0.1%, derived values) and writes the
 //            bucket of each photon and the sort's first tile counts
 //   sort     stable LSD radix sort of the photon indices by bucket (radix.h): the slot order is by
 //            bucket, then by photon index, which is deterministic and equals a serial run of
 //            the reference's scatter
-//   slots    k_slots: positions copied to slot order as float4 (x, y, z, index bits), slot + 1 at
-//            the last slot of each bucket into its end
-//   boxes    k_bucket_box: bounds of each bucket's photons
-//   ends     k_ends carries the ends over the empty buckets (an inclusive max-scan; what comes
-//            before a tile of buckets is found by searching the sorted keys)
-// 4M photons, 8M buckets: 444 us in 26 launches before the sort was rewritten and the smaller
-// launches were merged, now 331 in 13.
+//   slots    k_slots: positions copied to slot order as float4 (x, y, z, index bits), and the
+//            bounds of the buckets' photons among each 64 slots
+//   ends     k_ends: each bucket's end from the sorted keys, an inclusive max-scan carrying it
+//            over the empty buckets; it also joins the bounds of buckets that go on past 64 slots
+// 4M photons, 8M buckets: 446 us in 26 launches before the sort was rewritten and the smaller
+// launches were merged, now 291 in 12.
 // The query visits the same 8 buckets in the same order as the reference (duplicates
 // included), one query per wave, and keeps the k-capped, distance-sorted list in lanes 0..k-1
 // with the reference's insertion rule.  Squared distances are computed without fused
@@ -68,10 +67,8 @@ __device__ __forceinline__ void block_bounds(float* lo, float* hi) {
         }
 }
 
-// Bounds of the photons, one box per block, and the bucket ends cleared (a kernel's stores rather
-// than a memset node, so the build can be captured in a graph).
-__global__ __launch_bounds__(kBlock) void k_bounds(const unsigned char* ph, int stride, int off, int n, float* partial,
-                                                   int* ends, int table) {
+// Bounds of the photons, one box per block.
+__global__ __launch_bounds__(kBlock) void k_bounds(const unsigned char* ph, int stride, int off, int n, float* partial) {
     float lo[3] = {FLT_MAX, FLT_MAX, FLT_MAX}, hi[3] = {-FLT_MAX, -FLT_MAX, -FLT_MAX};
     const int step = gridDim.x * kBlock;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += step) {
@@ -83,7 +80,6 @@ __global__ __launch_bounds__(kBlock) void k_bounds(const unsigned char* ph, int 
             hi[k] = pick_max(hi[k], v);
         }
     }
-    for (int i = blockIdx.x * kBlock + threadIdx.x; i < table; i += step) ends[i] = 0;
     block_bounds(lo, hi);
     if (threadIdx.x < 6) partial[6 * blockIdx.x + threadIdx.x] = threadIdx.x < 3 ? lo[threadIdx.x] : hi[threadIdx.x - 3];
 }
@@ -138,37 +134,6 @@ __global__ __launch_bounds__(kBlock) void k_grid_keys(const unsigned char* ph, i
     tile.store(counts, n_tiles);
 }
 
-// Slot order: the photons' positions (four scattered reads of a thread in flight together), and at
-// a bucket's first slot its box cleared, at its last slot its end (the empty buckets' ends were
-// cleared before).
-constexpr int kSlotItems = 4;
-__global__ __launch_bounds__(kBlock) void k_slots(const unsigned char* ph, int stride, int off, int n, const int* order,
-                                                  const int* keys_sorted, float4* pos4, int* ends, uint32_t* box) {
-    const int base = blockIdx.x * kBlock * kSlotItems + (int)threadIdx.x;
-    float p[kSlotItems][3];
-    int idx[kSlotItems];
-#pragma unroll
-    for (int it = 0; it < kSlotItems; it++) idx[it] = order[min(base + it * kBlock, n - 1)];
-#pragma unroll
-    for (int it = 0; it < kSlotItems; it++) {
-        const float* q = photon_pos(ph, stride, off, idx[it]);
-        for (int k = 0; k < 3; k++) p[it][k] = q[k];
-    }
-#pragma unroll
-    for (int it = 0; it < kSlotItems; it++) {
-        const int s = base + it * kBlock;
-        if (s >= n) break;
-        pos4[s] = make_float4(p[it][0], p[it][1], p[it][2], __int_as_float(idx[it]));
-        const int b = keys_sorted[s];
-        if (s == n - 1 || keys_sorted[s + 1] != b) ends[b] = s + 1;
-        if (s == 0 || keys_sorted[s - 1] != b) {
-            uint32_t* e = box + 6 * (size_t)b;
-            e[0] = e[1] = e[2] = 0xFFFFFFFFu;  // min over nothing
-            e[3] = e[4] = e[5] = 0u;           // max over nothing
-        }
-    }
-}
-
 // One step of a scan over the wave's runs of equal keys: the bounds of the lane that the DPP control
 // names (in the rows of the mask) join this lane's if its key is the same.
 template <int CTRL, int ROWS>
@@ -183,35 +148,57 @@ __device__ __forceinline__ void join_bounds(int key, uint32_t* lo, uint32_t* hi)
     }
 }
 
-// Bounds of every non-empty bucket's photons (the queries skip buckets that lie beyond their
-// limit; an empty bucket's entry is never used), in the order-preserving integer form of
-// grid_query.h so that atomic min / max can combine them.  Every wave takes 64 consecutive slots
-// and reduces the runs of equal keys with DPP row shifts and broadcasts (the keys are sorted, so
-// equal keys are contiguous; with shuffles through LDS this took 39 us for 4M photons); the last lane
-// of each run combines the run's bounds into the bucket's entry with six atomics.  Hot buckets
-// thus cost one atomic per 64 photons.
-__global__ __launch_bounds__(kBlock) void k_bucket_box(const int* keys_sorted, int n, const float4* pos4, uint32_t* box) {
-    const int s = blockIdx.x * kBlock + threadIdx.x;
+// Slot order: the photons' positions, and the bounds of every non-empty bucket's photons (the
+// queries skip buckets that lie beyond their limit; an empty bucket's entry is never used), in the
+// order-preserving integer form of grid_query.h.  A wave takes 64 consecutive slots at a time and
+// reduces the runs of equal keys (the keys are sorted, so equal keys are contiguous) with DPP row
+// shifts and broadcasts; a run's last lane stores its bounds.  A run that began before these slots
+// leaves them in heads[slot / 64] instead, for k_ends to join.  Bound by the scattered reads of the
+// positions (a cache line each; a thread's four are in flight together): 4M photons 91 us.  With
+// the boxes cleared here and joined by atomics in a launch of their own it took 92 + 39.
+constexpr int kSlotItems = 4;
+__global__ __launch_bounds__(kBlock) void k_slots(const unsigned char* ph, int stride, int off, int n, const int* order,
+                                                  const int* keys_sorted, float4* pos4, uint32_t* box, uint32_t* heads) {
+    const int base = blockIdx.x * kBlock * kSlotItems + (int)threadIdx.x;
     const int lane = threadIdx.x & 63;
-    const bool valid = s < n;
-    const int key = valid ? keys_sorted[s] : -1;
-    const float4 p = pos4[min(s, n - 1)];
-    uint32_t lo[3], hi[3];
-    lo[0] = hi[0] = ordered_bits(p.x);
-    lo[1] = hi[1] = ordered_bits(p.y);
-    lo[2] = hi[2] = ordered_bits(p.z);
-    join_bounds<0x111, 0xF>(key, lo, hi);  // row_shr:1, 2, 4, 8: the 16 lanes of a row
-    join_bounds<0x112, 0xF>(key, lo, hi);
-    join_bounds<0x114, 0xF>(key, lo, hi);
-    join_bounds<0x118, 0xF>(key, lo, hi);
-    join_bounds<0x142, 0xA>(key, lo, hi);  // row_bcast:15: the last lane of rows 0, 2 to rows 1, 3
-    join_bounds<0x143, 0xC>(key, lo, hi);  // row_bcast:31: lane 31 to rows 2 and 3
-    const int next = __shfl_down(key, 1, 64);
-    if (!valid || (lane < 63 && next == key)) return;  // not the last lane of its run
-    uint32_t* e = box + 6 * (size_t)key;
-    for (int a = 0; a < 3; a++) {
-        atomicMin(e + a, lo[a]);
-        atomicMax(e + 3 + a, hi[a]);
+    float p[kSlotItems][3];
+    int idx[kSlotItems], keys[kSlotItems], before[kSlotItems];
+#pragma unroll
+    for (int it = 0; it < kSlotItems; it++) {
+        const int s = base + it * kBlock;
+        idx[it] = order[min(s, n - 1)];
+        keys[it] = s < n ? keys_sorted[s] : -1;
+        before[it] = s - lane > 0 && s - lane < n ? keys_sorted[s - lane - 1] : -1;  // key before the wave's slots
+    }
+#pragma unroll
+    for (int it = 0; it < kSlotItems; it++) {
+        const float* q = photon_pos(ph, stride, off, idx[it]);
+        for (int k = 0; k < 3; k++) p[it][k] = q[k];
+    }
+#pragma unroll
+    for (int it = 0; it < kSlotItems; it++) {
+        const int s = base + it * kBlock;
+        const int key = keys[it];
+        uint32_t lo[3], hi[3];
+#pragma unroll
+        for (int a = 0; a < 3; a++) lo[a] = hi[a] = ordered_bits(p[it][a]);
+        join_bounds<0x111, 0xF>(key, lo, hi);  // row_shr:1, 2, 4, 8: the 16 lanes of a row
+        join_bounds<0x112, 0xF>(key, lo, hi);
+        join_bounds<0x114, 0xF>(key, lo, hi);
+        join_bounds<0x118, 0xF>(key, lo, hi);
+        join_bounds<0x142, 0xA>(key, lo, hi);  // row_bcast:15: the last lane of rows 0, 2 to rows 1, 3
+        join_bounds<0x143, 0xC>(key, lo, hi);  // row_bcast:31: lane 31 to rows 2 and 3
+        const int next = __shfl_down(key, 1, 64);
+        if (s < n) {
+            pos4[s] = make_float4(p[it][0], p[it][1], p[it][2], __int_as_float(idx[it]));
+            if (lane == 63 || next != key) {  // the run's last lane (-1 is no key)
+                uint2* e = reinterpret_cast<uint2*>(before[it] == key ? heads + 6 * (size_t)(s >> 6)
+                                                                      : box + 6 * (size_t)key);
+                e[0] = make_uint2(lo[0], lo[1]);
+                e[1] = make_uint2(lo[2], hi[0]);
+                e[2] = make_uint2(hi[1], hi[2]);
+            }
+        }
     }
 }
 
@@ -233,29 +220,85 @@ __device__ __forceinline__ int slots_before(const int* keys_sorted, int n, int b
     return lo;
 }
 
-// Inclusive max-scan of the bucket ends in place, a tile of buckets per block.
-__global__ __launch_bounds__(kBlock) void k_ends(int* v, int table, const int* keys_sorted, int n) {
-    __shared__ int wmax[kBlock / 64];
+// The buckets' ends, 2048 buckets per block: the block finds its slots in the sorted keys, marks slot +
+// 1 at the last slot of each bucket in LDS, and an inclusive max-scan from the slots before carries it
+// over the empty buckets.  Where the block's buckets hold many slots each bucket's end is searched
+// instead, so that a crowded bucket costs the steps of a search and not a walk (the line lies at 64 slots
+// a thread, well above the 1/2 a bucket that the table's size gives).  4M photons, 8M buckets: 34 us;
+// with the ends cleared and marked in memory by the launches before, the scan took 28 and the launch
+// that cleared them 5 more.
+constexpr int kManySlots = 8 * kScanTile;
+__global__ __launch_bounds__(kBlock) void k_ends(int* ends, int table, const int* keys_sorted, int n,
+                                                 const uint32_t* heads, uint32_t* box) {
+    __shared__ int range[kBlock / 64];
+    __shared__ __attribute__((aligned(16))) int mark[kScanTile];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int base = blockIdx.x * kScanTile;
-    int run = slots_before(keys_sorted, n, base);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int it = 0; it < kScanItems; it++) {
-        const int i = base + it * kBlock + threadIdx.x;
-        int x = i < table ? v[i] : 0;
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(x, o, 64);
-            if (lane >= o) x = max(x, y);
+    // The runs that go on past 64 slots (table >= 2 n, so the grid has n / 64 threads).
+    const long long begin = 64ll * ((int)blockIdx.x * kBlock + t);
+    if (begin > 0 && begin < n) {
+        const int key = keys_sorted[begin];
+        if (keys_sorted[begin - 1] == key) {
+            const uint32_t* h = heads + 6 * (begin >> 6);
+            uint32_t* e = box + 6 * (size_t)key;
+            for (int a = 0; a < 3; a++) {
+                atomicMin(e + a, h[a]);
+                atomicMax(e + 3 + a, h[3 + a]);
+            }
         }
-        if (lane == 63) wmax[wave] = x;
-        __syncthreads();
-        int wm = 0, total = 0;
-        for (int w = 0; w < kBlock / 64; w++) {
-            if (w < wave) wm = max(wm, wmax[w]);
-            total = max(total, wmax[w]);
+    }
+    if (wave < 2) {
+        const int r = slots_before(keys_sorted, n, wave == 0 ? base : min(table, base + kScanTile));
+        if (lane == 0) range[wave] = r;
+    }
+    int4* mark4 = reinterpret_cast<int4*>(mark);
+    for (int i = t; i < kScanTile / 4; i += kBlock) mark4[i] = make_int4(0, 0, 0, 0);
+    __syncthreads();
+    const int lo = range[0], hi = range[1];
+    __syncthreads();
+    int x[kScanItems];
+    if (hi - lo <= kManySlots) {
+        for (int s = lo + t; s < hi; s += kBlock) {
+            const int key = keys_sorted[s];
+            if (s == n - 1 || keys_sorted[s + 1] != key) mark[key - base] = s + 1;
         }
-        if (i < table) v[i] = max(run, max(wm, x));
-        run = max(run, total);
         __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kScanItems; k += 4) {
+            const int4 m = mark4[(t * kScanItems + k) / 4];
+            x[k] = m.x, x[k + 1] = m.y, x[k + 2] = m.z, x[k + 3] = m.w;
+        }
+    } else {  // the first slot after the bucket, by halving, the thread's buckets side by side
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++) x[k] = lo;
+        for (int step = 1 << (31 - __clz(hi - lo)); step > 0; step >>= 1)
+#pragma unroll
+            for (int k = 0; k < kScanItems; k++)
+                if (x[k] + step <= hi && keys_sorted[x[k] + step - 1] <= base + t * kScanItems + k) x[k] += step;
+    }
+#pragma unroll
+    for (int k = 1; k < kScanItems; k++) x[k] = max(x[k], x[k - 1]);
+    int run = x[kScanItems - 1];
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(run, o, 64);
+        if (lane >= o) run = max(run, y);
+    }
+    if (lane == 63) range[wave] = run;
+    const int up = __shfl_up(run, 1, 64);
+    run = max(lo, lane > 0 ? up : 0);
+    __syncthreads();
+    for (int w = 0; w < wave; w++) run = max(run, range[w]);
+    const int first = base + t * kScanItems;
+#pragma unroll
+    for (int k = 0; k < kScanItems; k++) x[k] = max(x[k], run);
+    if (first + kScanItems <= table) {
+#pragma unroll
+        for (int k = 0; k < kScanItems; k += 4)
+            *reinterpret_cast<int4*>(ends + first + k) = make_int4(x[k], x[k + 1], x[k + 2], x[k + 3]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < kScanItems; k++)
+            if (first + k < table) ends[first + k] = x[k];
     }
 }
 
@@ -489,25 +532,26 @@ int imba_hashgrid_build(ImbaHashGrid* g, const void* photons, int stride, int po
     }
     g->count = count;
     const unsigned char* ph = (const unsigned char*)photons;
-    const int nparts = std::min(kBoundsBlocks, std::max(1, ceil_div(std::max(count, table / 8), kBlock)));
+    const int nparts = std::min(kBoundsBlocks, std::max(1, ceil_div(count, kBlock)));
     const int n_tiles = radix_tiles<kSortItems>(count);
-    hipLaunchKernelGGL(k_bounds, dim3(nparts), dim3(kBlock), 0, s, ph, stride, pos_offset, count, g->partial,
-                       g->cell_ends, table);
+    hipLaunchKernelGGL(k_bounds, dim3(nparts), dim3(kBlock), 0, s, ph, stride, pos_offset, count, g->partial);
     hipLaunchKernelGGL(k_grid_keys, dim3(std::max(1, n_tiles)), dim3(kBlock), 0, s, ph, stride, pos_offset, count,
                        g->partial, nparts, g->d_params, radius, table, g->keys_a, n_tiles, g->digits);
+    int* keys_sorted = nullptr;
+    uint32_t* heads = nullptr;
     if (count > 0) {
         int bits = 1;
         while (bits < 31 && (1 << bits) < table) bits++;  // buckets are < table
-        int* keys_sorted = nullptr;
         radix_sort<kSortItems>(g->keys_a, g->keys_b, g->vals_a, g->vals_b, count, bits, g->digits, g->order,
                                &keys_sorted, s);
+        // The sort's other key buffer: 6 words per 64 slots after the first 64.
+        heads = (uint32_t*)(keys_sorted == g->keys_a ? g->keys_b : g->keys_a);
         hipLaunchKernelGGL(k_slots, dim3(ceil_div(count, kBlock * kSlotItems)), dim3(kBlock), 0, s, ph, stride,
-                           pos_offset, count, g->order, keys_sorted, g->pos4, g->cell_ends, g->bucket_box);
-        hipLaunchKernelGGL(k_bucket_box, dim3(ceil_div(count, kBlock)), dim3(kBlock), 0, s, keys_sorted, count, g->pos4,
-                           g->bucket_box);
-        hipLaunchKernelGGL(k_ends, dim3(ceil_div(table, kScanTile)), dim3(kBlock), 0, s, g->cell_ends, table,
-                           keys_sorted, count);
+                           pos_offset, count, g->order, keys_sorted, g->pos4, g->bucket_box, heads);
     }
+    if (table > 0)
+        hipLaunchKernelGGL(k_ends, dim3(ceil_div(table, kScanTile)), dim3(kBlock), 0, s, g->cell_ends, table,
+                           keys_sorted, count, heads, g->bucket_box);
     IMBA_HIP_TRY(hipGetLastError());
     if (sync) IMBA_HIP_TRY(hipStreamSynchronize(s));
     return IMBA_OK;
