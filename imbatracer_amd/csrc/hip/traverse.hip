@@ -399,11 +399,17 @@ struct ImbaTraceBatch {
 namespace imba {
 namespace {
 
+int grow_spill(ImbaTraceBatch* b, int g, size_t bytes, hipStream_t s) {
+    if (b->spill[g].bytes >= bytes) return IMBA_OK;
+    const int r = not_capturing(s, "a larger spill stack");
+    return r ? r : grow_buffer(b->spill[g], bytes);
+}
+
 // One launch of group g: chunks of 64 rays with one lane each, or (QUADS) quarters of chunks with
-// four lanes per ray; `limit` as in k_trace_batch.  With `reserve` only the spill stack the launch
-// would need is allocated (for a later launch that is recorded into a graph).
+// four lanes per ray; `limit` as in k_trace_batch.  With `need` nothing is launched: *need is raised
+// to the bytes of the spill stack the launch would use.
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE, bool QUADS>
-int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, bool reserve, hipStream_t s) {
+int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, size_t* need, hipStream_t s) {
     const DeviceProps* p = device_props();
     auto kern = k_trace_batch<BLOCK, STACK_LDS, ANY, MASKED, TREE, QUADS>;
     const int max_stack = b->max_stack[TREE ? 1 : 0][g];
@@ -419,16 +425,16 @@ int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, 
     int spill_depth = 0;
     if (!QUADS && max_stack > STACK_LDS) {
         spill_depth = max_stack - STACK_LDS;
-        const size_t need = (size_t)spill_depth * grid * BLOCK * sizeof(int);
-        if (b->spill[g].bytes < need) {
-            int r = not_capturing(s, "a larger spill stack");
-            if (r) return r;
-            r = grow_buffer(b->spill[g], need);
+        const size_t bytes = (size_t)spill_depth * grid * BLOCK * sizeof(int);
+        if (need) {
+            *need = std::max(*need, bytes);
+        } else {
+            const int r = grow_spill(b, g, bytes, s);
             if (r) return r;
         }
         spill = (int*)b->spill[g].ptr;
     }
-    if (reserve) return IMBA_OK;
+    if (need) return IMBA_OK;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), 0, s, b->d_items[TREE], b->groups.first[g],
                        b->groups.first[g + 1] - b->groups.first[g], b->d_group_chunks + g, b->d_counters + 2 * g,
                        spill, spill_depth, limit);
@@ -437,31 +443,33 @@ int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, 
 }
 
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE>
-int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, bool reserve, hipStream_t s) {
+int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, bool open, size_t* need, hipStream_t s) {
     const DeviceProps* p = device_props();
     if (!p) return fail(IMBA_ERR_NO_DEVICE, "no HIP device");
     if constexpr (TREE == 2) {
         const int limit = blocks_per_cu <= 0 ? quad_rays(p, b->max_stack[1][g], STACK_LDS) / 64 : 0;
-        if (limit > 0 && !reserve) {
-            // a graph replays its launches with whatever sizes a later update brings
-            const bool small = b->capacity_chunks[g] <= limit && !b->captured;
-            if (small || b->device_counts[g] || b->captured) {
-                const int r = launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, true>(b, g, 0, limit, false, s);
-                if (r) return r;
-                return launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, 0, limit, small, s);
-            }
+        // a graph replays its launches with whatever sizes a later update brings
+        const bool small = b->capacity_chunks[g] <= limit && !b->captured;
+        if (limit > 0 && (small || b->device_counts[g] || b->captured)) {
+            int r = need ? IMBA_OK
+                         : launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, true>(b, g, 0, limit, nullptr, s);
+            if (r || (small && open)) return r;  // (recorded, the open choice takes the BVH2)
+            size_t later = 0;  // small: what a later launch that is recorded needs
+            r = launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, 0, limit, small ? &later : need, s);
+            return r ? r : grow_spill(b, g, later, s);
         }
     }
-    return launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, blocks_per_cu, -1, reserve, s);
+    return launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, blocks_per_cu, -1, need, s);
 }
 
 template <bool ANY, bool MASKED, int TREE>
-int dispatch_batch(ImbaTraceBatch* b, int g, const ImbaTraceConfig* cfg, hipStream_t s, bool reserve = false) {
+int dispatch_batch(ImbaTraceBatch* b, int g, const ImbaTraceConfig* cfg, hipStream_t s, bool open = false,
+                   size_t* need = nullptr) {
     const int block = cfg && cfg->block_size ? cfg->block_size : kDefaultBlock;
     const int stack = cfg && cfg->stack_lds ? cfg->stack_lds : kDefaultStack;
     const int bpc = cfg ? cfg->blocks_per_cu : 0;
 #define IMBA_SHAPE(B, S) \
-    if (block == B && stack == S) return launch_batch_group<B, S, ANY, MASKED, TREE>(b, g, bpc, reserve, s);
+    if (block == B && stack == S) return launch_batch_group<B, S, ANY, MASKED, TREE>(b, g, bpc, open, need, s);
     IMBA_SHAPE(256, 16)
     IMBA_SHAPE(256, 8)
     IMBA_SHAPE(256, 32)
@@ -670,9 +678,14 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
     const bool other = closest == 2 && tree_code(cfg, 0) == 0;
     for (int g = 0; g < 4; g++) {
         if (b->groups.first[g + 1] == b->groups.first[g] || b->capacity_chunks[g] == 0) continue;
-        if (other && g < 2) {
-            r = g == 0 ? dispatch_batch<false, false, 0>(b, g, cfg, s, true)
-                       : dispatch_batch<false, true, 0>(b, g, cfg, s, true);
+        if (other && g < 2) {  // both trees' spill stacks at once: growing later would wait and free
+            size_t need = 0;
+            r = g == 0 ? dispatch_batch<false, false, 0>(b, g, cfg, s, true, &need)
+                       : dispatch_batch<false, true, 0>(b, g, cfg, s, true, &need);
+            if (!r)
+                r = g == 0 ? dispatch_batch<false, false, 2>(b, g, cfg, s, true, &need)
+                           : dispatch_batch<false, true, 2>(b, g, cfg, s, true, &need);
+            if (!r) r = grow_spill(b, g, need, s);
             if (r) return r;
         }
         switch (g + 4 * (g >= 2 ? any : closest)) {
@@ -684,8 +697,8 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
             case 5: r = dispatch_batch<false, true, 1>(b, g, cfg, s); break;
             case 6: r = dispatch_batch<true, false, 1>(b, g, cfg, s); break;
             case 7: r = dispatch_batch<true, true, 1>(b, g, cfg, s); break;
-            case 8: r = dispatch_batch<false, false, 2>(b, g, cfg, s); break;
-            case 9: r = dispatch_batch<false, true, 2>(b, g, cfg, s); break;
+            case 8: r = dispatch_batch<false, false, 2>(b, g, cfg, s, other); break;
+            case 9: r = dispatch_batch<false, true, 2>(b, g, cfg, s, other); break;
             case 10: r = dispatch_batch<true, false, 2>(b, g, cfg, s); break;
             default: r = dispatch_batch<true, true, 2>(b, g, cfg, s); break;
         }
