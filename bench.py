@@ -91,7 +91,7 @@ def cfg_dict(cfg):
     if cfg is None:
         return "default"
     return {"block": cfg.block_size or 256, "stack_lds": cfg.stack_lds or 16, "persistent": cfg.persistent,
-            "bvh_width": cfg.bvh_width or 2, "quantized": cfg.quantized, "treelet": cfg.treelet}
+            "bvh_width": cfg.bvh_width, "quantized": cfg.quantized, "treelet": cfg.treelet}
 
 
 BVH2_CFG_ARGS = (256, 16, 0, 0, 2, 0, 0)  # TraceConfig of the reference's binary tree
@@ -120,7 +120,8 @@ BYTES_RULE = ("per ray 32 (ray) + 16 (hit) + 64 x inner nodes of the reference's
 
 
 def node_bytes_of(cfg):
-    """Bytes of one node of the tree a configuration walks: BVH2 64, 4-wide 128, quantized 64."""
+    """Bytes of one node of the tree a configuration walks: BVH2 64, 4-wide 128, quantized 64 (a
+    configuration of None leaves the tree open, so 64 in either case)."""
     return 128 if cfg is not None and cfg.bvh_width == 4 and not cfg.quantized else 64
 
 
@@ -209,15 +210,14 @@ def shadow_tune(pt, frames=3):
 def frame_tune(pt, queues, frames=3):
     """Per-scene launch configuration for whole frames: the library's autotuner on queues of
     three sizes (a frame's queues shrink from bounce to bounce), each distinct winner and a few
-    plain quantized launches (with and without a 64-node treelet, persistent or not) timed over
-    whole frames (the traversal kernels' times per bounce).  The frame's tree is the one of the
-    fastest candidate; each bounce then takes the fastest candidate on that tree for its own
+    plain quantized launches (persistent or not) timed over whole frames (the traversal kernels'
+    times per bounce).  The frame's tree is the one of the fastest candidate; each bounce then takes the fastest candidate on that tree for its own
     queue, so every bounce walks the same tree (same visits, same algorithmic bytes)."""
     from imbatracer_amd import native as N
 
     cands = [autotune(pt.gpu_scene, queues[b]) for b in sorted({1, len(queues) // 2, len(queues) - 2})
              if 0 < b < len(queues) and len(queues[b])]
-    cands += [N.TraceConfig(256, 16, 0, 0, 4, 1, 0), N.TraceConfig(256, 16, 0, 0, 4, 1, 64),
+    cands += [N.TraceConfig(256, 16, 0, 0, 4, 1, 0),
               N.TraceConfig(128, 16, 0, 0, 4, 1, 0), N.TraceConfig(64, 32, 0, 0, 4, 1, 0),
               N.TraceConfig(256, 16, 32, 0, 4, 1, 0), N.TraceConfig(256, 16, 8, 0, 4, 1, 0)]
     seen, timed = set(), []
@@ -690,12 +690,11 @@ def run_c4(args):
     batch = S.TraceBatch([q[:6] for q in queues])
     st = N.Stream()
     if cfg is None and not args.no_autotune:
-        # the batched launch over every queue, timed for each tree (quantized also with a 64-node
-        # LDS treelet per wave) and a few shapes
+        # the batched launch over every queue, timed for each tree and a few shapes
         best, tried = None, []
-        for width, quant, tl in ((2, 0, 0), (4, 0, 0), (4, 1, 0), (4, 1, 64)):
+        for width, quant in ((2, 0), (4, 0), (4, 1)):
             for block, stack in ((256, 16), (256, 8), (128, 32)):
-                c = N.TraceConfig(block, stack, 0, 0, width, quant, tl)
+                c = N.TraceConfig(block, stack, 0, 0, width, quant, 0)
                 batch.launch(c, st)
                 e0, e1 = N.Event(), N.Event()
                 e0.record(st)
@@ -703,8 +702,7 @@ def run_c4(args):
                 e1.record(st)
                 st.sync()
                 ms = e0.elapsed_ms(e1)
-                tried.append("%d/%d/w%d%s%s %.2f" % (block, stack, width, "q" if quant else "",
-                                                     "/tl%d" % tl if tl else "", ms))
+                tried.append("%d/%d/w%d%s %.2f" % (block, stack, width, "q" if quant else "", ms))
                 if best is None or ms < best[0]:
                     best = (ms, c)
         cfg = best[1]
@@ -1036,11 +1034,10 @@ def run_c3_ppm(args):
         cfg, ms = pm.gpu_scene.autotune(lr, hb, pm.P, reps=3)
         log("autotune (light rays, %d): %s, %.3f ms" % (pm.P, cfg_dict(cfg), ms))
         del lr, ls, hb
-        # the winner on the first light queue and the plain quantized launches (with and
-        # without a 64-node treelet), each timed over whole frames (light and camera passes,
+        # the winner on the first light queue and the plain quantized launches, each timed over whole frames (light and camera passes,
         # where the traversal runs); the fastest wins
         best, seen = None, set()
-        for c in (cfg, N.TraceConfig(256, 16, 0, 0, 4, 1, 0), N.TraceConfig(256, 16, 0, 0, 4, 1, 64),
+        for c in (cfg, N.TraceConfig(256, 16, 0, 0, 4, 1, 0),
                   N.TraceConfig(256, 8, 0, 0, 4, 1, 0)):
             key = tuple(getattr(c, f) for f, _ in c._fields_)
             if key in seen:
@@ -1199,7 +1196,7 @@ def run_c3(args):
                         shadow_cfg=N.TraceConfig(256, 16, 0, 0, 4, 1, 0))
     if cfg is None and not args.no_autotune:
         best = None
-        for c in (N.TraceConfig(256, 16, 0, 0, 4, 1, 0), N.TraceConfig(256, 16, 0, 0, 4, 1, 64),
+        for c in (N.TraceConfig(256, 16, 0, 0, 4, 1, 0),
                   N.TraceConfig(256, 8, 0, 0, 4, 1, 0), N.TraceConfig(128, 16, 0, 0, 4, 1, 0)):
             vr.cfg = c
             vr.frame()
@@ -1435,7 +1432,7 @@ def main():
                     help="tree the traversal walks: 2 = the scene's BVH2, 4 = the derived 4-wide tree (0 = default)")
     ap.add_argument("--quantized", action="store_true", help="walk the quantized 4-wide tree")
     ap.add_argument("--treelet", type=int, default=0,
-                    help="quantized tree: nodes of its top levels each block stages in LDS (0..256)")
+                    help="the configuration's treelet field (0..256, quantized tree only; no effect)")
     ap.add_argument("--no-autotune", action="store_true", help="use the library's default launch configuration")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--no-serving", action="store_true", help="pt: skip the served-vs-plain comparison")
