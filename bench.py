@@ -91,7 +91,7 @@ def cfg_dict(cfg):
     if cfg is None:
         return "default"
     return {"block": cfg.block_size or 256, "stack_lds": cfg.stack_lds or 16, "persistent": cfg.persistent,
-            "bvh_width": cfg.bvh_width, "quantized": cfg.quantized, "treelet": cfg.treelet}
+            "bvh_width": cfg.bvh_width or 2, "quantized": cfg.quantized, "treelet": cfg.treelet}
 
 
 BVH2_CFG_ARGS = (256, 16, 0, 0, 2, 0, 0)  # TraceConfig of the reference's binary tree
@@ -120,8 +120,7 @@ BYTES_RULE = ("per ray 32 (ray) + 16 (hit) + 64 x inner nodes of the reference's
 
 
 def node_bytes_of(cfg):
-    """Bytes of one node of the tree a configuration walks: BVH2 64, 4-wide 128, quantized 64 (a
-    configuration of None leaves the tree open, so 64 in either case)."""
+    """Bytes of one node of the tree a configuration walks: BVH2 64, 4-wide 128, quantized 64."""
     return 128 if cfg is not None and cfg.bvh_width == 4 and not cfg.quantized else 64
 
 

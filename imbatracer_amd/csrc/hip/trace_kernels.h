@@ -973,9 +973,7 @@ struct BatchGroups {
 };
 
 // One block of 1024 threads: ray counts of this launch, each queue's first chunk, chunks per group.
-// `also` (or null): another table of the same queues that gets the same numbers.
-__global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchItem* also, BatchGroups groups,
-                                                       int* group_chunks) {
+__global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchGroups groups, int* group_chunks) {
     // thread t owns the queues [b0, b1); items are ordered by group, so a queue's chunk_begin is
     // its exclusive chunk prefix over all queues minus that of its group's first queue
     __shared__ int part[1024];
@@ -989,7 +987,6 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchIt
         int n = items[i].capacity;
         if (items[i].count_dev) n = min(max(*items[i].count_dev, 0), n);
         items[i].a.count = n;
-        if (also) also[i].a.count = n;
         sum += (n + 63) >> 6;
     }
     part[t] = sum;
@@ -1013,7 +1010,6 @@ __global__ __launch_bounds__(1024) void k_batch_prefix(BatchItem* items, BatchIt
     for (int i = b0; i < b1; i++) {
         while (g < 3 && groups.first[g + 1] <= i) g++;
         items[i].chunk_begin = run - base[g];
-        if (also) also[i].chunk_begin = run - base[g];
         run += (items[i].a.count + 63) >> 6;
     }
     if (t < 4) {

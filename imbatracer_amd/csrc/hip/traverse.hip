@@ -145,22 +145,18 @@ constexpr int kDefaultBlock = 256;
 constexpr int kDefaultStack = 16;
 
 // Tree a configuration asks for: 0 the BVH2, 1 the 4-wide tree, 2 its quantized form; -1 if
-// the configuration is invalid; `otherwise` when it leaves the choice open.
-int tree_code(const ImbaTraceConfig* cfg, int otherwise) {
+// the configuration is invalid.  An open choice is the BVH2, whose hits the contract fixes: a box is
+// culled by rounded distances, so where triangles meet or overlap a wider box may let in one that
+// the BVH2's boxes cull.  Of 400,000 rays each, closest hits of the quantized tree differ for 3,555
+// over axis-aligned boxes that overlap, 5,127 aimed at the vertices of a sphere and 36,257 aimed at
+// the vertices of a decal on a floor, some of them in t.
+int tree_code(const ImbaTraceConfig* cfg) {
     const int w = cfg ? cfg->bvh_width : 0;
-    if (w == 0) return (cfg && cfg->quantized) ? -1 : otherwise;
-    if (w == 2) return cfg->quantized ? -1 : 0;
-    if (w == 4) return cfg->quantized ? 2 : 1;
+    const int quantized = cfg ? cfg->quantized : 0;
+    if (w == 0 || w == 2) return quantized ? -1 : 0;
+    if (w == 4) return quantized ? 2 : 1;
     return -1;
 }
-
-// The tree when the configuration leaves it open.  A closest hit does not depend on the tree
-// (every tree has the BVH2's leaves, and a wider box only adds candidates), so it takes the
-// quantized one where the scene has it: 4,096 rays over 4,096 triangles 63 us on the BVH2, 34 us;
-// 300K diffuse rays over 250K triangles 537 against 385; 200K rays over masked instances 1,090
-// against 809.  An any-hit answer is the first hit in the BVH2's order: it stays there, and so
-// do visit counts and stack depths, which describe a tree.
-int default_tree(bool any, bool has_quantized) { return !any && has_quantized ? 2 : 0; }
 
 // The treelet size of a configuration (accepted for the quantized tree, without effect: every
 // node is read through the caches, which hold the top levels anyway).
@@ -168,7 +164,7 @@ int check_treelet(const ImbaTraceConfig* cfg) {
     if (!cfg || !cfg->treelet) return IMBA_OK;
     if (cfg->treelet < 0 || cfg->treelet > kTreeletMaxNodes)
         return fail(IMBA_ERR_INVALID_ARG, "treelet must be 0..%d nodes", kTreeletMaxNodes);
-    if (tree_code(cfg, 0) != 2) return fail(IMBA_ERR_INVALID_ARG, "treelet needs the quantized 4-wide tree");
+    if (tree_code(cfg) != 2) return fail(IMBA_ERR_INVALID_ARG, "treelet needs the quantized 4-wide tree");
     return IMBA_OK;
 }
 
@@ -260,17 +256,17 @@ int launch_trace(const TreeView& t, int* d_err, const ImbaRay* rays, ImbaHit* hi
 }
 
 // The tree of `s` that `cfg` asks for.
-int pick_tree(const ImbaTraceConfig* cfg, int otherwise, const ImbaSceneDesc* d2, const SceneInfo* i2,
-              const ImbaSceneDesc* d4, const ImbaSceneDesc* d4q, const SceneInfo* i4, TreeView* t) {
-    const int code = tree_code(cfg, otherwise);
+int pick_tree(const ImbaTraceConfig* cfg, const ImbaSceneDesc* d2, const SceneInfo* i2, const ImbaSceneDesc* d4,
+              const ImbaSceneDesc* d4q, const SceneInfo* i4, TreeView* t) {
+    const int code = tree_code(cfg);
     if (code < 0) return fail(IMBA_ERR_INVALID_ARG, "bvh_width must be 0, 2 or 4 (quantized only with 4)");
     if (code == 2 && !d4q->nodes) return fail(IMBA_ERR_INVALID_ARG, "the scene has no quantized 4-wide tree");
     *t = code == 0 ? TreeView{d2, i2, 0} : code == 1 ? TreeView{d4, i4, 1} : TreeView{d4q, i4, 2};
     return IMBA_OK;
 }
 
-int tree_of(const ImbaScene* s, const ImbaTraceConfig* cfg, int otherwise, TreeView* t) {
-    return pick_tree(cfg, otherwise, &s->dev, &s->info, &s->dev4, &s->dev4q, &s->info4, t);
+int tree_of(const ImbaScene* s, const ImbaTraceConfig* cfg, TreeView* t) {
+    return pick_tree(cfg, &s->dev, &s->info, &s->dev4, &s->dev4q, &s->info4, t);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -406,10 +402,10 @@ int grow_spill(ImbaTraceBatch* b, int g, size_t bytes, hipStream_t s) {
 }
 
 // One launch of group g: chunks of 64 rays with one lane each, or (QUADS) quarters of chunks with
-// four lanes per ray; `limit` as in k_trace_batch.  With `need` nothing is launched: *need is raised
-// to the bytes of the spill stack the launch would use.
+// four lanes per ray; `limit` as in k_trace_batch.  With `size_only` nothing is launched: the spill
+// stack is made as large as the launch would need it.
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE, bool QUADS>
-int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, size_t* need, hipStream_t s) {
+int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, bool size_only, hipStream_t s) {
     const DeviceProps* p = device_props();
     auto kern = k_trace_batch<BLOCK, STACK_LDS, ANY, MASKED, TREE, QUADS>;
     const int max_stack = b->max_stack[TREE ? 1 : 0][g];
@@ -425,16 +421,11 @@ int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, 
     int spill_depth = 0;
     if (!QUADS && max_stack > STACK_LDS) {
         spill_depth = max_stack - STACK_LDS;
-        const size_t bytes = (size_t)spill_depth * grid * BLOCK * sizeof(int);
-        if (need) {
-            *need = std::max(*need, bytes);
-        } else {
-            const int r = grow_spill(b, g, bytes, s);
-            if (r) return r;
-        }
+        const int r = grow_spill(b, g, (size_t)spill_depth * grid * BLOCK * sizeof(int), s);
+        if (r) return r;
         spill = (int*)b->spill[g].ptr;
     }
-    if (need) return IMBA_OK;
+    if (size_only) return IMBA_OK;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(BLOCK), 0, s, b->d_items[TREE], b->groups.first[g],
                        b->groups.first[g + 1] - b->groups.first[g], b->d_group_chunks + g, b->d_counters + 2 * g,
                        spill, spill_depth, limit);
@@ -443,7 +434,7 @@ int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, 
 }
 
 template <int BLOCK, int STACK_LDS, bool ANY, bool MASKED, int TREE>
-int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, bool open, size_t* need, hipStream_t s) {
+int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, hipStream_t s) {
     const DeviceProps* p = device_props();
     if (!p) return fail(IMBA_ERR_NO_DEVICE, "no HIP device");
     if constexpr (TREE == 2) {
@@ -451,25 +442,22 @@ int launch_batch_group(ImbaTraceBatch* b, int g, int blocks_per_cu, bool open, s
         // a graph replays its launches with whatever sizes a later update brings
         const bool small = b->capacity_chunks[g] <= limit && !b->captured;
         if (limit > 0 && (small || b->device_counts[g] || b->captured)) {
-            int r = need ? IMBA_OK
-                         : launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, true>(b, g, 0, limit, nullptr, s);
-            if (r || (small && open)) return r;  // (recorded, the open choice takes the BVH2)
-            size_t later = 0;  // small: what a later launch that is recorded needs
-            r = launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, 0, limit, small ? &later : need, s);
-            return r ? r : grow_spill(b, g, later, s);
+            const int r = launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, true>(b, g, 0, limit, false, s);
+            if (r) return r;
+            // small: only what a later launch that is recorded needs
+            return launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, 0, limit, small, s);
         }
     }
-    return launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, blocks_per_cu, -1, need, s);
+    return launch_batch_kernel<BLOCK, STACK_LDS, ANY, MASKED, TREE, false>(b, g, blocks_per_cu, -1, false, s);
 }
 
 template <bool ANY, bool MASKED, int TREE>
-int dispatch_batch(ImbaTraceBatch* b, int g, const ImbaTraceConfig* cfg, hipStream_t s, bool open = false,
-                   size_t* need = nullptr) {
+int dispatch_batch(ImbaTraceBatch* b, int g, const ImbaTraceConfig* cfg, hipStream_t s) {
     const int block = cfg && cfg->block_size ? cfg->block_size : kDefaultBlock;
     const int stack = cfg && cfg->stack_lds ? cfg->stack_lds : kDefaultStack;
     const int bpc = cfg ? cfg->blocks_per_cu : 0;
 #define IMBA_SHAPE(B, S) \
-    if (block == B && stack == S) return launch_batch_group<B, S, ANY, MASKED, TREE>(b, g, bpc, open, need, s);
+    if (block == B && stack == S) return launch_batch_group<B, S, ANY, MASKED, TREE>(b, g, bpc, s);
     IMBA_SHAPE(256, 16)
     IMBA_SHAPE(256, 8)
     IMBA_SHAPE(256, 32)
@@ -658,37 +646,20 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
     if (b->n == 0) return IMBA_OK;
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
-    const bool capturing = is_capturing(s);
-    // Closest-hit and any-hit queues may take different trees.  A launch recorded into a graph
-    // must do for every queue a later update brings, so there the open choice is the BVH2.
-    const int closest = tree_code(cfg, default_tree(false, b->quantized_ok && !capturing));
-    const int any = tree_code(cfg, default_tree(true, false));
-    if (closest < 0) return fail(IMBA_ERR_INVALID_ARG, "bvh_width must be 0, 2 or 4 (quantized only with 4)");
-    if (closest == 2 && !b->quantized_ok) return fail(IMBA_ERR_INVALID_ARG, "a queue's scene has no quantized tree");
+    const int tree = tree_code(cfg);
+    if (tree < 0) return fail(IMBA_ERR_INVALID_ARG, "bvh_width must be 0, 2 or 4 (quantized only with 4)");
+    if (tree == 2 && !b->quantized_ok) return fail(IMBA_ERR_INVALID_ARG, "a queue's scene has no quantized tree");
     int r = check_treelet(cfg);
     if (r) return r;
-    if (capturing) {
+    if (is_capturing(s)) {
         b->captured = true;
         b->captured_groups = b->groups;
     }
-    hipLaunchKernelGGL(k_batch_prefix, dim3(1), dim3(1024), 0, s, b->d_items[closest],
-                       any == closest ? (BatchItem*)nullptr : b->d_items[any], b->groups, b->d_group_chunks);
+    hipLaunchKernelGGL(k_batch_prefix, dim3(1), dim3(1024), 0, s, b->d_items[tree], b->groups, b->d_group_chunks);
     IMBA_HIP_TRY(hipGetLastError());
-    // the tree an open choice takes in a graph
-    const bool other = closest == 2 && tree_code(cfg, 0) == 0;
     for (int g = 0; g < 4; g++) {
         if (b->groups.first[g + 1] == b->groups.first[g] || b->capacity_chunks[g] == 0) continue;
-        if (other && g < 2) {  // both trees' spill stacks at once: growing later would wait and free
-            size_t need = 0;
-            r = g == 0 ? dispatch_batch<false, false, 0>(b, g, cfg, s, true, &need)
-                       : dispatch_batch<false, true, 0>(b, g, cfg, s, true, &need);
-            if (!r)
-                r = g == 0 ? dispatch_batch<false, false, 2>(b, g, cfg, s, true, &need)
-                           : dispatch_batch<false, true, 2>(b, g, cfg, s, true, &need);
-            if (!r) r = grow_spill(b, g, need, s);
-            if (r) return r;
-        }
-        switch (g + 4 * (g >= 2 ? any : closest)) {
+        switch (g + 4 * tree) {
             case 0: r = dispatch_batch<false, false, 0>(b, g, cfg, s); break;
             case 1: r = dispatch_batch<false, true, 0>(b, g, cfg, s); break;
             case 2: r = dispatch_batch<true, false, 0>(b, g, cfg, s); break;
@@ -697,8 +668,8 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
             case 5: r = dispatch_batch<false, true, 1>(b, g, cfg, s); break;
             case 6: r = dispatch_batch<true, false, 1>(b, g, cfg, s); break;
             case 7: r = dispatch_batch<true, true, 1>(b, g, cfg, s); break;
-            case 8: r = dispatch_batch<false, false, 2>(b, g, cfg, s, other); break;
-            case 9: r = dispatch_batch<false, true, 2>(b, g, cfg, s, other); break;
+            case 8: r = dispatch_batch<false, false, 2>(b, g, cfg, s); break;
+            case 9: r = dispatch_batch<false, true, 2>(b, g, cfg, s); break;
             case 10: r = dispatch_batch<true, false, 2>(b, g, cfg, s); break;
             default: r = dispatch_batch<true, true, 2>(b, g, cfg, s); break;
         }
@@ -729,7 +700,7 @@ int imba_autotune(const ImbaScene* sc, const ImbaRay* rays, ImbaHit* hits, int c
             ImbaTraceConfig cfg{shape[0], shape[1], refill, 0, tree[0], tree[1], 0};
             if (tree[1] && !sc->dev4q.nodes) continue;
             TreeView t{};
-            r = tree_of(sc, &cfg, 0, &t);
+            r = tree_of(sc, &cfg, &t);
             if (!r)
                 r = launch_trace(t, sc->d_error, rays, hits, nullptr, count, any_hit != 0, !sc->info.all_opaque, &cfg,
                                  s);
@@ -773,8 +744,7 @@ static int trace_entry(const ImbaScene* s, const ImbaRay* rays, ImbaHit* hits, u
                        uint32_t* depth_hist = nullptr) {
     IMBA_CHECK_ARG(s, "scene is NULL");
     TreeView t{};
-    const bool stats = counts || depth_hist;
-    int r = tree_of(s, cfg, stats ? 0 : default_tree(any, s->dev4q.nodes != nullptr), &t);
+    int r = tree_of(s, cfg, &t);
     if (r) return r;
     return launch_trace(t, s->d_error, rays, hits, counts, count, any, !s->info.all_opaque, cfg, stream, count_dev,
                         depth_hist);

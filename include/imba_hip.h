@@ -286,10 +286,11 @@ typedef struct ImbaTraceConfig {
                               rays (0 = default: persistent launches fill the resident
                               blocks, others launch one thread per ray)                 */
     int bvh_width;         /* 2: the scene's BVH2 as given; 4: the 4-wide tree derived from
-                              it at upload (same leaves); 0 = default: any hits, visit counts,
-                              stack depths and batches recorded into a graph take the BVH2,
-                              closest hits (which do not depend on the tree) the quantized
-                              4-wide tree where the scene has one                          */
+                              it at upload (same leaves); 0 = default, the BVH2.  Boxes are
+                              culled by rounded distances, so where triangles meet or overlap
+                              the 4-wide trees may report a closest hit (another triangle, or
+                              a nearer t) that the BVH2's boxes cull; elsewhere closest hits
+                              are the same.  Any hits are the first in the tree's order      */
     int quantized;         /* with bvh_width 4: 64-byte nodes whose child boxes are 8-bit
                               offsets from the node box, rounded outward                  */
     int treelet;           /* quantized tree only, 0..256: accepted, without effect (every node
@@ -366,7 +367,8 @@ int imba_trace_batch_release(ImbaTraceBatch* b);
 /* Launch shape autotuning: times every supported shape (static and persistent) of every tree
  * (BVH2, 4-wide, quantized) on the given device queue
  * with HIP events, `reps` launches each after one warm-up, and returns the fastest in *best
- * (and its mean time per launch in *best_ms, nullable).  Results do not depend on the shape. */
+ * (and its mean time per launch in *best_ms, nullable).  Results do not depend on the shape; what
+ * depends on the tree is said at ImbaTraceConfig.bvh_width. */
 int imba_autotune(const ImbaScene* s, const ImbaRay* rays, ImbaHit* hits, int count, int any_hit, int reps,
                   ImbaTraceConfig* best, float* best_ms, void* stream);
 

@@ -201,3 +201,78 @@ def test_single_triangle_and_dummy_parent(gpu):
     want, bad = oracle.trace(a, rays)
     assert bad == 0 and _same(got, want)
     assert list(got["tri_id"]) == [0, 0, 0]
+
+
+def _ties(name):
+    """A scene where triangles meet or overlap, and rays that find them there."""
+    if name == "boxes":
+        return T.box_scene(), T.random_rays(100000, seed=3, box=(0.0, 2.2))
+    b, points = T.sphere_scene() if name == "sphere" else T.decal_scene()
+    return b, T.aimed_rays(points, 100000, seed=5)
+
+
+@pytest.mark.parametrize("name", ["boxes", "sphere", "decal"])
+def test_default_where_triangles_meet(gpu, name):
+    """Overlapping coplanar faces, shared vertices and a coplanar decal: which triangles a walk
+    tests there depends on its boxes.  Launches that leave the tree open give the oracle's BVH2
+    answer: plain, with a device count, through the FFI, batched, and batched in a graph."""
+    b, rays = _ties(name)
+    a = b.arrays()
+    sc = S.Scene(b.desc())
+    n = len(rays)
+    rb, cnt = N.DeviceBuffer.from_array(rays), N.DeviceBuffer.from_array(np.array([n], np.int32))
+    for any_hit in (False, True):
+        want, bad = oracle.trace(a, rays, any_hit=any_hit, threads=8)
+        assert bad == 0 and (want["tri_id"] >= 0).sum() > n // 4
+        for k in (4096, n):
+            got = sc.trace_host(rays[:k], any_hit=any_hit)
+            assert _same(got, want[:k]), _report(got, want[:k])
+        hb = N.DeviceBuffer(16 * n)
+        fn = N.lib.imba_occluded_dev if any_hit else N.lib.imba_intersect_dev
+        N.check(fn(sc.h, rb.ptr, hb.ptr, n, cnt.ptr, None, None), "dev")
+        assert _same(hb.download(N.HIT_DTYPE, n), want)
+        bufs = {k: N.DeviceBuffer.from_array(a[k]) for k in
+                ("nodes", "instances", "tris", "indices", "texcoords", "masks", "mask_buffer")}
+        hb = N.DeviceBuffer(16 * n)
+        ffi = N.lib.occluded_gpu_masked_instanced if any_hit else N.lib.intersect_gpu_masked_instanced
+        ffi(a["root"], bufs["nodes"].ptr, bufs["instances"].ptr, bufs["tris"].ptr, rb.ptr, hb.ptr, bufs["indices"].ptr,
+            bufs["texcoords"].ptr, bufs["masks"].ptr, bufs["mask_buffer"].ptr, n)
+        assert _same(hb.download(N.HIT_DTYPE, n), want)
+        hb = N.DeviceBuffer(16 * n)
+        st = N.Stream()
+        batch = S.TraceBatch([(sc, rb, hb, n, None, any_hit)])
+        batch.launch(None, st)
+        st.sync()
+        assert _same(hb.download(N.HIT_DTYPE, n), want)
+        S.Graph.begin(st)
+        try:
+            batch.launch(None, st)
+        finally:
+            g = S.Graph.end(st)
+        for _ in range(2):
+            hb.upload(np.full(4 * n, 7, np.int32))
+            g.launch(st)
+            st.sync()
+            assert _same(hb.download(N.HIT_DTYPE, n), want)
+    assert sc.error_count() == 0
+
+
+def test_default_launch_is_recorded_without_spill(gpu):
+    """A scene whose BVH2 stack fits the LDS part, though its 4-wide one does not: the first call
+    on a stream that leaves the tree open can be recorded into a graph."""
+    b = T.sphere_scene()[0]
+    depth = C.c_int()
+    N.check(N.lib.imba_scene_validate(C.byref(b.desc()), C.byref(depth), None), "validate")
+    assert depth.value <= 16 < S.wide_tree(b.arrays())["max_stack"]
+    sc = S.Scene(b.desc())
+    rays = T.random_rays(4096, seed=6, box=(-1.5, 1.5))
+    want, _ = oracle.trace(b.arrays(), rays, threads=8)
+    rb, hb, st = N.DeviceBuffer.from_array(rays), N.DeviceBuffer(16 * 4096), N.Stream()
+    S.Graph.begin(st)
+    try:
+        sc.intersect(rb, hb, 4096, None, st)
+    finally:
+        g = S.Graph.end(st)
+    g.launch(st)
+    st.sync()
+    assert _same(hb.download(N.HIT_DTYPE, 4096), want)
