@@ -150,15 +150,17 @@ __device__ __forceinline__ int query_wave_list(const GridParams& g, const float4
     constexpr int kMany = 10;    // candidates of a group above which the bound is worth finding
     constexpr int kHalvings = 7;
     constexpr uint32_t kOctaves = 6;  // the bound is sought down to limit / 64
-    const float inf = __int_as_float(0x7f800000);
+    // Lanes past a bucket's end and past the list's end hold NaN, which is at most no limit: infinity
+    // would be at most an infinite one (an unlimited radius).
+    const float none = __int_as_float(0x7fc00000);
     const int lane = (int)(threadIdx.x & 63);
     my_id = -1;
     int count = 0;
     // Distances are compared as their bits where they are wave-uniform (squares' sums are never
     // negative, so the order is the same), which keeps that work on the scalar unit.
     const uint32_t radius_bits = __float_as_uint(g.radius_sqr);
-    uint32_t kth = 0x7f800000u;  // dist[k - 1], infinity until the list is full
-    my_dist = inf;               // lanes past the list's end
+    uint32_t kth = 0x7fc00000u;  // dist[k - 1]; above every distance until the list is full
+    my_dist = none;
     for (int j = 0; j < 8; j++) {
         const int beg = __builtin_amdgcn_readlane(probes.begin, first + j);
         const int n = __builtin_amdgcn_readlane(probes.size, first + j);
@@ -168,8 +170,7 @@ __device__ __forceinline__ int query_wave_list(const GridParams& g, const float4
             float4 p[kGroup];
 #pragma unroll
             for (int i = 0; i < kGroup; i++) {
-                // past the bucket's end: x = +inf, which no limit admits
-                p[i] = make_float4(inf, 0.0f, 0.0f, 0.0f);
+                p[i] = make_float4(none, 0.0f, 0.0f, 0.0f);
                 if (base + 64 * i < n && base + 64 * i + lane < n) p[i] = pos4[beg + base + 64 * i + lane];
             }
             float d2[kGroup];
@@ -187,7 +188,7 @@ __device__ __forceinline__ int query_wave_list(const GridParams& g, const float4
                 float least = d2[0];
 #pragma unroll
                 for (int i = 1; i < kGroup; i++) least = fminf(least, d2[i]);
-                const float listed = lane < k ? my_dist : inf;
+                const float listed = lane < k ? my_dist : none;
                 if (__popcll(__ballot(least <= __uint_as_float(lim))) + count >= k) {
                     // lim: always a distance that at least k values do not exceed
                     uint32_t lo = max(lim, kOctaves << 23) - (kOctaves << 23);

@@ -15,9 +15,9 @@
 // 4M photons, 8M buckets: 446 us in 26 launches before the sort was rewritten and the smaller
 // launches were merged, now 291 in 12.
 // The query visits the same 8 buckets in the same order as the reference (duplicates
-// included), one query per wave, and keeps the k-capped, distance-sorted list in lanes 0..k-1
-// with the reference's insertion rule.  Squared distances are computed without fused
-// multiply-add, as on the host.
+// included), a wave taking its queries one after the other (two where there are enough), and keeps
+// the k-capped, distance-sorted list in lanes 0..k-1 with the reference's insertion rule.  Squared
+// distances are computed without fused multiply-add, as on the host.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -219,3 +219,22 @@ def test_build_tile_edges(gpu, n, spread):
     _check_build(g, og, n)
     queries = photons[:: max(1, n // 8), :3] + np.float32(0.3 * radius)
     _check_queries(g, og, np.ascontiguousarray(queries), 10)
+
+
+@pytest.mark.parametrize("radius", [1e19, 1e20, 3.4028234663852886e38])
+@pytest.mark.parametrize("n", [3, 40, 200, 257, 700])
+def test_unlimited_radius(gpu, n, radius):
+    """A radius whose square is infinite (or, 1e19, nearly so) asks for the k nearest without a
+    limit: lists shorter and longer than the photons there are, on both sides of the two query
+    kernels; every eighth photon is so far away that its squared distance is infinite too."""
+    rng = np.random.default_rng(n)
+    photons = np.zeros((n, 4), np.float32)
+    photons[:, :3] = rng.integers(0, 9, (n, 3))
+    photons[::8, :3] *= np.float32(1e25)
+    g, _ = _grid(photons, radius)
+    og = oracle.Grid()
+    og.build(photons[:, :3], radius)
+    _check_build(g, og, n)
+    queries = np.concatenate([rng.integers(0, 9, (37, 3)), photons[:24, :3]]).astype(np.float32)
+    for k in (1, 2, 3, 4, 10, 41, 63, 64, 65, 300):
+        assert _check_queries(g, og, queries, k) > 0, k

@@ -226,6 +226,44 @@ def test_fused_merge(pm):
     assert np.allclose(fused, lists, rtol=1e-5, atol=1e-6 * np.abs(lists).max())
 
 
+@pytest.mark.parametrize("m", [3, 70, 700])
+def test_fused_merge_unlimited_radius(pm, m):
+    """A grid whose radius is unlimited (its square infinite) over fewer and more photons than the list
+    holds: the fused launch adds the image of the index lists, which are the oracle's."""
+    from imbatracer_amd import scene as S
+
+    radius, nq = 1e20, pm.n_cam
+    g = S.HashGrid()
+    g.build(pm.photon_rays, 32, 0, m, radius)
+    rec = N.DeviceBuffer(m * 32)
+    N.check(N.lib.imba_ppm_merge_records(g.h, pm.photon_rays.ptr, pm.photon_states.ptr, rec.ptr, None),
+            "ppm_merge_records")
+    oi, od, oc = N.DeviceBuffer(nq * pm.k * 4), N.DeviceBuffer(nq * pm.k * 4), N.DeviceBuffer(nq * 4)
+    g.query(pm.queries, 64, 0, nq, pm.k, oi, oc, od)
+    og = oracle.Grid()
+    og.build(np.ascontiguousarray(pm.photons_host()[0]["pos"][:m]), radius)
+    pos = np.ascontiguousarray(pm.queries_host()["pos"])
+    want_i, _, want_c = og.query_many(pos, pm.k)
+    idx, cnt = oi.download(np.int32, nq * pm.k).reshape(nq, -1), oc.download(np.int32, nq)
+    assert np.array_equal(cnt, want_c) and (cnt > 0).any()
+    used = np.arange(pm.k) < cnt[:, None]
+    assert np.array_equal(idx[used], want_i[used])
+    images = []
+    for fused in (False, True):
+        pm.clear_image()
+        pm.stream.sync()
+        if fused:
+            N.check(N.lib.imba_ppm_merge_grid(g.h, rec.ptr, pm.queries.ptr, nq, pm.k, pm.radius, pm.P, pm.image.ptr,
+                                              pm.stream.handle), "ppm_merge_grid")
+        else:
+            N.check(N.lib.imba_ppm_merge(pm.queries.ptr, nq, pm.k, oi.ptr, od.ptr, oc.ptr, pm.photon_rays.ptr,
+                                         pm.photon_states.ptr, pm.radius, pm.P, pm.image.ptr, pm.stream.handle),
+                    "ppm_merge")
+        images.append(pm.image.download(np.float32, pm.w * pm.h * 3, pm.stream).astype(np.float64))
+    assert np.count_nonzero(images[0]) > 0
+    assert np.allclose(images[1], images[0], rtol=1e-5, atol=1e-6 * np.abs(images[0]).max())
+
+
 def test_fused_frame(pm):
     """A frame with merge="fused" renders the image of the query + merge frame."""
     pm.clear_image()

@@ -145,6 +145,28 @@ def test_merging_matches_restatement(vr):
     assert total > 100
 
 
+@pytest.mark.parametrize("m", [3, 70, 700])
+def test_merging_unlimited_radius(vr, m):
+    """A grid whose radius is unlimited (its square infinite) over fewer and more light vertices than
+    the list holds: the merge is the restatement's over the oracle grid's lists."""
+    from imbatracer_amd import scene as S
+
+    a, b = vr.cache_host()
+    g, og = S.HashGrid(), oracle.Grid()
+    g.build(vr.vtx_a, 32, 0, m, 1e20)
+    og.build(np.ascontiguousarray(a["pos"][:m]), 1e20)
+    rec = N.DeviceBuffer(m * 32)
+    N.check(N.lib.imba_vcm_merge_records(g.h, vr.vtx_a.ptr, vr.vtx_b.ptr, rec.ptr, None), "vcm_merge_records")
+    q = vr.kept["camera"][0]["queries"]
+    qb, image = N.DeviceBuffer.from_array(q), N.DeviceBuffer.from_array(np.zeros(vr.w * vr.h * 3, np.float32))
+    N.check(N.lib.imba_vcm_merge(N.C.byref(vr.frame_args), g.h, rec.ptr, qb.ptr, len(q), None, vr.k, image.ptr, None),
+            "vcm_merge")
+    got = image.download(np.float32, vr.w * vr.h * 3).astype(np.float64).reshape(-1, 3)
+    want, merged = _merge_restated(vr, q, og, a, b)
+    assert merged > 100
+    assert np.allclose(got, want, rtol=1e-4, atol=1e-5 * np.abs(want).max())
+
+
 # ---- every step restated (oracle/vcm.py) on the GPU's own queues ----
 
 def _params(vr):
