@@ -34,11 +34,10 @@ struct ImbaHashGrid {
     uint32_t* bucket_box = nullptr;  // per bucket: bounds of its photons (lo xyz, hi xyz) as
                                      // ordered_bits, written for the non-empty buckets of the last
                                      // build
-    int box_cap = 0;
     imba::GridParams* d_params = nullptr;
     float* partial = nullptr;  // 6 per bounds block
     int* digits = nullptr;     // the sort's tile counts
-    int digits_cap = 0;
+    size_t digits_cap = 0;
 };
 
 namespace imba {

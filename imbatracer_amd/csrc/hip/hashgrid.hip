@@ -25,6 +25,7 @@
 
 #include "common.h"
 #include "grid_query.h"
+#include "grid_size.h"
 #include "radix.h"
 
 namespace imba {
@@ -448,13 +449,36 @@ __global__ __launch_bounds__(64) void k_query_lds(const GridParams* gp, const in
     if (lane == 0) out_count[q] = count;
 }
 
-template <typename T>
-int ensure(T*& p, int& cap_now, int want) {
-    if (p && cap_now >= want) return IMBA_OK;
+// A new buffer of `want` elements in place of p, one of those whose capacity is `cap`: zero from
+// when the old one is gone.
+template <typename T, typename CAP>
+int replace(T*& p, CAP& cap, size_t want) {
     if (p) IMBA_HIP_TRY(hipFree(p));
     p = nullptr;
-    IMBA_HIP_TRY(hipMalloc((void**)&p, sizeof(T) * (size_t)std::max(want, 1)));
-    cap_now = want;
+    cap = 0;
+    IMBA_HIP_TRY(hipMalloc((void**)&p, sizeof(T) * std::max<size_t>(want, 1)));
+    return IMBA_OK;
+}
+
+// Buffers for `count` photons and `table` buckets.
+int reserve(ImbaHashGrid* g, int count, int table) {
+    int r = IMBA_OK;
+    if (table > g->table_cap) {
+        if ((r = replace(g->cell_ends, g->table_cap, table))) return r;
+        if ((r = replace(g->bucket_box, g->table_cap, grid_box_words(table)))) return r;
+        g->table_cap = table;
+    }
+    if (count > g->cap) {
+        for (int** p : {&g->order, &g->keys_a, &g->vals_a, &g->keys_b, &g->vals_b})
+            if ((r = replace(*p, g->cap, count))) return r;
+        if ((r = replace(g->pos4, g->cap, count))) return r;
+        g->cap = count;
+    }
+    const size_t digits = radix_counts_size<kSortItems>(std::max(count, 1));
+    if (digits > g->digits_cap) {
+        if ((r = replace(g->digits, g->digits_cap, digits))) return r;
+        g->digits_cap = digits;
+    }
     return IMBA_OK;
 }
 
@@ -496,40 +520,23 @@ int imba_hashgrid_release(ImbaHashGrid* g) {
 int imba_hashgrid_build(ImbaHashGrid* g, const void* photons, int stride, int pos_offset, int count, float radius,
                         void* stream) {
     IMBA_CHECK_ARG(g, "grid is NULL");
-    IMBA_CHECK_ARG(count >= 0 && count <= (1 << 29), "count out of range");
+    IMBA_CHECK_ARG(count >= 0 && count <= kGridMaxPhotons, "count out of range");
     IMBA_CHECK_ARG(count == 0 || photons, "photons is NULL");
     IMBA_CHECK_ARG(stride >= 12 && stride % 4 == 0 && pos_offset >= 0 && pos_offset % 4 == 0 && pos_offset + 12 <= stride,
                    "stride/pos_offset must be multiples of 4 with the position inside the record");
     IMBA_CHECK_ARG(radius > 0.0f, "radius must be positive");
     bool sync;
     hipStream_t s = resolve_stream(stream, &sync);
-    // Bucket table: max(previous size, 2 * count) (rangesearch.h:33-34).
-    const int table = std::max(g->table_size, 2 * count);
-    if (table > g->table_cap) {
-        int r = ensure(g->cell_ends, g->table_cap, table);
-        if (r) return r;
-    }
-    if (table > g->box_cap) {  // 6 uint32 per bucket
-        int c = 0, r = ensure(g->bucket_box, c, 6 * table);
-        if (r) return r;
-        g->box_cap = table;
+    const int table = grid_table_size(g->table_size, count);
+    const int reserved = reserve(g, count, table);
+    if (reserved) {
+        if (g->table_cap == 0 || g->cap < g->count) {  // the last build's buffers are gone
+            g->table_size = 0;
+            g->count = 0;
+        }
+        return reserved;
     }
     g->table_size = table;
-    if (count > g->cap) {
-        int c = 0, r;
-        if ((r = ensure(g->order, c, count))) return r;
-        c = 0; if ((r = ensure(g->keys_a, c, count))) return r;
-        c = 0; if ((r = ensure(g->vals_a, c, count))) return r;
-        c = 0; if ((r = ensure(g->keys_b, c, count))) return r;
-        c = 0; if ((r = ensure(g->vals_b, c, count))) return r;
-        c = 0; if ((r = ensure(g->pos4, c, count))) return r;
-        g->cap = count;
-    }
-    const int ndigits = (int)radix_counts_size<kSortItems>(std::max(count, 1));
-    if (ndigits > g->digits_cap) {
-        int r = ensure(g->digits, g->digits_cap, ndigits);
-        if (r) return r;
-    }
     g->count = count;
     const unsigned char* ph = (const unsigned char*)photons;
     const int nparts = std::min(kBoundsBlocks, std::max(1, ceil_div(count, kBlock)));
