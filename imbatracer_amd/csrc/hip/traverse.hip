@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -390,6 +391,10 @@ struct ImbaTraceBatch {
     bool captured = false;  // launched into a graph: the tables may no longer move, and the
                             // queues per launch group (kernel arguments) may no longer change
     imba::BatchGroups captured_groups{};
+    // What the launches recorded into graphs can trace, per tree width and group: the deepest stack
+    // (recorded launches keep their kernels and spill depths), 0 where nothing was launched.
+    int captured_stack[2][4] = {{INT_MAX, INT_MAX, INT_MAX, INT_MAX}, {INT_MAX, INT_MAX, INT_MAX, INT_MAX}};
+    bool captured_quantized = false;  // one of them walks the quantized tree
 };
 
 namespace imba {
@@ -494,6 +499,7 @@ int set_tables(ImbaTraceBatch* b, const ImbaTraceItem* items, int n_items, hipSt
     bool quantized_ok = true;
     BatchGroups groups{};
     int max_stack[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    int used_stack[2][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}};  // of the queues that may hold rays
     long long chunks[4] = {0, 0, 0, 0};
     bool device_counts[4] = {false, false, false, false};
     for (int g = 0; g < 4; g++) {
@@ -517,6 +523,10 @@ int set_tables(ImbaTraceBatch* b, const ImbaTraceItem* items, int n_items, hipSt
             e.group = g;
             max_stack[0][g] = std::max(max_stack[0][g], it.scene->info.max_stack);
             max_stack[1][g] = std::max(max_stack[1][g], it.scene->info4.max_stack);
+            if (it.count > 0) {
+                used_stack[0][g] = std::max(used_stack[0][g], it.scene->info.max_stack);
+                used_stack[1][g] = std::max(used_stack[1][g], it.scene->info4.max_stack);
+            }
             chunks[g] += ceil_div(it.count, 64);
             device_counts[g] |= it.count_dev != nullptr;
             table.push_back(e);
@@ -537,6 +547,14 @@ int set_tables(ImbaTraceBatch* b, const ImbaTraceItem* items, int n_items, hipSt
     if (b->captured && std::memcmp(&groups, &b->captured_groups, sizeof(groups)) != 0)
         return fail(IMBA_ERR_INVALID_ARG, "batch was launched into a graph: the number of queues per kind "
                     "(closest / any hit, masked / opaque) must stay as captured");
+    for (int w = 0; w < 2; w++)
+        for (int g = 0; g < 4; g++)
+            if (used_stack[w][g] > b->captured_stack[w][g])
+                return fail(IMBA_ERR_CAPACITY, "batch was launched into a graph with queues of this kind that need at "
+                            "most %d stack entries; a queue's scene may need %d", b->captured_stack[w][g], used_stack[w][g]);
+    if (b->captured_quantized && !quantized_ok)
+        return fail(IMBA_ERR_INVALID_ARG, "batch was launched into a graph over the quantized tree; a queue's scene "
+                    "has none");
     const size_t bytes = sizeof(BatchItem) * (size_t)n;
     if (n > b->cap) {
         // grow: device tables and staging buffers (synchronous).  A graph replays its launches
@@ -654,6 +672,14 @@ int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void*
     if (is_capturing(s)) {
         b->captured = true;
         b->captured_groups = b->groups;
+        b->captured_quantized |= tree == 2;
+        const int stack_lds = cfg && cfg->stack_lds ? cfg->stack_lds : kDefaultStack;
+        for (int g = 0; g < 4; g++) {
+            // one lane per ray: the LDS part and a spill stack for the rest; four lanes per ray are
+            // only recorded where that many entries fit their LDS
+            int& held = b->captured_stack[tree ? 1 : 0][g];
+            held = std::min(held, b->capacity_chunks[g] == 0 ? 0 : std::max(stack_lds, b->max_stack[tree ? 1 : 0][g]));
+        }
     }
     hipLaunchKernelGGL(k_batch_prefix, dim3(1), dim3(1024), 0, s, b->d_items[tree], b->groups, b->d_group_chunks);
     IMBA_HIP_TRY(hipGetLastError());

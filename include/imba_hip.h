@@ -358,7 +358,11 @@ typedef struct ImbaTraceBatch ImbaTraceBatch;
 int imba_trace_batch_create(const ImbaTraceItem* items, int n_items, ImbaTraceBatch** out);
 /* Replaces the batch's queues (same rules as create).  The new table is copied on `stream`
  * (pinned staging, no device-wide synchronisation unless the batch must grow): launch on the
- * same stream after it.  For request loops whose set of queues changes every step. */
+ * same stream after it.  For request loops whose set of queues changes every step.  Launches recorded
+ * into a graph keep their kernels and stacks: after one, the number of queues per kind must stay, and
+ * an update is refused (the queues stay as they were) where a queue's scene may need a deeper stack
+ * than the recorded queues of its kind (IMBA_ERR_CAPACITY; kinds recorded without rays stay so) or
+ * has no quantized tree and the recorded launches walk it (IMBA_ERR_INVALID_ARG). */
 int imba_trace_batch_update(ImbaTraceBatch* b, const ImbaTraceItem* items, int n_items, void* stream);
 /* cfg: block_size / stack_lds / blocks_per_cu as for imba_intersect; every launch is persistent. */
 int imba_trace_batch_launch(ImbaTraceBatch* b, const ImbaTraceConfig* cfg, void* stream);

@@ -214,3 +214,56 @@ def test_autotune_returns_a_supported_shape(gpu):
     assert (cfg.block_size, cfg.stack_lds) in [(256, 16), (256, 8), (256, 32), (128, 16), (128, 32), (64, 32), (64, 64)]
     assert cfg.persistent in (0, 32) and ms > 0
     assert _same(sc.trace_host(rays, cfg=cfg), oracle.trace(b.arrays(), rays, threads=8)[0])
+
+
+@pytest.mark.parametrize("cfg", [None, N.TraceConfig(256, 8, 0, 0, 2, 0, 0), N.TraceConfig(256, 16, 0, 0, 4, 1, 0),
+                                 N.TraceConfig(256, 8, 0, 0, 4, 1, 0)], ids=["bvh2", "bvh2-8", "q4", "q4-8"])
+def test_recorded_batch_refuses_what_it_cannot_trace(gpu, cfg):
+    """A recorded launch keeps its kernels and stacks.  An update whose scene may need a deeper stack,
+    has no quantized tree where the recording walks it, or gives rays to a kind of queue that was
+    recorded without, is refused and leaves the queues as they were; one that fits is replayed."""
+    small, deep = T.random_tri_scene(500)[0], T.random_tri_scene(200000)[0]
+    far = np.array([[-3e38, 0, 0], [3e38, 0, 0], [0, 1, 0]], np.float32)
+    huge = T._mesh_scene(np.concatenate([far, far + np.float32(1)]), np.array([[0, 1, 2], [3, 4, 5]]))
+    assert len(S.wide_tree(huge.arrays())["qnodes"]) == 0
+    sc, sd, sh = (S.Scene(b.desc()) for b in (small, deep, huge))
+    rays = T.random_rays(3000, seed=31)
+    rb = N.DeviceBuffer.from_array(rays)
+    hits, none = _filled_hits(3000), _filled_hits(3000)
+    want, _ = oracle.trace(small.arrays(), rays)
+    want_any, _ = oracle.trace(small.arrays(), rays, any_hit=True)
+    st = N.Stream()
+    queues = [(sc, rb, hits, 2000, None, False), (sc, rb, none, 0, None, True)]
+    batch = S.TraceBatch(queues)
+    batch.launch(cfg, st)
+    st.sync()
+    S.Graph.begin(st)
+    try:
+        batch.launch(cfg, st)
+    finally:
+        g = S.Graph.end(st)
+    refused = [(sd, rb, hits, 2000, None, False), (sc, rb, none, 0, None, True)], \
+              [(sc, rb, hits, 2000, None, False), (sc, rb, none, 10, None, True)]
+    for items in refused:
+        with pytest.raises(N.ImbaError, match="capacity"):
+            batch.update(items, st)
+    if cfg is not None and cfg.quantized:
+        with pytest.raises(N.ImbaError, match="quantized"):
+            batch.update([(sh, rb, hits, 2000, None, False), queues[1]], st)
+    # an empty queue of the deeper scene, and more rays of the recorded one, can be traced
+    batch.update([(sc, rb, hits, 3000, None, False), (sd, rb, none, 0, None, True)], st)
+    for n in (3000, 2000):
+        if n == 2000:
+            batch.update(queues, st)
+        hits.upload(np.repeat(SENTINEL, 3000), st)
+        g.launch(st)
+        st.sync()
+        got = hits.download(N.HIT_DTYPE, 3000)
+        assert _same(got[:n], want[:n]) and _same(got[n:], np.repeat(SENTINEL, 3000 - n))
+    assert _same(none.download(N.HIT_DTYPE, 3000), np.repeat(SENTINEL, 3000))
+    # another batch is not bound by this one's recording
+    other = S.TraceBatch(queues)
+    other.update([(sc, rb, none, 3000, None, True)])
+    other.launch(None)
+    assert _same(none.download(N.HIT_DTYPE, 3000), want_any)
+    assert sc.error_count() == 0
