@@ -653,6 +653,13 @@ __device__ __forceinline__ void stack_init(LaneStack<BLOCK, STACK_LDS>& st, int*
 // over masked instances 790 -> 743, 48 queues in a batch 1,040 -> 917; path-traced frame 640x480
 // 4,261 -> 4,002.
 
+// Stack entries written before are read after by other lanes of the wave.  The hardware keeps a
+// wave's accesses to one address in order, in LDS and in memory; this holds the compiler to it.
+__device__ __forceinline__ void stack_shared() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Lane (4 q + k) receives the value of lane 4 q + {A, B, C, D}[k].
 template <int A, int B, int C, int D>
 __device__ __forceinline__ uint32_t quad_u(uint32_t v) {
@@ -762,6 +769,7 @@ __device__ __forceinline__ bool advance_quad(const TraceArgs& a, TraceState& s, 
             const int top = st.sp + max((int)cnt - 1, 0);
             if (st.holds(top)) {
                 if (j > 0 && (uint32_t)j < cnt) st.put(top - j, (int)c);
+                stack_shared();
                 st.sp = top;
             } else {
                 s.bad = 1;  // not for the trees the launch was checked for
@@ -851,6 +859,7 @@ __device__ __forceinline__ void wave_trace(const TraceArgs& a, LaneStack<BLOCK, 
     LaneStack<BLOCK, STACK_LDS> theirs = st;
     theirs.lane_slot += from - lane;
     theirs.spill_slot += from - lane;
+    stack_shared();
     while (__ballot(live)) {
         if (live && advance_quad<ANY, MASKED>(a, s, theirs, j)) {
             write_quad(a, s, id, j);
