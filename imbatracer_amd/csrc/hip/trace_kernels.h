@@ -45,6 +45,7 @@ struct TraceArgs {
     int* err;             // incremented once per ray that met a malformed structure
     int* spill;           // global stack entries beyond the LDS part
     int spill_depth;      // spill entries per thread
+    int spill_stride;     // threads that may spill (the first of the grid)
     int* work_counter;    // persistent variant: next ray to fetch
     const int* count_dev; // device ray count read when the launch runs (<= count), or null
     int quad;             // quantized tree: a launch of at most this many rays gives each ray four lanes
@@ -628,7 +629,7 @@ __device__ __forceinline__ void stack_init(LaneStack<BLOCK, STACK_LDS>& st, int*
     st.spill_depth = a.spill_depth;
     st.lane_slot = threadIdx.x;
     st.spill_slot = blockIdx.x * BLOCK + threadIdx.x;
-    st.spill_stride = gridDim.x * BLOCK;
+    st.spill_stride = a.spill_stride;
     st.sp = 0;
 }
 

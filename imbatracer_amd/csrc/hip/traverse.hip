@@ -111,11 +111,13 @@ int launch_one(const TraceArgs& args_in, int max_stack, int blocks_per_cu, int r
     }
     a.spill = nullptr;
     a.spill_depth = 0;
+    // Blocks past `needed` only work with four lanes per ray, which do not spill.
+    a.spill_stride = std::min(grid, std::max(1, needed)) * BLOCK;
     if (max_stack > STACK_LDS) {
         a.spill_depth = max_stack - STACK_LDS;
         std::lock_guard<std::mutex> lock(g_scratch_mutex);
         Scratch& sc = g_spill[std::make_pair(p->device, s)];
-        const size_t need = (size_t)a.spill_depth * grid * BLOCK * sizeof(int);
+        const size_t need = (size_t)a.spill_depth * a.spill_stride * sizeof(int);
         if (sc.bytes < need) {
             int r = not_capturing(s, "a larger spill stack");
             if (r) return r;

@@ -121,3 +121,34 @@ def test_recorded_batch(gpu):
             st.sync()
             got = hb.download(N.HIT_DTYPE, len(rays))
             assert _same(got[:n], want[:n]) and (np.ascontiguousarray(got[n:]).view(np.int32) == 7).all(), (n, cfg)
+
+
+def test_spill_is_sized_for_one_lane_per_ray(gpu):
+    """The launch of a small queue has four threads per ray, and its spill stack those of one lane per
+    ray: a strided launch on a stream leaves room enough to record the small queue's.
+    A device count on either side of the largest small queue then finds its place in it."""
+    b = T.random_tri_scene(200000, N.BUILDER_BINNED_SAH)[0]
+    sc = S.Scene(b.desc())
+    assert S.wide_tree(b.arrays())["max_stack"] > 16
+    for cap in (20000, LARGEST + 20000):
+        rays = T.random_rays(cap, seed=12)
+        want = sc.trace_host(rays, cfg=ONE_LANE)
+        rb, hb, st = N.DeviceBuffer.from_array(rays), N.DeviceBuffer(16 * cap), N.Stream()
+        cnt = N.DeviceBuffer.from_array(np.array([cap], np.int32))
+        # eight blocks per CU: one thread per ray here, so the spill of one lane per ray
+        strided = N.TraceConfig(256, 16, 0, 8, 4, 1, 0)
+        sc.intersect(rb, hb, cap, strided, st)
+        st.sync()
+        S.Graph.begin(st)
+        try:
+            N.check(N.lib.imba_intersect_dev(sc.h, rb.ptr, hb.ptr, cap, cnt.ptr, N.C.byref(Q4), st.handle), "intersect_dev")
+        finally:
+            g = S.Graph.end(st)
+        for n in (cap, 77, min(cap, LARGEST + 1), cap):
+            cnt.upload(np.array([n], np.int32))
+            hb.upload(np.full(4 * cap, 7, np.int32))
+            g.launch(st)
+            st.sync()
+            got = hb.download(N.HIT_DTYPE, cap)
+            assert _same(got[:n], want[:n]) and (np.ascontiguousarray(got[n:]).view(np.int32) == 7).all(), (cap, n)
+    assert sc.error_count() == 0
