@@ -314,8 +314,10 @@ int run_compact(CompactArgs a, int* new_count, void* stream, bool static_scratch
         int r = scratch_for_device(dev, &a.block_counts);
         if (r) return r;
     } else {
+        // Room for every smaller queue too (one of 1,048,576 entries has more tiles than a larger
+        // one), so that a call that was made once can be recorded with any smaller size.
         Scratch& sc = t_offsets[dev & 63];
-        int r = grow_buffer(sc, sizeof(int) * ((size_t)nb + 1));
+        int r = grow_buffer(sc, sizeof(int) * ((size_t)std::max(max_tiles(a.n), kSmallTiles) + 1));
         if (r) return r;
         a.block_counts = (int*)sc.ptr;
     }

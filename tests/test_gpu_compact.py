@@ -171,3 +171,51 @@ def test_sort_tile_and_digit_edges(gpu, count, num_mats):
     """The sort at the edges of its tiles (2048 entries), of the scan over tiles (256 of them) and of
     its digits (keys up to 1, 255 and 65536: one, one and three passes)."""
     test_sort_by_material_matches_oracle(gpu, count, num_mats)
+
+
+@pytest.mark.parametrize("warm,recorded", [(100, 1 << 20), ((1 << 20) + 1, 1 << 20), (5000, 2000000)])
+def test_recorded_after_another_size(gpu, warm, recorded):
+    """A host thread's first compaction allocates its tile counts; one of another size (with more
+    tiles: 2,048 at 1,048,576 entries, 513 at one entry more) can then be recorded into a graph."""
+    import threading
+
+    def work():
+        try:
+            n = max(warm, recorded)
+            rng = np.random.default_rng(3)
+            rays = np.zeros(n, N.RAY_DTYPE)
+            rays["org"][:, 0] = np.arange(n) % (1 << 24)
+            hits = np.zeros(n, N.HIT_DTYPE)
+            hits["tri_id"] = np.where(rng.random(n) < 0.6, np.arange(n), -1)
+            bufs = [N.DeviceBuffer.from_array(x) for x in (rays, hits, np.arange(n, dtype=np.int32))]
+            outs = [N.DeviceBuffer(b.nbytes) for b in bufs]
+            st = N.Stream()
+
+            def call(count):
+                N.check(N.lib.imba_compact_hits(*[b.ptr for b in bufs], 4, count, *[o.ptr for o in outs], None, st.handle),
+                        "compact_hits")
+
+            call(warm)
+            st.sync()
+            S.Graph.begin(st)
+            try:
+                call(recorded)
+            finally:
+                g = S.Graph.end(st)
+            want = np.nonzero(hits["tri_id"][:recorded] >= 0)[0]
+            for _ in range(2):
+                for o in outs:
+                    o.upload(np.zeros(o.nbytes, np.uint8))
+                g.launch(st)
+                st.sync()
+                assert np.array_equal(outs[2].download(np.int32, len(want)), want)
+                assert np.array_equal(outs[1].download(N.HIT_DTYPE, len(want))["tri_id"], want)
+        except BaseException as e:
+            failed.append(e)
+
+    failed = []
+    t = threading.Thread(target=work)
+    t.start()
+    t.join()
+    if failed:
+        raise failed[0]
