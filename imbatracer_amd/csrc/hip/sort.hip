@@ -90,9 +90,10 @@ int imba_sort_by_material(const int* indices, int tri_count, ImbaRay* rays, cons
     }
     int bits = 1;
     while ((1 << bits) <= num_mats) bits++;  // keys go up to num_mats
-    // scratch: keys and values twice, digit counts
+    // scratch: keys and values twice, digit counts; at least two pages, so that the first small call
+    // makes room for all small ones (a later one may be recorded into a graph)
     const size_t n4 = (size_t)count * 4;
-    const size_t need = 4 * n4 + radix_counts_size<kItems>(count) * 4;
+    const size_t need = std::max<size_t>(4 * n4 + radix_counts_size<kItems>(count) * 4, 8192);
     int dev = 0;
     IMBA_HIP_TRY(hipGetDevice(&dev));
     Scratch& sc = t_sort[dev & 63];

@@ -173,49 +173,86 @@ def test_sort_tile_and_digit_edges(gpu, count, num_mats):
     test_sort_by_material_matches_oracle(gpu, count, num_mats)
 
 
-@pytest.mark.parametrize("warm,recorded", [(100, 1 << 20), ((1 << 20) + 1, 1 << 20), (5000, 2000000)])
-def test_recorded_after_another_size(gpu, warm, recorded):
-    """A host thread's first compaction allocates its tile counts; one of another size (with more
-    tiles: 2,048 at 1,048,576 entries, 513 at one entry more) can then be recorded into a graph."""
+def _in_new_thread(fn):
+    """Runs fn in a host thread of its own (scratch buffers are kept per thread)."""
     import threading
+
+    failed = []
 
     def work():
         try:
-            n = max(warm, recorded)
-            rng = np.random.default_rng(3)
-            rays = np.zeros(n, N.RAY_DTYPE)
-            rays["org"][:, 0] = np.arange(n) % (1 << 24)
-            hits = np.zeros(n, N.HIT_DTYPE)
-            hits["tri_id"] = np.where(rng.random(n) < 0.6, np.arange(n), -1)
-            bufs = [N.DeviceBuffer.from_array(x) for x in (rays, hits, np.arange(n, dtype=np.int32))]
-            outs = [N.DeviceBuffer(b.nbytes) for b in bufs]
-            st = N.Stream()
-
-            def call(count):
-                N.check(N.lib.imba_compact_hits(*[b.ptr for b in bufs], 4, count, *[o.ptr for o in outs], None, st.handle),
-                        "compact_hits")
-
-            call(warm)
-            st.sync()
-            S.Graph.begin(st)
-            try:
-                call(recorded)
-            finally:
-                g = S.Graph.end(st)
-            want = np.nonzero(hits["tri_id"][:recorded] >= 0)[0]
-            for _ in range(2):
-                for o in outs:
-                    o.upload(np.zeros(o.nbytes, np.uint8))
-                g.launch(st)
-                st.sync()
-                assert np.array_equal(outs[2].download(np.int32, len(want)), want)
-                assert np.array_equal(outs[1].download(N.HIT_DTYPE, len(want))["tri_id"], want)
+            fn()
         except BaseException as e:
             failed.append(e)
 
-    failed = []
     t = threading.Thread(target=work)
     t.start()
     t.join()
     if failed:
         raise failed[0]
+
+
+def _recorded(call, warm, recorded, outs, check):
+    """call(warm) as it is, then call(recorded) in a graph, replayed twice."""
+    st = N.Stream()
+    call(warm, st)
+    st.sync()
+    S.Graph.begin(st)
+    try:
+        call(recorded, st)
+    finally:
+        g = S.Graph.end(st)
+    for _ in range(2):
+        for o in outs:
+            o.upload(np.zeros(o.nbytes, np.uint8))
+        g.launch(st)
+        st.sync()
+        check()
+
+
+@pytest.mark.parametrize("warm,recorded", [(100, 1 << 20), ((1 << 20) + 1, 1 << 20), (5000, 2000000)])
+def test_recorded_after_another_size(gpu, warm, recorded):
+    """A host thread's first compaction allocates its tile counts; one of another size (with more
+    tiles: 2,048 at 1,048,576 entries, 513 at one entry more) can then be recorded into a graph."""
+    def work():
+        n = max(warm, recorded)
+        rays, hits = np.zeros(n, N.RAY_DTYPE), np.zeros(n, N.HIT_DTYPE)
+        hits["tri_id"] = np.where(np.random.default_rng(3).random(n) < 0.6, np.arange(n), -1)
+        bufs = [N.DeviceBuffer.from_array(x) for x in (rays, hits, np.arange(n, dtype=np.int32))]
+        outs = [N.DeviceBuffer(b.nbytes) for b in bufs]
+        want = np.nonzero(hits["tri_id"][:recorded] >= 0)[0]
+
+        def call(count, st):
+            N.check(N.lib.imba_compact_hits(*[b.ptr for b in bufs], 4, count, *[o.ptr for o in outs], None, st.handle),
+                    "compact_hits")
+
+        def check():
+            assert np.array_equal(outs[2].download(np.int32, len(want)), want)
+            assert np.array_equal(outs[1].download(N.HIT_DTYPE, len(want))["tri_id"], want)
+
+        _recorded(call, warm, recorded, outs, check)
+
+    _in_new_thread(work)
+
+
+def test_small_sort_recorded_after_a_smaller_one(gpu):
+    """A host thread's first sort of a few rays makes room for one of a few more in a graph."""
+    def work():
+        n = 191
+        hits = np.zeros(n, N.HIT_DTYPE)
+        hits["tri_id"] = np.random.default_rng(4).integers(0, 50, n)
+        indices = np.zeros((50, 4), np.int32)
+        indices[:, 3] = np.arange(50) % 7
+        rb, hb, ib = N.DeviceBuffer(32 * n), N.DeviceBuffer.from_array(hits), N.DeviceBuffer.from_array(indices)
+        out = N.DeviceBuffer(4 * n)
+
+        def call(count, st):
+            N.check(N.lib.imba_sort_by_material(ib.ptr, 50, rb.ptr, hb.ptr, count, 7, out.ptr, None, st.handle), "sort")
+
+        def check():
+            want = np.argsort(hits["tri_id"] % 7, kind="stable")
+            assert np.array_equal(out.download(np.int32, n), want)
+
+        _recorded(call, 50, n, [out], check)
+
+    _in_new_thread(work)
