@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cstring>
 #include <map>
@@ -416,9 +417,15 @@ int launch_batch_kernel(ImbaTraceBatch* b, int g, int blocks_per_cu, int limit, 
     const DeviceProps* p = device_props();
     auto kern = k_trace_batch<BLOCK, STACK_LDS, ANY, MASKED, TREE, QUADS>;
     const int max_stack = b->max_stack[TREE ? 1 : 0][g];
-    int resident = 0;
-    IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, BLOCK, 0));
-    if (resident <= 0) resident = 1;
+    // Blocks per CU, a property of this kernel and the device: asked for once per device (a group of
+    // small queues over the quantized tree needs two kernels' numbers on every launch).
+    static std::atomic<int> resident_on[64] = {};
+    int resident = resident_on[p->device & 63].load(std::memory_order_relaxed);
+    if (resident == 0) {
+        IMBA_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&resident, kern, BLOCK, 0));
+        if (resident <= 0) resident = 1;
+        resident_on[p->device & 63].store(resident, std::memory_order_relaxed);
+    }
     if (blocks_per_cu > 0) resident = std::min(resident, blocks_per_cu);
     const long long chunks = b->capacity_chunks[g];
     const long long pieces = QUADS ? 4 * std::min<long long>(chunks, limit) : chunks;  // 64 threads each
