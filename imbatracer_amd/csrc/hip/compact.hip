@@ -28,11 +28,17 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 // Entries per tile: 512 in queues of up to 2,048 such tiles, so that a small queue has blocks for
-// every CU, else 2,048.
+// every CU, else 2,048: the tiles' sums of the counts before them cost more than the blocks gain.
+// us with 512 / 2,048, compact_hits with 40-byte states (16-byte states and compact_rays cross at
+// 0.9 to 1.3M entries too): 65,536 entries 9 / 22, 524,288 21 / 33, 786,432 33 / 37, 1,048,576 44 / 39,
+// 2,097,152 103 / 99; compact_rays 7 / 15, 16 / 23, 22 / 28, 33 / 34, 65 / 61.
 constexpr int kSmallItems = 2, kLargeItems = 8;
 constexpr int kSmallTiles = 2048;
-// Tiles up to which every block of the scatter adds up the counts itself: all blocks together
-// read tiles^2 / 2 counts from L2 (33 MB at 4,096 tiles), a launch of its own costs 4.7 us.
+// Tiles up to which every block of the scatter adds up the counts itself: all blocks together read
+// tiles^2 counts from L2 (67 MB at 4,096 tiles).  us with the sums / with a launch between the two that
+// makes offsets of the counts, 16-byte states, compact_hits and compact_rays: 1,048,576 entries (512
+// tiles) 30 / 32 and 19 / 21, 8,388,608 (4,096) 293 / 296 and 165 / 165, 12,582,912 437 / 442 and
+// 263 / 257, 16,777,216 585 / 595 and 358 / 351.
 constexpr int kSumTiles = 4096;
 
 constexpr int tile_of(int n) {
@@ -134,7 +140,7 @@ __global__ __launch_bounds__(1024) void k_scan_offsets(int* offs, int nb, int* c
 // places from `dst`: rays and hits a record per lane; states a unit (4, 8 or 16 bytes) per
 // lane, so that neighbouring lanes read and write neighbouring memory (a 40-byte state copied by
 // its own lane takes ten instructions that touch every line of the wave's 2.5 KB each).
-// `list` holds 64 ints of the wave's LDS.
+// `list` holds 64 bytes of the wave's LDS.
 template <int MODE, typename UNIT>
 __device__ __forceinline__ void move_records(const CompactArgs& a, int first, unsigned long long mask, int dst,
                                              uint8_t* list) {
