@@ -2,8 +2,8 @@
 autotuner (GPU).
 
 Every queue's hits are checked against the oracle's traversal of the same rays: closest hits
-bit for bit on every tree (the closest hit does not depend on the traversal order), any hits
-bit for bit on the BVH2 (the oracle walks the BVH2 in the kernel's order) and, on the 4-wide
+bit for bit on every tree (the scenes' triangles are in general position, where every tree tests the
+nearest one), any hits bit for bit on the BVH2 (the oracle walks the BVH2 in the kernel's order) and, on the 4-wide
 trees, whose order differs, the occlusion answer plus bit equality with a single-queue launch
 of the same tree.  The device-count variants read the queue size when they run; a graph
 replays the very launches of an eager frame (whose every bounce the path-tracing image test
@@ -56,8 +56,8 @@ def _filled_hits(n):
     return hb
 
 
-# (block, stack) or (block, stack, bvh_width, quantized, treelet); batches clamp treelets to 64
-# nodes per wave, and a treelet never changes a result
+# (block, stack) or (block, stack, bvh_width, quantized, treelet); the treelet field is accepted and
+# changes nothing
 CFGS = [None, (128, 32), (64, 64), (256, 16, 4, 1, 0), (256, 16, 4, 1, 64), (128, 32, 4, 1, 256)]
 
 
@@ -78,7 +78,7 @@ def test_batch_matches_single_launches(gpu, cfg):
         rb = N.DeviceBuffer.from_array(rays) if n else N.DeviceBuffer(32)
         queues.append((sc, rb, _filled_hits(n), n, None, any_hit, rays, arrays))
     tc = _cfg(cfg)
-    single = _cfg(cfg[:4]) if cfg and len(cfg) > 4 else tc  # the same tree without a treelet
+    single = _cfg(cfg[:4]) if cfg and len(cfg) > 4 else tc  # the same tree, treelet field 0
     batch = S.TraceBatch([q[:6] for q in queues])
     for rep in range(2):  # the work counters must return to zero after a launch
         for q in queues:
@@ -97,8 +97,7 @@ def test_batch_matches_single_launches(gpu, cfg):
 @pytest.mark.parametrize("cfg", [None, (256, 16, 4, 1, 64)])
 def test_batch_device_counts_and_many_queues(gpu, cfg):
     """256 queues over 8 scenes, sizes read from device memory at launch time; entries past a
-    queue's device count are left untouched.  With a treelet every wave reloads its LDS copy
-    whenever its next chunk belongs to another scene."""
+    queue's device count are left untouched."""
     bs = [T.random_tri_scene(2000 + 500 * k, N.BUILDER_SBVH if k % 2 else N.BUILDER_BINNED_SAH, seed=40 + k)[0]
           for k in range(8)]
     scenes = [S.Scene(b.desc()) for b in bs]

@@ -2,8 +2,9 @@
 go over to that when 16 rays are left: hits equal those of the persistent kernel (one lane per
 ray throughout) bit for bit, closest and any hit, and the oracle's closest hits, at the edges of
 quads, waves and the largest queue that starts this way, over leaves longer than a quad, stacks
-deeper than the LDS part, instances and masks, for device-side counts and batches; closest hits
-of the default launch equal the BVH2's.
+deeper than the LDS part, instances and masks, for device-side counts and batches.  The scenes'
+triangles are in general position (or coincide, which no tree tells apart), so the default launch's
+closest hits, the BVH2's, are the same.
 """
 import numpy as np
 import pytest
@@ -76,7 +77,7 @@ def test_device_counts_and_batches(gpu):
         N.check(N.lib.imba_intersect_dev(sc.h, rb.ptr, hb.ptr, len(rays), cnt.ptr, None, None), "intersect_dev")
         got = hb.download(N.HIT_DTYPE, len(rays))
         assert _same(got[:n], want[:n]) and (np.ascontiguousarray(got[n:]).view(np.int32) == 7).all(), n
-        # two closest queues and an any-hit queue of the same rays, default trees per kind
+        # two closest queues and an any-hit queue of the same rays
         k = n // 3
         batch = S.TraceBatch([(sc, rb, hb, k, None, False), (sc, rb.at(32 * k), hb.at(16 * k), len(rays) - k, cnt, False),
                               (sc, rb, ha, n, None, True)])

@@ -2,11 +2,11 @@
 BVH2 traversal.
 
 The 4-wide tree keeps the BVH2's leaves and leaf boxes and uses the same box and triangle
-arithmetic, so closest hits (smallest t, then smaller triangle id, then smaller instance id)
-must equal the oracle's bit for bit.  An occlusion query may stop at another triangle than the
+arithmetic, and the scenes' triangles are in general position, so closest hits (smallest t, then
+smaller triangle id, then smaller instance id) must equal the oracle's bit for bit.  An occlusion query may stop at another triangle than the
 BVH2's first hit; its occluded / unoccluded answer must be the same, and a reported hit must be
-a real one (t inside the ray's interval).  Staging the quantized tree's top levels in LDS
-(treelet) changes only where those nodes are read from, so its results are held to the same bar.
+a real one (t inside the ray's interval).  The configuration's treelet
+field is accepted for the quantized tree and changes nothing.
 """
 import numpy as np
 import pytest
@@ -19,7 +19,7 @@ from tests import scenes as T
 pytestmark = pytest.mark.gpu
 
 WIDE = N.TraceConfig(0, 0, 0, 0, 4)
-# 4-wide, 4-wide quantized, quantized with its top 256 nodes staged in LDS
+# 4-wide, 4-wide quantized, quantized with the treelet field at its largest
 TREES = [N.TraceConfig(0, 0, 0, 0, 4, 0), N.TraceConfig(0, 0, 0, 0, 4, 1), N.TraceConfig(0, 0, 0, 0, 4, 1, 256)]
 TREE_IDS = ["wide", "quantized", "treelet"]
 
@@ -137,8 +137,7 @@ def test_visit_counts_and_batch(gpu):
 
 
 def test_treelet_arguments(gpu):
-    """A treelet needs the quantized tree and at most 256 nodes; a larger request than the tree
-    has is clamped to the tree."""
+    """The treelet field needs the quantized tree and is at most 256, which a small tree takes too."""
     v = np.array([[-1, -1, 1, 1], [1, -1, 1, 1], [0, 1, 1, 1]], np.float32)
     b = S.SceneBuild()
     b.add_mesh(v, np.array([[0, 1, 2, 0]], np.uint32))
