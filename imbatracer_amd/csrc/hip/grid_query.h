@@ -137,8 +137,8 @@ inline int queries_per_wave(int nq, int cu_count) {
 // with SLOTS the photon's slot in the grid order (pos4[slot]).  Returns the list length
 // (wave-uniform); lanes >= count hold (0, -1).  Every lane of the wave must call it.
 //
-// Bound by instruction issue: 720 vector and 540 scalar instructions per query at k = 10 over
-// 1,000 probed photons, 70% of the kernel's time.  Before the bound (which leaves 11-15 insertions
+// Bound by instruction issue: 690 vector and 500 scalar instructions per query at k = 10 over 1,000
+// probed photons, vector issue 95% of the SIMDs' time.  Before the bound (which leaves 11-15 insertions
 // of 45), 600,000 queries over 2M photons took 1,557 us, now 785; 200,000 with k = 64 860, now 636;
 // with k = 1 265, now 137.  Groups of 2 or 8 chunks and testing a bucket's end per chunk were slower.
 template <bool SLOTS>

@@ -648,8 +648,8 @@ __device__ __forceinline__ void stack_init(LaneStack<BLOCK, STACK_LDS>& st, int*
 // 187; 1M primary rays 360 -> 694 (the chip is full and four lanes do more work per ray).
 //
 // Waves of larger queues start with a lane per ray and go over to it (wave_trace): with 37% (1M
-// primary rays) to 23% (diffuse rays) of the lanes busy on average, most steps of a wave serve few
-// rays.  Moving the state costs about one step.  us per launch before -> now: 1M primary rays
+// primary rays) to 23% (diffuse rays) of the lanes busy on average without that, most steps of a wave
+// serve few rays (with it 46% for the primary rays).  Moving the state costs about one step.  us per launch before -> now: 1M primary rays
 // 361 -> 353, 1M shadow rays 534 -> 486, 300K diffuse rays over 250K triangles 397 -> 334, 200K rays
 // over masked instances 790 -> 743, 48 queues in a batch 1,040 -> 917; path-traced frame 640x480
 // 4,261 -> 4,002.
