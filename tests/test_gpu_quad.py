@@ -153,3 +153,23 @@ def test_spill_is_sized_for_one_lane_per_ray(gpu):
             got = hb.download(N.HIT_DTYPE, cap)
             assert _same(got[:n], want[:n]) and (np.ascontiguousarray(got[n:]).view(np.int32) == 7).all(), (cap, n)
     assert sc.error_count() == 0
+
+
+@pytest.mark.parametrize("name", ["boxes", "sphere", "decal"])
+def test_where_triangles_meet(gpu, name):
+    """Where triangles meet or overlap the quantized tree's hits are its own (boxes are culled by rounded
+    distances), and the same for every mapping of rays to lanes."""
+    if name == "boxes":
+        b, rays = T.box_scene(), T.random_rays(LARGEST + 5000, seed=3, box=(0.0, 2.2))
+    else:
+        b, points = T.sphere_scene() if name == "sphere" else T.decal_scene()
+        rays = T.aimed_rays(points, LARGEST + 5000, seed=5)
+    sc = S.Scene(b.desc())
+    for any_hit in (False, True):
+        want = sc.trace_host(rays, any_hit=any_hit, cfg=ONE_LANE)
+        for n in (1000, LARGEST, len(rays)):
+            assert _same(sc.trace_host(rays[:n], any_hit=any_hit, cfg=Q4), want[:n]), n
+            assert _same(sc.trace_host(rays[:n], any_hit=any_hit, cfg=STRIDED), want[:n]), n
+        if not any_hit:
+            assert not _same(want, sc.trace_host(rays))  # the rays find such places
+    assert sc.error_count() == 0
